@@ -190,6 +190,54 @@ def test_cat_wave_kernel(dev, B, A):
     run_cat(dev, B, A, seed=B + A, vf_clip=0.2)
 
 
+# widths around every change of form: groups of 1 to 64 lanes and 1 to 4 chunks
+# per lane, rows that end inside a chunk, the LDS wave tiles with one or two
+# logits to spare, the wave-per-row kernel above
+FORM_WIDTHS = [1, 2, 3, 4, 5, 8, 9, 10, 16, 17, 19, 20, 21, 27, 31, 32, 33, 36, 41, 43, 44, 45, 64,
+               65, 127, 128, 129, 256, 257, 511, 512, 513, 1023, 1024, 1025]
+
+
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("A", FORM_WIDTHS)
+def test_cat_forms(dev, A, offset):
+    """Every categorical form, aligned and on a view that starts 4 bytes into
+    its storage, over a batch that ends inside a tile: masked (-inf) logits
+    against the oracle; then a NaN and an infinite logit, which make their own
+    rows' gradients NaN and change no other row."""
+    B = 205
+    g = torch.Generator().manual_seed(900 + A)
+    inp = list(cat_inputs(B, A, seed=900 + A))
+    mask = torch.rand(B, A, generator=g) < 0.1
+    mask.scatter_(1, inp[1].long()[:, None], False)
+    inp[0] = inp[0].masked_fill(mask, -float("inf"))
+    lp = torch.log_softmax(inp[0], -1).gather(1, inp[1].long()[:, None]).squeeze(1)
+    inp[2] = lp + 0.05 * torch.randn(B, generator=g)
+
+    def run(logits):
+        buf = torch.empty(B * A + offset, device=dev)
+        buf[offset:] = logits.reshape(-1).to(dev)
+        print(f"loss_cat form A={A} offset={offset}", flush=True)
+        return ppo_amd.ppo_loss_discrete_fused(
+            buf[offset:].view(B, A), *[x.to(dev) for x in inp[1:]], 0.2, 0.2, 0.5, 0.01)
+
+    scalars, dlogits, dvalues = run(inp[0])
+    o = ref.loss_categorical_reference(*inp, 0.2, 0.2, 0.5, 0.01)
+    edge = clip_edge_rows(o["ratio"], lp, inp[2])
+    assert_scalars_close(scalars, o, edge_rows=int(edge.sum()), lp_scale=math.log(A + 1))
+    assert_rows_close(dlogits, o["dlogits"], edge)
+    assert_grad_close(dvalues, o["dvalues"])
+
+    bad = inp[0].clone()
+    bad[3, A // 2] = float("nan")
+    bad[B - 1, A - 1] = float("inf")
+    _, dbad, dvbad = run(bad)
+    rows = torch.ones(B, dtype=torch.bool)
+    rows[[3, B - 1]] = False
+    assert torch.isnan(dbad[~rows.to(dev)]).all()
+    assert torch.equal(dbad[rows.to(dev)], dlogits[rows.to(dev)])
+    assert torch.equal(dvbad, dvalues)
+
+
 def test_cat_int64_actions(dev):
     run_cat(dev, 1000, 18, seed=3, act_dtype=torch.int64)
 

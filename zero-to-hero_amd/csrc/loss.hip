@@ -17,14 +17,12 @@
 //     dvalue    = vc * 2 * (v - R) / B          (or the clipped-value form)
 // Gaussian variant: Normal(mu, exp(log_std)) summed over the action dims.
 //
-// Layout: one thread per row.  A workgroup walks 256-row tiles of the
-// [B,A] logits (each tile a contiguous block of 256*A floats) on a grid
-// capped at a few workgroups per CU; per tile it prefetches the per-row
-// inputs into registers, stages the logits through LDS with float4 loads
-// (row stride padded to an odd number of words, so the row-per-thread LDS
-// reads are bank-conflict-free), and writes dlogits back through the same
-// tile.  Loss scalars are summed per workgroup in fp64 and combined in a fixed
-// order by a one-block finaliser kernel (deterministic, no float atomics).
+// Layout: tiles of whole rows on a grid capped at what is resident at once.
+// Narrow categorical rows are staged through LDS one row per lane
+// (loss_cat_wtile_kernel), wider ones spread over neighbouring lanes
+// (loss_cat_lanes_kernel); Gaussian rows take one lane each.  Loss scalars are
+// summed per workgroup in fp64 and combined in a fixed order (deterministic,
+// no float atomics).
 #include <float.h>
 
 #include <algorithm>
@@ -36,10 +34,9 @@
 namespace ppo {
 namespace {
 
-// Widths handled by the row-per-thread kernels, chosen so that the LDS tiles
-// (256 rows x odd-padded width, one tile for logits, two for mu/actions) plus
-// the static reduction arrays stay under the 64 KiB a workgroup may address.
-constexpr int kMaxCatRowWidth = 48;  // A above this uses the wave-per-row kernel
+constexpr int kMaxWtileWidth = 44;    // widest row of the LDS wave tiles (cat_wtile)
+constexpr int kMaxLanesWidth = 1024;  // A above this uses the wave-per-row kernel
+constexpr int kNarrowWidth = 48;      // workspace: a block per 64 rows up to here, per 4 above
 constexpr int kMaxGaussDim = 24;     // D limit of the Gaussian kernel
 constexpr int kScalarSlots = 8;      // per-block partial doubles reserved for the loss scalars
 constexpr int kGaussSlots = kScalarSlots + kMaxGaussDim;
@@ -430,210 +427,7 @@ __device__ __forceinline__ ActT row_action_raw(const LossArgs& a, long row) {
 }
 
 // ---------------------------------------------------------------------------
-// Categorical, A <= kMaxCatRowWidth: one thread per row, logits staged
-// through LDS.  Softmax statistics in two passes over the row:
-//   m = max z;  s = sum e_j, e_j = exp(z_j - m);  S = sum e_j (z_j - m)
-//   log p_j = (z_j - m) - log s;   H = log s - S / s
-// and a third pass recomputes e_j for the gradient (2 exp per logit).  The
-// per-logit exponentials use the hardware exp2 (__expf: one multiply by
-// log2(e) and v_exp_f32, relative error ~1e-6 for |z_j - m| <= 20); the
-// accurate expf sequence costs ~10 VALU ops and made this kernel VALU-bound.
-// The ratio exp(lp - old_lp) keeps the accurate expf.
-// ---------------------------------------------------------------------------
-template <typename ActT, bool kVec>
-__global__ void __launch_bounds__(kBlock) loss_cat_kernel(LossArgs a, long ntiles) {
-  extern __shared__ float s_tile[];
-  const int A = a.A;
-  const int AS = A | 1;
-  const float invA = 1.0f / (float)A;
-  const float ge = a.ec * a.inv_b;
-  const int tid = threadIdx.x;
-  double acc[5] = {0, 0, 0, 0, 0};
-
-  for (long tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-    const long row0 = tile * kBlock;
-    const int nrows = (int)std::min<long>(kBlock, a.B - row0);
-    const long row = row0 + tid;
-    RowIn in = {0, 0, 0, 0, 0};
-    int ai = -1;
-    if (tid < nrows) {
-      in = load_row(a, row);
-      ai = row_action<ActT>(a, row);
-    }
-    stage_in<kVec>(a.x + row0 * A, nrows * A, A, invA, AS, s_tile);
-    __syncthreads();
-
-    if (tid < nrows) {
-      float* z = s_tile + tid * AS;
-      float m = -INFINITY;
-      for (int j = 0; j < A; ++j) m = fmaxf(m, z[j]);
-      float s = 0.0f, S = 0.0f;
-      for (int j = 0; j < A; ++j) {
-        const float t = z[j] - m;
-        const float e = __expf(t);
-        s += e;
-        S += e > 0.0f ? e * t : 0.0f;
-      }
-      const float log_s = logf(s);
-      const float inv_s = 1.0f / s;
-      const float H = log_s - S * inv_s;
-      const float lp = ai >= 0 ? (z[ai] - m) - log_s : __builtin_nanf("");
-      const RowOut o = ppo_row(a, row, in, lp);
-      for (int j = 0; j < A; ++j) {
-        const float t = z[j] - m;
-        const float p = __expf(t) * inv_s;
-        const float logp = fmaxf(t - log_s, -FLT_MAX);
-        const float onehot = j == ai ? 1.0f : 0.0f;
-        z[j] = o.g_lp * (onehot - p) + ge * (p * (logp + H));
-      }
-      accumulate(acc, o, H);
-    }
-    __syncthreads();
-    stage_out<kVec>(a.dx + row0 * A, nrows * A, A, invA, AS, s_tile);
-    __syncthreads();
-  }
-  store_scalar_partials(a, acc);
-  if (a.finish) loss_publish<0>(a);
-}
-
-// ---------------------------------------------------------------------------
-// Categorical, A <= 4*PF: the same per-row math as loss_cat_kernel,
-// software-pipelined for 16-byte-aligned inputs.  Each
-// thread holds up to PF float4 of the next tile's logits plus its row
-// inputs in registers: while tile i is computed out of LDS, the loads of
-// tile i+1 are already in flight, so a workgroup never waits on HBM between
-// tiles.  All streamed accesses are nontemporal.
-// ---------------------------------------------------------------------------
-template <typename ActT, int PF>
-struct CatPrefetch {
-  f4 x[PF];
-  float tail;   // element n4*4 + tid of a tile whose size is not a multiple of 4
-  RowIn in;
-  ActT act;     // raw action (validated when the tile is processed)
-  int nrows;
-};
-
-template <typename ActT, int PF>
-__device__ __forceinline__ void cat_prefetch(const LossArgs& a, long tile, CatPrefetch<ActT, PF>& p) {
-  const int tid = threadIdx.x;
-  const long row0 = tile * kBlock;
-  p.nrows = (int)std::min<long>(kBlock, a.B - row0);
-  const int count = p.nrows * a.A;
-  const int n4 = count >> 2;
-  const f4* src = reinterpret_cast<const f4*>(a.x + row0 * a.A);
-#pragma unroll
-  for (int k = 0; k < PF; ++k) {
-    const int i = k * kBlock + tid;
-    if (i < n4) p.x[k] = ldnt(src + i);
-  }
-  if (tid < count - (n4 << 2)) p.tail = ldnt(a.x + row0 * a.A + (n4 << 2) + tid);
-  if (tid < p.nrows) {
-    const long row = row0 + tid;
-    p.in = load_row(a, row);
-    p.act = row_action_raw<ActT>(a, row);
-  }
-}
-
-template <typename ActT, int PF>
-__global__ void __launch_bounds__(kBlock) loss_cat_pipe_kernel(LossArgs a, long ntiles) {
-  extern __shared__ float s_tile[];
-  const int A = a.A;
-  const int AS = A | 1;
-  const float invA = 1.0f / (float)A;
-  const float ge = a.ec * a.inv_b;
-  const int tid = threadIdx.x;
-  double acc[5] = {0, 0, 0, 0, 0};
-  CatPrefetch<ActT, PF> pf;
-  long tile = blockIdx.x;
-  if (tile < ntiles) cat_prefetch<ActT, PF>(a, tile, pf);
-
-  for (; tile < ntiles; tile += gridDim.x) {
-    // registers -> LDS for the current tile
-    const int nrows = pf.nrows;
-    const int count = nrows * A;
-    const int n4 = count >> 2;
-#pragma unroll
-    for (int k = 0; k < PF; ++k) {
-      const int i = k * kBlock + tid;
-      if (i < n4) {
-        const int e = i << 2;
-        int r = row_of(e, invA);
-        int c = e - r * A;
-#pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          s_tile[r * AS + c] = pf.x[k][q];
-          if (++c == A) { c = 0; ++r; }
-        }
-      }
-    }
-    if (tid < count - (n4 << 2)) {
-      const int e = (n4 << 2) + tid;
-      const int r = row_of(e, invA);
-      s_tile[r * AS + (e - r * A)] = pf.tail;
-    }
-    const RowIn in = pf.in;
-    const int ai = tid < nrows ? action_index<ActT>(a, pf.act) : -1;
-    const long row0 = tile * kBlock;
-    __syncthreads();
-
-    // next tile's loads go out before this tile's math
-    const long next = tile + gridDim.x;
-    if (next < ntiles) cat_prefetch<ActT, PF>(a, next, pf);
-
-    if (tid < nrows) {
-      const long row = row0 + tid;
-      float* z = s_tile + tid * AS;
-      float m = -INFINITY;
-      for (int j = 0; j < A; ++j) m = fmaxf(m, z[j]);
-      float s = 0.0f, S = 0.0f;
-      for (int j = 0; j < A; ++j) {
-        const float t = z[j] - m;
-        const float e = __expf(t);
-        s += e;
-        S += e > 0.0f ? e * t : 0.0f;
-      }
-      const float log_s = logf(s);
-      const float inv_s = 1.0f / s;
-      const float H = log_s - S * inv_s;
-      const float lp = ai >= 0 ? (z[ai] - m) - log_s : __builtin_nanf("");
-      const RowOut o = ppo_row(a, row, in, lp);
-      for (int j = 0; j < A; ++j) {
-        const float t = z[j] - m;
-        const float p = __expf(t) * inv_s;
-        const float logp = fmaxf(t - log_s, -FLT_MAX);
-        const float onehot = j == ai ? 1.0f : 0.0f;
-        z[j] = o.g_lp * (onehot - p) + ge * (p * (logp + H));
-      }
-      accumulate(acc, o, H);
-    }
-    __syncthreads();
-    // LDS -> dlogits, nontemporal float4 stores
-    f4* dst = reinterpret_cast<f4*>(a.dx + row0 * A);
-    for (int i = tid; i < n4; i += kBlock) {
-      const int e = i << 2;
-      int r = row_of(e, invA);
-      int c = e - r * A;
-      f4 v;
-#pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[q] = s_tile[r * AS + c];
-        if (++c == A) { c = 0; ++r; }
-      }
-      stnt(v, dst + i);
-    }
-    if (tid < count - (n4 << 2)) {
-      const int e = (n4 << 2) + tid;
-      const int r = row_of(e, invA);
-      a.dx[row0 * A + e] = s_tile[r * AS + (e - r * A)];
-    }
-    __syncthreads();
-  }
-  store_scalar_partials(a, acc);
-  if (a.finish) loss_publish<0>(a);
-}
-
-// ---------------------------------------------------------------------------
-// Categorical, A <= MAXA and A % 4 != 0, 16-byte-aligned inputs: wave tiles,
+// Categorical, A <= kMaxWtileWidth, 16-byte-aligned inputs (cat_wtile): wave tiles,
 // the register-resident form.  Each wave owns a tile of 64 consecutive rows
 // (one contiguous span of 64*A floats, 16*A float4) and stages it through its
 // own slice of LDS in its global layout (one ds_write_b128 / ds_read_b128 per
@@ -650,7 +444,10 @@ __global__ void __launch_bounds__(kBlock) loss_cat_pipe_kernel(LossArgs a, long 
 // log s); the 1[j == a] * g_lp term is added by one LDS read-modify-write per
 // row.  That is ~10 VALU operations per logit against ~40 for the LDS-pass
 // form, which was VALU-bound on MI355X.  KA > 0 fixes A at compile time (no
-// per-logit predicates); KA == 0 takes A from the arguments, A <= MAXA.
+// per-logit predicates); KA == 0 takes A from the arguments, MAXA - 2 <= A <=
+// MAXA, so that at most two logits are tested against A (with all of them
+// tested the scalar branches cost more than the row's arithmetic: B =
+// 1,000,000, A = 13 35.0 -> 29.9 us, A = 17 41.2 -> 35.7).
 //
 // Full tiles run branch-free: lane l moves float4 min(64k + l, 16A - 1) for
 // k < ceil(A/4) (lanes past the end repeat the last float4: same address,
@@ -703,12 +500,14 @@ __device__ __forceinline__ void wave_lds_handoff() {
 
 // One row from LDS (zr: A logits) to its gradient in place; accumulates the
 // row's loss terms (the formulas above).
-template <int KA, int MAXA>
+template <int MAXA, int MINA>
 __device__ __forceinline__ void cat_row_math(const LossArgs& a, float* zr, int A, long row,
                                              const RowIn& in, int ai, float ge,
                                              double (&acc)[5]) {
+  if constexpr (MINA == MAXA && MAXA % 4 == 0)
+    zr = static_cast<float*>(__builtin_assume_aligned(zr, 16));
   float H;
-  const RowOut o = cat_row_grad<MAXA>(a, zr, A, ai, ge, in, H);
+  const RowOut o = cat_row_grad<MAXA, MINA>(a, zr, A, ai, ge, in, H);
   stnt(o.dval, a.dval + row);
   accumulate(acc, o, H);
 }
@@ -716,6 +515,7 @@ __device__ __forceinline__ void cat_row_math(const LossArgs& a, float* zr, int A
 template <typename ActT, int KA, int MAXA, bool kVclip>
 __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long nfull) {
   constexpr int PF = (MAXA + 3) / 4;
+  constexpr int kMinA = KA > 0 ? KA : MAXA - 2;
   constexpr int kWavesPerBlock = kBlock / kWave;
   extern __shared__ float s_lds[];
   const int A = KA > 0 ? KA : a.A;
@@ -744,7 +544,7 @@ __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long
     const long next = wt + wstride;
     if (next < nfull) wave_prefetch<ActT, PF, kVclip>(a, next, lane, n4, pf);
 
-    cat_row_math<KA, MAXA>(a, s_tile + lane * A, A, row0 + lane, in, ai, ge, acc);
+    cat_row_math<MAXA, kMinA>(a, s_tile + lane * A, A, row0 + lane, in, ai, ge, acc);
     wave_lds_handoff();
     f4* dst = reinterpret_cast<f4*>(a.dx + row0 * A);
 #pragma unroll
@@ -767,7 +567,7 @@ __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long
     wave_lds_handoff();
     if (lane < nrows) {
       const long row = row0 + lane;
-      cat_row_math<KA, MAXA>(a, s_tile + lane * A, A, row, load_row_t<kVclip>(a, row),
+      cat_row_math<MAXA, kMinA>(a, s_tile + lane * A, A, row, load_row_t<kVclip>(a, row),
                              row_action<ActT>(a, row), ge, acc);
     }
     wave_lds_handoff();
@@ -780,7 +580,271 @@ __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long
 }
 
 // ---------------------------------------------------------------------------
-// Categorical, any A: one wave per row (lanes stride the actions).
+// Categorical, rows spread over lanes: G neighbouring lanes hold one row, VW
+// consecutive logits each in C chunks (lane q of the group holds columns
+// (q + c G) VW ..), so a wave loads 64 / G whole rows per step straight from
+// memory, coalesced, and needs no LDS transposition.  A wave tile is I steps
+// (I * 64 / G rows, I <= G): the tile's logits stay in registers (at most 64
+// VGPRs) from their one load to the gradient's store.  Per step a DPP tree
+// over the group forms the row's max, s = sum e and S = sum e t, and lane i of
+// each group keeps step i's: the row's scalar math (log, the ratio's exp,
+// the clipped surrogate, the value loss) then runs once per tile with one row
+// per lane instead of once per row in every lane, and its results return to
+// the groups through LDS (one broadcast 16-byte read per step).
+//
+// Loads are VW-wide at 4-byte alignment (global memory takes them), so rows of
+// any width and misaligned views use the same code: the row's last chunk is
+// moved back to end at the row's end (kRagged), its columns already owned by
+// the previous lane are left out of the sums and both lanes store the same
+// gradient there.
+//
+// What bounds it: HBM for full groups (A = 64: 4.6 TB/s), wave instructions
+// (about 150 per step) where lanes of a group idle.  Measured on MI355X, vf_clip:
+//   B = 262,144, A = 64:  169 -> 31 us (a wave per row before: three dependent
+//     passes over each row, one row in flight per wave)
+//   B = 200,000, A = 100: 177 -> 44 us;  B = 20,000, A = 1000: 90 -> 37 us
+//   B = 8,388,608, A = 4: 132 -> 104 us;  B = 2,000,000, A = 16: 64 -> 59 us
+//     (rows padded in LDS before, ~40 instructions per logit)
+//   misaligned B = 1,000,000, A = 18: 70 -> 45 us
+// Steps of 4 (16 logits per lane at most): 8 or 16 steps put more loads in
+// flight per wave but leave fewer waves (A = 64: 31 us at 4 steps, 33 at 8, 35
+// at 16; 2 steps, 39).  128-byte row segments per step: 8 lanes x 2 chunks
+// instead of 16 x 1 measures the same at A = 64 and 38 against 29 us at A = 50,
+// 4 lanes x 2 chunks at A = 24 71 against 48.
+// ---------------------------------------------------------------------------
+template <int kCtrl>
+__device__ __forceinline__ float dpp_move_f(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                               kCtrl, 0xF, 0xF, false));
+}
+
+// max that keeps a NaN (v_maximum3_f32: one instruction, where fmaxf of loaded
+// values needs each quieted first).
+__device__ __forceinline__ float max_nan(float x, float y) {
+  return __builtin_elementwise_maximum(x, y);
+}
+
+// Sum / max over each group of G neighbouring lanes, the same value in every
+// lane of the group (DPP within 16 lanes, the LDS crossbar above).
+template <int G>
+__device__ __forceinline__ float group_sum(float x) {
+  if constexpr (G >= 2) x += dpp_move_f<0xB1>(x);   // quad_perm [1,0,3,2]
+  if constexpr (G >= 4) x += dpp_move_f<0x4E>(x);   // quad_perm [2,3,0,1]
+  if constexpr (G >= 8) x += dpp_move_f<0x141>(x);  // row_half_mirror
+  if constexpr (G >= 16) x += dpp_move_f<0x140>(x); // row_mirror
+  if constexpr (G >= 32) x += __shfl_xor(x, 16, kWave);
+  if constexpr (G >= 64) x += __shfl_xor(x, 32, kWave);
+  return x;
+}
+template <int G>
+__device__ __forceinline__ float group_max(float x) {
+  if constexpr (G >= 2) x = max_nan(x, dpp_move_f<0xB1>(x));
+  if constexpr (G >= 4) x = max_nan(x, dpp_move_f<0x4E>(x));
+  if constexpr (G >= 8) x = max_nan(x, dpp_move_f<0x141>(x));
+  if constexpr (G >= 16) x = max_nan(x, dpp_move_f<0x140>(x));
+  if constexpr (G >= 32) x = max_nan(x, __shfl_xor(x, 16, kWave));
+  if constexpr (G >= 64) x = max_nan(x, __shfl_xor(x, 32, kWave));
+  return x;
+}
+
+template <int VW>
+struct LaneChunk {
+  typedef float type __attribute__((ext_vector_type(VW), aligned(4)));
+};
+template <>
+struct LaneChunk<1> {
+  typedef float type;
+};
+template <int VW, typename T>
+__device__ __forceinline__ float chunk_at(const T& x, int k) {
+  if constexpr (VW == 1) return x;
+  else return x[k];
+}
+
+template <typename ActT, int VW, int G, int C, int I, bool kRagged, bool kVclip>
+__global__ void __launch_bounds__(kBlock) loss_cat_lanes_kernel(LossArgs a, long ntiles) {
+  static_assert(I <= G && G <= kWave, "a step's row is kept by a lane of its group");
+  typedef typename LaneChunk<VW>::type chunk_t;
+  constexpr int kRowsStep = kWave / G;      // rows per step
+  constexpr int kRows = I * kRowsStep;      // rows per wave tile
+  constexpr int kWavesPerBlock = kBlock / kWave;
+  constexpr float kLog2e = 1.4426950408889634f;
+  struct RowBack {
+    float K, inv_s, g_lp;
+    int ai;
+  };
+  __shared__ __attribute__((aligned(16))) RowBack s_back[kWavesPerBlock][kRows];
+  __shared__ float s_ta[kWavesPerBlock][kRows + 1];
+  __shared__ int s_ai[kWavesPerBlock][kRows];
+  const int A = a.A;
+  const float ge = a.ec * a.inv_b;
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wid = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+  const int g = lane / G, q = lane % G;
+  int col[C];  // first column of each chunk as loaded
+  int own[C];  // first column this lane sums (>= A: none)
+#pragma unroll
+  for (int c = 0; c < C; ++c) {
+    own[c] = (q + c * G) * VW;
+    col[c] = std::min(own[c], A - VW);
+  }
+  const bool mine = q < I;               // this lane keeps a row of the tile
+  const int myrow = q * kRowsStep + g;
+  double acc[5] = {0, 0, 0, 0, 0};
+  // (with a.collector, workgroup 0 takes no tiles: it only collects the others' partials)
+  const long c0 = a.collector;
+  const long wstride = ((long)gridDim.x - c0) * kWavesPerBlock;
+  long wt = (long)blockIdx.x < c0 ? ntiles : ((long)blockIdx.x - c0) * kWavesPerBlock + wid;
+  for (; wt < ntiles; wt += wstride) {
+    const long row0 = wt * kRows;
+    // (nothing is stored or summed for rows past the last)
+    const int last = (int)std::min<long>(kRows, a.B - row0) - 1;
+    // byte offsets from the tile's start: rows past the last read its last chunk
+    const int end = (last * A + A - VW) * 4;
+    chunk_t x[I][C];
+    const char* src = reinterpret_cast<const char*>(a.x + row0 * A);
+#pragma unroll
+    for (int i = 0; i < I; ++i)
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+        x[i][c] = __builtin_nontemporal_load(reinterpret_cast<const chunk_t*>(
+            src + (unsigned)std::min(((i * kRowsStep + g) * A + col[c]) * 4, end)));
+    const int lrow = std::min(mine ? myrow : 0, last);
+    const RowIn in = load_row_t<kVclip>(a, row0 + lrow);
+    const int ai = action_index<ActT>(a, row_action_raw<ActT>(a, row0 + lrow));
+    if (mine) s_ai[wid][myrow] = ai;
+    wave_lds_handoff();
+
+    float km = 0.0f, ks = 0.0f, kS = 0.0f;
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const int r = i * kRowsStep + g;
+      float m = chunk_at<VW>(x[i][0], 0);
+#pragma unroll
+      for (int c = 0; c < C; ++c)
+#pragma unroll
+        for (int k = 0; k < VW; ++k) m = max_nan(m, chunk_at<VW>(x[i][c], k));
+      m = group_max<G>(m);
+      const int act = s_ai[wid][r];
+      float s = 0.0f, S = 0.0f;
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        // the action's t goes to the lane that keeps this row (lanes without
+        // it write an unused word: no branch splits the steps)
+        const int rel = act - col[c];
+        float ta = 0.0f, sc, Sc;
+#pragma unroll
+        for (int k = 0; k < VW; ++k) {
+          const float t = chunk_at<VW>(x[i][c], k) - m;
+          ta = rel == k ? t : ta;
+          // (a NaN logit, or an infinite one: t = inf - inf, is NaN in e and
+          // so in s and in the row's whole gradient)
+          float e = __builtin_amdgcn_exp2f(t * kLog2e);
+          const float tc = fmaxf(t, -FLT_MAX);
+          if constexpr (VW == 1) x[i][c] = tc;
+          else x[i][c][k] = tc;
+          if constexpr (kRagged) e = col[c] + k >= own[c] ? e : 0.0f;
+          sc = k == 0 ? e : sc + e;
+          Sc = k == 0 ? e * tc : fmaf(e, tc, Sc);
+        }
+        const bool counted = own[c] < A;
+        s += counted ? sc : 0.0f;
+        S += counted ? Sc : 0.0f;
+        s_ta[wid][rel >= 0 && rel < VW ? r : kRows] = ta;
+      }
+      s = group_sum<G>(s);
+      S = group_sum<G>(S);
+      const bool keep = q == i;
+      km = keep ? m : km;
+      ks = keep ? s : ks;
+      kS = keep ? S : kS;
+    }
+    wave_lds_handoff();
+
+    // Of more than 16 logits per lane the exponentials are formed again for the
+    // gradient rather than kept from the sums (one VGPR per logit): the empty
+    // asm hides from the compiler that t is unchanged.
+    if constexpr (I * C > 4) {
+#pragma unroll
+      for (int i = 0; i < I; ++i)
+#pragma unroll
+        for (int c = 0; c < C; ++c) asm volatile("" : "+v"(x[i][c]));
+    }
+    if (mine) {
+      const float log_s = logf(ks);
+      const float inv_s = 1.0f / ks;
+      const float H = log_s - kS * inv_s;
+      const float lp = ai >= 0 ? s_ta[wid][myrow] - log_s : __builtin_nanf("");
+      const RowOut o = ppo_row_math(a, in, lp);
+      if (myrow <= last) {
+        stnt(o.dval, a.dval + row0 + myrow);
+        accumulate(acc, o, H);
+      }
+      RowBack b;
+      b.K = ge * (H - log_s) - o.g_lp;
+      b.inv_s = inv_s;
+      b.g_lp = o.g_lp;
+      b.ai = ai;
+      s_back[wid][myrow] = b;
+    }
+    wave_lds_handoff();
+
+    char* dst = reinterpret_cast<char*>(a.dx + row0 * A);
+#pragma unroll
+    for (int i = 0; i < I; ++i) {
+      const int r = i * kRowsStep + g;
+      const RowBack b = s_back[wid][r];
+#pragma unroll
+      for (int c = 0; c < C; ++c) {
+        const int rel = b.ai - col[c];
+        chunk_t y;
+#pragma unroll
+        for (int k = 0; k < VW; ++k) {
+          const float t = chunk_at<VW>(x[i][c], k);
+          const float p = __builtin_amdgcn_exp2f(t * kLog2e) * b.inv_s;
+          const float d = fmaf(p, fmaf(ge, t, b.K), rel == k ? b.g_lp : 0.0f);
+          if constexpr (VW == 1) y = d;
+          else y[k] = d;
+        }
+        if (own[c] < A && r <= last)
+          __builtin_nontemporal_store(
+              y, reinterpret_cast<chunk_t*>(dst + (unsigned)((r * A + col[c]) * 4)));
+      }
+    }
+    wave_lds_handoff();
+  }
+  store_scalar_partials(a, acc);
+  if (a.finish) loss_publish<0>(a);
+}
+
+// Lanes form of a row width: kernel and rows per wave tile.
+struct LanesForm {
+  const void* kern;
+  int rows;
+};
+
+template <typename ActT, bool kVclip>
+LanesForm lanes_form(int A) {
+#define PPO_LANES(VW, G, C, I)                                                             \
+  LanesForm{A % VW != 0 ? (const void*)loss_cat_lanes_kernel<ActT, VW, G, C, I, true, kVclip> \
+                        : (const void*)loss_cat_lanes_kernel<ActT, VW, G, C, I, false, kVclip>, \
+            I * (kWave / G)}
+  if (A < 4) return PPO_LANES(1, 4, 1, 4);
+  if (A == 4) return PPO_LANES(4, 1, 1, 1);
+  if (A <= 8) return PPO_LANES(4, 2, 1, 2);
+  if (A <= 16) return PPO_LANES(4, 4, 1, 4);
+  if (A <= 32) return PPO_LANES(4, 8, 1, 4);
+  if (A <= 64) return PPO_LANES(4, 16, 1, 4);
+  if (A <= 128) return PPO_LANES(4, 16, 2, 4);
+  if (A <= 256) return PPO_LANES(4, 32, 2, 4);
+  if (A <= 512) return PPO_LANES(4, 64, 2, 4);
+  if (A <= kMaxLanesWidth) return PPO_LANES(4, 64, 4, 2);
+#undef PPO_LANES
+  return LanesForm{nullptr, 0};
+}
+
+// ---------------------------------------------------------------------------
+// Categorical, A > kMaxLanesWidth: one wave per row (lanes stride the actions).
 // ---------------------------------------------------------------------------
 __device__ __forceinline__ float wave_max_f(float x) {
 #pragma unroll
@@ -1266,7 +1330,8 @@ long row_tiles(long B) { return (B + kBlock - 1) / kBlock; }
 //    8,388,608 in the step 258.2-258.4 against 261.2-262.4 us, step 291.9-292.4
 //    against 295.3-296.0 us; B = 1,048,576 40.4-40.5 against 40.7-41.0 us.
 // So the wave-tile kernels finish in-kernel with a dedicated collector at
-// every batch size, the other forms in-kernel up to kCatFinishRows rows.
+// every batch size, the lanes forms (a dedicated collector as well) up to
+// kCatFinishRows rows.
 // PPO_AMD_CAT_FINISH=0 selects the finaliser launch everywhere (no
 // in-kernel wait: for callers that share the GPU).
 constexpr long kCatFinishRows = 1L << 22;
@@ -1276,8 +1341,20 @@ bool cat_finish_in_kernel() {
   return !(env && env[0] == '0');
 }
 
+// Row widths that take the LDS wave tiles (16-byte-aligned inputs).  Row
+// strides that are no multiple of 4 words read LDS without bank conflicts;
+// measured on MI355X against the lanes form at B = 1,000,000: A = 18 37 against
+// 44 us, 21 42 against 50, 30 55 against 54, 35 61 against 87, 43 74 against 86.
+// Multiples of 4 read 16 bytes per lane, free of conflicts only for an odd
+// number of them per row, and pay where the lanes form leaves 3 or more lanes
+// of 8 idle (A = 20 41 against 45 us, 36 64 against 83, 44 76 against 86; but
+// 12 28 against 28, 28 54 against 52, 40 82 against 81).
+bool cat_wtile(int A) {
+  return A <= kMaxWtileWidth && (A % 4 != 0 || A == 20 || A == 36 || A == 44);
+}
+
 long cat_blocks(long B, int A) {
-  if (A <= kMaxCatRowWidth) return std::min(row_tiles(B), kLossGridCap);
+  if (A <= kNarrowWidth) return std::min((B + kWave - 1) / kWave + 1, kLossGridCap);
   return std::max(1L, std::min((B + 3) / 4, kWaveRowBlocks));
 }
 
@@ -1324,12 +1401,12 @@ int loss_cat_launch(const float* logits, int64_t B, int32_t A, const void* actio
   a.partial = reinterpret_cast<double*>(static_cast<char*>(workspace) + kHeaderBytes);
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
   long blocks = cat_blocks(B, A);
-  const long tiles = row_tiles(B);
-  if (A <= kMaxCatRowWidth) {
+  if (A <= kMaxLanesWidth) {
     const bool vec = aligned(logits, 16) && aligned(dlogits, 16);
-    size_t lds = (size_t)kBlock * (A | 1) * sizeof(float);
     const void* kern;
-    const bool dense = vec && (A % 4) != 0 && A <= 20;
+    int rows = kWave;  // per wave tile
+    constexpr long kWaves = kBlock / kWave;
+    const bool dense = vec && cat_wtile(A);
     const bool vclip = a.use_vclip != 0;
 #define PPO_DENSE(KA, M)                                                                 \
   (actions_are_int64                                                                     \
@@ -1337,7 +1414,15 @@ int loss_cat_launch(const float* logits, int64_t B, int32_t A, const void* actio
                 : (const void*)loss_cat_wtile_kernel<int64_t, KA, M, false>)             \
        : (vclip ? (const void*)loss_cat_wtile_kernel<int32_t, KA, M, true>               \
                 : (const void*)loss_cat_wtile_kernel<int32_t, KA, M, false>))
-    if (dense && A == 2)
+    if (dense && A == 20)
+      kern = PPO_DENSE(20, 20);
+    else if (dense && A == 36)
+      kern = PPO_DENSE(36, 36);
+    else if (dense && A == 44)
+      kern = PPO_DENSE(44, 44);
+    else if (dense && A == 1)
+      kern = PPO_DENSE(1, 1);
+    else if (dense && A == 2)
       kern = PPO_DENSE(2, 2);
     else if (dense && A == 3)
       kern = PPO_DENSE(3, 3);
@@ -1351,42 +1436,51 @@ int loss_cat_launch(const float* logits, int64_t B, int32_t A, const void* actio
       kern = PPO_DENSE(9, 9);
     else if (dense && A == 18)
       kern = PPO_DENSE(18, 18);
-    else if (dense && A <= 4)
-      kern = PPO_DENSE(0, 4);
-    else if (dense && A <= 8)
-      kern = PPO_DENSE(0, 8);
-    else if (dense && A <= 12)
-      kern = PPO_DENSE(0, 12);
+    else if (dense && A <= 11)
+      kern = PPO_DENSE(0, 11);
+    else if (dense && A <= 15)
+      kern = PPO_DENSE(0, 15);
+    else if (dense && A <= 19)
+      kern = PPO_DENSE(0, 19);
+    else if (dense && A <= 23)
+      kern = PPO_DENSE(0, 23);
+    else if (dense && A <= 27)
+      kern = PPO_DENSE(0, 27);
+    else if (dense && A <= 31)
+      kern = PPO_DENSE(0, 31);
+    else if (dense && A <= 35)
+      kern = PPO_DENSE(0, 35);
+    else if (dense && A <= 39)
+      kern = PPO_DENSE(0, 39);
     else if (dense)
-      kern = PPO_DENSE(0, 20);
+      kern = PPO_DENSE(0, 43);
 #undef PPO_DENSE
-    else if (vec && (A + 3) / 4 <= 2)
-      kern = actions_are_int64 ? (const void*)loss_cat_pipe_kernel<int64_t, 2>
-                               : (const void*)loss_cat_pipe_kernel<int32_t, 2>;
-    else if (vec && (A + 3) / 4 <= 5)
-      kern = actions_are_int64 ? (const void*)loss_cat_pipe_kernel<int64_t, 5>
-                               : (const void*)loss_cat_pipe_kernel<int32_t, 5>;
-    else if (vec)
-      kern = actions_are_int64 ? (const void*)loss_cat_kernel<int64_t, true>
-                               : (const void*)loss_cat_kernel<int32_t, true>;
-    else
-      kern = actions_are_int64 ? (const void*)loss_cat_kernel<int64_t, false>
-                               : (const void*)loss_cat_kernel<int32_t, false>;
-    if (dense) lds = (size_t)kBlock * A * sizeof(float);
+    else {
+      const LanesForm f =
+          actions_are_int64 ? (vclip ? lanes_form<int64_t, true>(A) : lanes_form<int64_t, false>(A))
+                            : (vclip ? lanes_form<int32_t, true>(A) : lanes_form<int32_t, false>(A));
+      kern = f.kern;
+      rows = f.rows;
+    }
+    const long wtiles = dense ? B / kWave : (B + rows - 1) / rows;  // (dense: full tiles)
+    const size_t lds = dense ? (size_t)kBlock * A * sizeof(float) : 0;
     // one wave of resident workgroups looping over the tiles
     const long resident = resident_blocks(kern, kBlock, lds, 0);
+    const bool finish =
+        resident > 0 && cat_finish_in_kernel() && (dense || B <= kCatFinishRows);
+    const long need = ((dense ? (B + kWave - 1) / kWave : wtiles) + kWaves - 1) / kWaves;
+    blocks = std::min(blocks, need + (finish ? 1 : 0));
     blocks = std::min(blocks, resident > 0 ? resident : blocks);
     // in-kernel finish (cat_finish_in_kernel), for a grid resident at once
-    if (resident > 0 && cat_finish_in_kernel() && (dense ? blocks > 1 : B <= kCatFinishRows)) {
-      a.collector = dense ? 1 : 0;
+    if (finish && blocks > 1) {
+      a.collector = 1;
       int wst = wait_ctl(a.wc);
       if (wst) return wst;
       a.finish = 1;
       a.epoch = &static_cast<WsHeader*>(workspace)->epoch;
       a.tag_slot = kScalarSlots - 1;
     }
-    const long wfull = B / kWave;  // full wave tiles
-    void* args[] = {&a, const_cast<long*>(dense ? &wfull : &tiles)};
+    void* args[] = {&a, const_cast<long*>(&wtiles)};
     st = hip_status(hipLaunchKernel(kern, grid_of(blocks), dim3(kBlock), args, lds, stream));
     if (st) return st;
   } else {

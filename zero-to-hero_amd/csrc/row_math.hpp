@@ -122,8 +122,9 @@ __device__ __forceinline__ RowOut ppo_row_math(const P& a, const RowIn& in, floa
 // term).  The per-logit exponentials use the hardware exp2 (one multiply by
 // log2(e) and v_exp_f32, relative error ~1e-6 for |z_j - m| <= 20).  ai is
 // the action index, -1 when outside [0, A) (the log-prob is then NaN).
-// Returns the row's loss terms; H receives the row's entropy.
-template <int MAXA, typename P>
+// Returns the row's loss terms; H receives the row's entropy.  MINA <= A <=
+// MAXA: only logits from MINA on are tested against A.
+template <int MAXA, int MINA = 0, typename P>
 __device__ __forceinline__ RowOut cat_row_grad(const P& a, float* zr, int A, int ai, float ge,
                                                const RowIn& in, float& H) {
   constexpr float kLog2e = 1.4426950408889634f;
@@ -131,16 +132,19 @@ __device__ __forceinline__ RowOut cat_row_grad(const P& a, float* zr, int A, int
   float m = -INFINITY;
 #pragma unroll
   for (int j = 0; j < MAXA; ++j)
-    if (j < A) {
+    if (j < MINA || j < A) {
       t[j] = zr[j];
       m = fmaxf(m, t[j]);
     }
   float s = 0.0f, S = 0.0f;
 #pragma unroll
   for (int j = 0; j < MAXA; ++j)
-    if (j < A) {
-      const float tj = fmaxf(t[j] - m, -FLT_MAX);
-      const float ej = __builtin_amdgcn_exp2f(tj * kLog2e);
+    if (j < MINA || j < A) {
+      const float d = t[j] - m;
+      // (a NaN logit, or an infinite one: inf - inf, is NaN in e and so in s
+      // and in the row's whole gradient)
+      const float ej = __builtin_amdgcn_exp2f(d * kLog2e);
+      const float tj = fmaxf(d, -FLT_MAX);
       t[j] = tj;
       e[j] = ej;
       s += ej;
@@ -154,7 +158,7 @@ __device__ __forceinline__ RowOut cat_row_grad(const P& a, float* zr, int A, int
   const float K = ge * (H - log_s) - o.g_lp;
 #pragma unroll
   for (int j = 0; j < MAXA; ++j)
-    if (j < A) zr[j] = (e[j] * inv_s) * fmaf(ge, t[j], K);
+    if (j < MINA || j < A) zr[j] = (e[j] * inv_s) * fmaf(ge, t[j], K);
   if (ai >= 0) zr[ai] += o.g_lp;
   return o;
 }
