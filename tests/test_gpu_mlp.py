@@ -89,6 +89,16 @@ def test_mlp_grads_match_oracle(dev, n, D, H, A, act, B):
     _check(dev, n, D, H, A, act, B, seed=n + 7 * D + H + A)
 
 
+# workgroups per network: 128 * 128 / H; a workgroup's second and third row
+# block, and a last block of 1 and of 15 rows
+@pytest.mark.parametrize("H,B", [(128, 16 * 128 + 1), (128, 2 * 16 * 128 + 15), (64, 16 * 256 + 1),
+                                 (32, 16 * 512 + 15), (16, 2 * 16 * 1024 + 1)])
+# both sides of the tiles of observations (16, then 64) and of actions (16, 32)
+@pytest.mark.parametrize("D,A", [(1, 1), (16, 16), (17, 17), (64, 32)])
+def test_mlp_grads_blocks_and_tiles(dev, H, B, D, A):
+    _check(dev, B + 3, D, H, A, "tanh", B, seed=H + D + A, vf_clip=0.2)
+
+
 def test_mlp_grads_value_clipping_and_int64_actions(dev):
     _check(dev, 512, 4, 64, 2, "tanh", 200, seed=3, vf_clip=0.2, act64=True)
 

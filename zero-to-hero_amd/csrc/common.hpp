@@ -43,6 +43,12 @@ __device__ __forceinline__ double dpp_move(double x) {
   return __builtin_bit_cast(double, r);
 }
 
+template <int kCtrl>
+__device__ __forceinline__ float dpp_move_f(float x) {
+  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
+                                                               kCtrl, 0xF, 0xF, false));
+}
+
 __device__ __forceinline__ double read_lane(double x, int lane) {
   const int2 v = __builtin_bit_cast(int2, x);
   int2 r;

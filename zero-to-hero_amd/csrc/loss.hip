@@ -612,12 +612,6 @@ __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long
 // instead of 16 x 1 measures the same at A = 64 and 38 against 29 us at A = 50,
 // 4 lanes x 2 chunks at A = 24 71 against 48.
 // ---------------------------------------------------------------------------
-template <int kCtrl>
-__device__ __forceinline__ float dpp_move_f(float x) {
-  return __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x),
-                                                               kCtrl, 0xF, 0xF, false));
-}
-
 // max that keeps a NaN (v_maximum3_f32: one instruction, where fmaxf of loaded
 // values needs each quieted first).
 __device__ __forceinline__ float max_nan(float x, float y) {

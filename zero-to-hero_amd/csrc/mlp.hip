@@ -16,19 +16,18 @@
 //
 // At the reference's sizes (4-64-64 or 4-128-128 networks, minibatches of
 // 64-4096 rows) the torch sequence is ~35 small launches per minibatch;
-// here it is two.  Layout: each block of kMlpRows = 16 minibatch rows is
-// handled by two 256-thread workgroups, one per network (the actor's and
-// the critic's forward, loss terms and backward share only the gathered
-// observations).  Observations, activations and row gradients live in LDS;
-// weights are read from global memory (a few KiB to 64 KiB per layer,
-// L2-resident).  Every layer is a set of 16x16 output tiles on the matrix
-// cores (v_mfma_f32_16x16x4f32, one tile per wave at a time): forward tiles
-// over output units, input-gradient tiles over input units, weight-gradient
-// tiles over (output, input) pairs summed over the 16 rows.  All arithmetic
-// is fp32, as torch's; sums over the minibatch differ from torch's GEMM
-// order only by rounding.
+// here it is two.  Layout: blocks of kMlpRows = 16 minibatch rows go to
+// workgroups that each run one network (the actor's and the critic's forward,
+// loss terms and backward share only the gathered observations) and keep its
+// weights and its gradient in registers over all their blocks.  Observations,
+// activations and row gradients pass through LDS.  Every layer is a set of
+// 16x16 output tiles on the matrix cores (v_mfma_f32_16x16x4f32), a wave owning
+// one tile of hidden units.  All arithmetic is fp32, as torch's, the sums over
+// row blocks fp64; they differ from torch's GEMM order only by rounding.
 #include <float.h>
 #include <stdlib.h>
+
+#include <algorithm>
 
 #include "common.hpp"
 #include "adam.hpp"
@@ -178,112 +177,6 @@ __device__ __forceinline__ void fwd_tile(const float* in, int ldin, int K,
   }
 }
 
-// Input-gradient tile of a layer with H inputs: gin[r][k] = act'(h[r][k]) *
-// sum_{m<M} d[r][m] W[m][k] for k in [16 tj, 16 tj + 16).  MC = M at compile
-// time (0: runtime M).  W rows are read along k: coalesced.
-template <int H, int MC, int kAct>
-__device__ __forceinline__ void back_tile(const float* d, int ldd, int M,
-                                          const float* __restrict__ W, int ldw, const float* h,
-                                          float* gin, int tj) {
-  constexpr int ld = act_ld<H>();
-  const int l = threadIdx.x % kWave, i = l % 16, kk = l / 16;
-  const int col = 16 * tj + i;
-  v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-  if constexpr (MC > 0) {
-    float bw[MC / 4];
-#pragma unroll
-    for (int q = 0; q < MC / 4; ++q) bw[q] = W[(long)(4 * q + kk) * ldw + col];
-#pragma unroll
-    for (int q = 0; q < MC / 4; ++q) c = mfma4(d[i * ldd + 4 * q + kk], bw[q], c);
-  } else {
-    for (int m0 = 0; m0 < M; m0 += 4) {
-      const int m = m0 + kk;
-      const float av = m < M ? d[i * ldd + m] : 0.0f;
-      const float bv = m < M ? W[(long)m * ldw + col] : 0.0f;
-      c = mfma4(av, bv, c);
-    }
-  }
-#pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    const int row = 4 * kk + r;
-    gin[row * ld + col] = act_grad<kAct>(c[r], h[row * ld + col]);
-  }
-}
-
-// Weight-gradient tile: gw[m][k] = sum over the 16 rows r of d[r][m] in[r][k]
-// for m in [16 ti, 16 ti + 16) below M and k in [16 tj, 16 tj + 16) below K,
-// written to the workgroup's partial (row-major [M][K]).
-__device__ __forceinline__ void wgrad_tile(const float* d, int ldd, int M, const float* in,
-                                           int ldin, int K, float* __restrict__ gw, int ti,
-                                           int tj) {
-  const int l = threadIdx.x % kWave, i = l % 16, kk = l / 16;
-  const int m = 16 * ti + i, k = 16 * tj + i;
-  v4f c = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-  for (int q = 0; q < 4; ++q) {
-    const int r = 4 * q + kk;
-    const float av = m < M ? d[r * ldd + m] : 0.0f;
-    const float bv = k < K ? in[r * ldin + k] : 0.0f;
-    c = mfma4(av, bv, c);
-  }
-  if (k < K) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int mo = 16 * ti + 4 * kk + r;
-      if (mo < M) gw[(long)mo * K + k] = c[r];
-    }
-  }
-}
-
-// Bias gradient: gb[m] = sum over the 16 rows of d[r][m], threads t < M of a
-// kBlock-thread workgroup.
-template <int kBlock>
-__device__ __forceinline__ void bgrad(const float* d, int ldd, int M, float* __restrict__ gb) {
-  for (int m = threadIdx.x; m < M; m += kBlock) {
-    float s = 0.0f;
-#pragma unroll
-    for (int r = 0; r < kMlpRows; ++r) s += d[r * ldd + m];
-    gb[m] = s;
-  }
-}
-
-// One network's backward from the gradient d3 [16][M3] at its output:
-// phase 1 (dW3, db3, gradient into the second hidden layer), phase 2 (dW2,
-// db2, gradient into the first), phase 3 (dW1, db1).  LDS-only barriers
-// between the phases (the gradient partials go to global memory and are read
-// by the next kernel); phase 3 leaves without one (the caller's next phase
-// must not write g1 before a barrier).
-template <int H, int kAct, int kBlock>
-__device__ __forceinline__ void net_backward(const MlpNet& net, const NetOffsets& o, float* gp,
-                                             const float* d3, int ld3, int M3, const float* x,
-                                             int D, const float* h1, const float* h2, float* g1,
-                                             float* g2) {
-  constexpr int ld = act_ld<H>();
-  constexpr int NT = H / 16;
-  const int w = threadIdx.x / kWave;
-  constexpr int kWaves = kBlock / kWave;
-  const int MT3 = (M3 + 15) / 16;
-  // phase 1
-  for (int t = w; t < MT3 * NT + NT; t += kWaves) {
-    if (t < MT3 * NT) wgrad_tile(d3, ld3, M3, h2, ld, H, gp + o.w[2], t / NT, t % NT);
-    else back_tile<H, 0, kAct>(d3, ld3, M3, net.w[2], net.ldw[2], h2, g2, t - MT3 * NT);
-  }
-  bgrad<kBlock>(d3, ld3, M3, gp + o.b[2]);
-  lds_barrier();
-  // phase 2
-  for (int t = w; t < NT * NT + NT; t += kWaves) {
-    if (t < NT * NT) wgrad_tile(g2, ld, H, h1, ld, H, gp + o.w[1], t / NT, t % NT);
-    else back_tile<H, H, kAct>(g2, ld, H, net.w[1], net.ldw[1], h1, g1, t - NT * NT);
-  }
-  bgrad<kBlock>(g2, ld, H, gp + o.b[1]);
-  lds_barrier();
-  // phase 3
-  const int DT = (D + 15) / 16;
-  for (int t = w; t < NT * DT; t += kWaves)
-    wgrad_tile(g1, ld, H, x, kXld, D, gp + o.w[0], t / DT, t % DT);
-  bgrad<kBlock>(g1, ld, H, gp + o.b[0]);
-}
-
 // Forward of both networks for the workgroup's 16 rows x (observations in
 // s_x): hidden activations into a1/a2 (actor) and c1/c2 (critic), logits into
 // z [16][kZld], values into v [16].  Tiles (network, column tile) over the
@@ -381,145 +274,458 @@ __device__ __forceinline__ MlpNet stage_net(const MlpNet& g, int D, int O, float
   return n;
 }
 
-// Forward of one network for the workgroup's 16 rows (observations in x):
-// hidden activations into h1/h2, the O outputs into out [16][ldout].  Column
-// tiles over the waves; LDS-only barriers between the layers and after the
-// last.  kBlock threads.
-template <int H, int kAct, int kBlock>
-__device__ __forceinline__ void net_forward(const MlpNet& net, const float* x, int D, int O,
-                                            float* h1, float* h2, float* out, int ldout) {
-  constexpr int ld = act_ld<H>();
-  constexpr int NT = H / 16;
-  constexpr int kWaves = kBlock / kWave;
-  const int w = threadIdx.x / kWave;
-  for (int t = w; t < NT; t += kWaves)
-    fwd_tile<0, kAct>(x, kXld, D, net.w[0], net.ldw[0], net.b[0], H, h1, ld, t);
-  lds_barrier();
-  for (int t = w; t < NT; t += kWaves)
-    fwd_tile<H, kAct>(h1, ld, H, net.w[1], net.ldw[1], net.b[1], H, h2, ld, t);
-  lds_barrier();
-  for (int t = w; t < (O + 15) / 16; t += kWaves)
-    fwd_tile<H, -1>(h2, ld, H, net.w[2], net.ldw[2], net.b[2], O, out, ldout, t);
-  lds_barrier();
+__device__ __forceinline__ float quad_sum(float x) {
+  x += dpp_move_f<0xB1>(x);  // quad_perm [1,0,3,2]
+  x += dpp_move_f<0x4E>(x);  // quad_perm [2,3,0,1]
+  return x;
 }
 
-// One minibatch block of 16 rows is handled by two workgroups, 2b (actor)
-// and 2b + 1 (critic): the networks share nothing but the gathered
-// observations, so each workgroup runs one network's forward, its part of
-// the per-row loss and its backward.  They write disjoint parts of the
-// block's partials (the actor's and the critic's parameter columns of
-// gpart row b; the policy / entropy / kl / clip-fraction sums and the value
-// sum of spart column b), so the reduction sees exactly the values one
-// workgroup doing both networks would leave.
+// cat_row_grad with a row in a quad of lanes (lane q of the quad holds logits
+// 16 c + 4 q .. + 3 of its row, c < MT; 16-byte-aligned zr with 16 MT logits
+// of room): the same formulas, the row's sums over the quad, its scalar terms
+// formed in all four lanes.  Logits past A and rows that are not `valid` get
+// gradient 0.
+template <int MT, typename P>
+__device__ __forceinline__ RowOut cat_quad_grad(const P& a, float* zr, int A, int ai, float ge,
+                                                const RowIn& in, bool valid, float& H) {
+  constexpr float kLog2e = 1.4426950408889634f;
+  const int q = threadIdx.x % 4;
+  float t[MT][4], e[MT][4];
+  float m = -INFINITY;
+#pragma unroll
+  for (int c = 0; c < MT; ++c) {
+    const float4 z = *reinterpret_cast<const float4*>(zr + 16 * c + 4 * q);
+    t[c][0] = z.x;
+    t[c][1] = z.y;
+    t[c][2] = z.z;
+    t[c][3] = z.w;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      t[c][k] = 16 * c + 4 * q + k < A ? t[c][k] : -INFINITY;
+      m = fmaxf(m, t[c][k]);
+    }
+  }
+  m = fmaxf(m, dpp_move_f<0xB1>(m));
+  m = fmaxf(m, dpp_move_f<0x4E>(m));
+  float s = 0.0f, S = 0.0f, ta = 0.0f;
+#pragma unroll
+  for (int c = 0; c < MT; ++c)
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const bool in_row = 16 * c + 4 * q + k < A;
+      const float d = t[c][k] - m;
+      ta += 16 * c + 4 * q + k == ai ? d : 0.0f;
+      // (a NaN logit is NaN in e and so in s and in the row's whole gradient)
+      e[c][k] = in_row ? __builtin_amdgcn_exp2f(d * kLog2e) : 0.0f;
+      t[c][k] = fmaxf(d, -FLT_MAX);
+      s += e[c][k];
+      S = fmaf(e[c][k], t[c][k], S);
+    }
+  s = quad_sum(s);
+  S = quad_sum(S);
+  ta = quad_sum(ta);
+  const float log_s = logf(s);
+  const float inv_s = 1.0f / s;
+  H = log_s - S * inv_s;
+  const float lp = ai >= 0 ? ta - log_s : __builtin_nanf("");
+  const RowOut o = ppo_row_math(a, in, lp);
+  const float K = ge * (H - log_s) - o.g_lp;
+#pragma unroll
+  for (int c = 0; c < MT; ++c) {
+    float y[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int col = 16 * c + 4 * q + k;
+      const float d = (e[c][k] * inv_s) * fmaf(ge, t[c][k], K);
+      y[k] = col < A && valid ? (col == ai ? d + o.g_lp : d) : 0.0f;
+    }
+    *reinterpret_cast<float4*>(zr + 16 * c + 4 * q) = make_float4(y[0], y[1], y[2], y[3]);
+  }
+  return o;
+}
+
+// One network's minibatch gradient: the grid's even workgroups run the actor,
+// the odd ones the critic (the networks share nothing but the gathered
+// observations).  Workgroup g of a network takes row blocks g, g + G, ... of 16
+// rows (G = a.nblocks workgroups per network) and keeps the gradient of all its
+// blocks in registers, so a minibatch leaves G partial gradients whatever its
+// size.
 //
-// Workgroups of grad_block<H>() threads: at H = 128 (weights read from
-// global memory, not staged in LDS) 16 waves, so that each wave takes a
-// quarter of the tiles it would among 4 (measured on MI355X, minibatches of
-// 128 rows: 20.1 -> 16.0 us per launch).
+// One wave per 16-column tile of the hidden layers (H / 16 waves).  Wave w's
+// weights stay in registers in the matrix core's operand layout for all its
+// blocks: W1 and W2 rows of its 16 output units (forward), W2 and W3 columns of
+// its 16 units (input gradients).  A product's result (lane l: rows 4 (l / 16) + r,
+// column l % 16) is at once the operand that the weight gradients need (4 rows
+// contracted per step in that order), so
+//   dW2[:, tile w] = g2^T h1,  dW3[:, tile w] = dz^T h2   (h from registers)
+//   dW1[tile w, :] = g1^T x                               (g1 from registers)
+// and only the other operand goes through LDS: row-major with stride H + 4,
+// 16-byte reads for the layer products (contraction order permuted, lane group
+// l / 16 taking 4 consecutive units), 4-byte column reads for the weight
+// gradients, both free of bank conflicts.  Each 16-row product is added to fp64
+// accumulators (fp32 within 16 rows, as the sum over row blocks always was).
+// The next block's observations and loss inputs are loaded during the current
+// block's layers.
+//
+// What bounds it: large minibatches, the matrix cores (half busy at H = 128: 5.7
+// us per block of 16 rows, of which the products take 3) and the five barriers
+// per block; small ones, the chain of dependent loads (index, row, then the
+// layers).  Measured on MI355X against one 16-row block per workgroup, its
+// gradients written out per block (us, gradient kernel + reduction):
+//   32,768 rows, 8-128-128-4 relu  241 + 72 -> 106 + 6.5  (partials 313 -> 19 MB)
+//   32,768 rows, 8-64-64-4 tanh    121 -> 55 for both
+//   4096 rows, 4-64-64-2 tanh      21.5 -> 20.4 for both
+//   256 rows, 4-64-64-2 tanh       12.4 -> 8.5 (gradient kernel)
 template <int H>
 constexpr int grad_block() {
-  return H == 128 ? 1024 : kMlpBlock;
+  return H / 16 * kWave;
 }
 
-template <int H, int kAct>
-__global__ void __launch_bounds__(grad_block<H>()) mlp_cat_grad_kernel(MlpArgs a) {
-  constexpr int kBlock = grad_block<H>();
+//
+// At H = 128 the transposed operand of g2 W2 comes from an LDS copy of W2: held
+// in registers as well it would spill (256 VGPRs at 2 waves per SIMD).  H = 64
+// at 4 waves per SIMD (128 VGPRs) spills and takes 17 us instead of 12.
+template <int H, int kAct, int DT, int MT>
+__global__ void __launch_bounds__(grad_block<H>(), H >= 64 ? 2 : 3) mlp_cat_grad_kernel(MlpArgs a) {
   constexpr int R = kMlpRows;
-  constexpr int ld = act_ld<H>();
-  __shared__ float s_x[R * kXld];
-  __shared__ float s_h1[R * ld], s_h2[R * ld];
-  __shared__ float s_g1[R * ld], s_g2[R * ld];
-  __shared__ float s_z[R * kZld];
-  __shared__ float s_v[R];
-  __shared__ long s_row[R];
+  constexpr int NT = H / 16;
+  constexpr int kThreads = grad_block<H>();
+  constexpr int ld = H + 4;
+  constexpr int ldx = 16 * DT + 4;
+  constexpr int ldz = 16 * MT + 4;
+  constexpr int kXPer = (R * 16 * DT + kThreads - 1) / kThreads;
+  __shared__ __attribute__((aligned(16))) float s_x[2][R * ldx];
+  __shared__ __attribute__((aligned(16))) float s_h1[R * ld], s_h2[R * ld], s_g2[R * ld];
+  __shared__ __attribute__((aligned(16))) float s_z[R * ldz];
+  __shared__ __attribute__((aligned(16))) float s_w3[16 * MT * ld];
+  __shared__ float s_b3[16 * MT];
+  constexpr bool kW2Lds = H >= 128;
+  __shared__ __attribute__((aligned(16))) float s_w2[kW2Lds ? H * ld : 1];
+  __shared__ long s_row[2][R];
+  __shared__ double s_acc[kMlpSums][R];
 
   const int tid = threadIdx.x;
+  const int lane = tid % kWave, i = lane % 16, kk = lane / 16;
+  const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
   const bool critic = (blockIdx.x & 1u) != 0u;
-  const long blk = (long)(blockIdx.x >> 1);
-  const long row0 = blk * R;
-  const int D = a.D, A = a.A;
-  // this workgroup's network, its weights staged in LDS when they fit
-  constexpr bool kStage = H <= kMlpLdsMaxH;
-  __shared__ __attribute__((aligned(16))) float s_w[kStage ? net_lds_floats<H>() : 1];
-  static_assert(!kStage || kBlock == kMlpBlock, "stage_net strides by kMlpBlock");
-  MlpNet net = critic ? a.critic : a.actor;
-  if constexpr (kStage) net = stage_net<H>(net, D, critic ? 1 : A, s_w);
-  // the loss inputs of row `tid` (tid < R) are loaded now, ahead of the
-  // forward pass that precedes their use
-  RowIn rin = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
-  long raw_act = 0;
-  if (tid < R) {
-    const long i = row0 + tid;
-    const long src = i < a.B ? (a.idx ? (long)a.idx[i] : i) : -1;
-    s_row[tid] = src;
-    const long sc = src >= 0 ? src : 0;
-    if (critic) {
-      rin.ret = a.ret[sc];
-      rin.vo = a.use_vclip ? a.old_val[sc] : 0.0f;
-    } else {
-      rin.old_lp = a.old_lp[sc];
-      rin.adv = a.adv[sc];
-      raw_act = a.act64 ? (long)reinterpret_cast<const int64_t*>(a.actions)[sc]
-                        : (long)reinterpret_cast<const int32_t*>(a.actions)[sc];
-    }
-  }
-  lds_barrier();
-  // gather the observation rows (padding rows past B are zeros)
-  for (int e = tid; e < R * D; e += kBlock) {
-    const int r = e / D, c = e - (e / D) * D;
-    const long src = s_row[r];
-    s_x[r * kXld + c] = (src >= 0 && src < a.n) ? a.obs[src * D + c] : 0.0f;
-  }
-  lds_barrier();
+  const long g = (long)(blockIdx.x >> 1);
+  const long G = a.nblocks;
+  const long nblk = (a.B + R - 1) / R;
+  const int D = a.D;
+  const int M3 = critic ? 1 : a.A;
+  const int mt = critic ? 1 : MT;
+  const MlpNet net = critic ? a.critic : a.actor;
+  const NetOffsets o = critic ? a.oc : a.oa;
 
-  if (critic) net_forward<H, kAct, kBlock>(net, s_x, D, 1, s_h1, s_h2, s_v, 1);
-  else net_forward<H, kAct, kBlock>(net, s_x, D, A, s_h1, s_h2, s_z, kZld);
-
-  // loss rows: logits -> dlogits in place (actor), value -> dvalue in place
-  // (critic; the value terms do not depend on the log-prob, which is given
-  // its old value here)
-  double acc[kMlpSums] = {0.0, 0.0, 0.0, 0.0, 0.0};
-  if (tid < R) {
-    const long src = s_row[tid];
-    float* zr = s_z + tid * kZld;
-    if (src >= 0) {
-      if (critic) {
-        RowIn in = rin;
-        in.v = s_v[tid];
-        const RowOut o = ppo_row_math(a, in, in.old_lp);
-        s_v[tid] = o.dval;
-        acc[1] = (double)o.vl;
-      } else {
-        const int ai = (raw_act >= 0 && raw_act < A) ? (int)raw_act : -1;
-        float H_ent;
-        const RowOut o = cat_row_grad<kMlpMaxA>(a, zr, A, ai, a.ec * a.inv_b, rin, H_ent);
-        acc[0] = (double)o.pol;
-        acc[2] = (double)H_ent;
-        acc[3] = (double)o.kl;
-        acc[4] = (double)o.clipped;
-      }
-    } else if (critic) {
-      s_v[tid] = 0.0f;
-    } else {
-      for (int j = 0; j < A; ++j) zr[j] = 0.0f;
-    }
-  }
-  block_sum<kMlpSums>(acc);  // its barriers also publish s_z / s_v
-  if (tid == 0) {
-    if (critic) {
-      a.spart[1 * a.nblocks + blk] = acc[1];
-    } else {
-      a.spart[0 * a.nblocks + blk] = acc[0];
+  // row index of row r of block b: -1 past the minibatch
+  auto row_src = [&](long b, int r) -> long {
+    const long k = b * R + r;
+    return b < nblk && k < a.B ? (a.idx ? (long)a.idx[k] : k) : -1;
+  };
+  auto in_range = [&](long src) { return src >= 0 && src < a.n; };
+  float xr[kXPer];
+  auto load_x = [&](const long* rows) {
 #pragma unroll
-      for (int k = 2; k < kMlpSums; ++k) a.spart[(long)k * a.nblocks + blk] = acc[k];
+    for (int q = 0; q < kXPer; ++q) {
+      const int e = tid + q * kThreads;
+      const int r = e / (16 * DT), c = e % (16 * DT);
+      const long src = r < R ? rows[r] : -1;
+      xr[q] = c < D && in_range(src) ? a.obs[src * D + c] : 0.0f;
     }
+  };
+  auto store_x = [&](float* x) {
+#pragma unroll
+    for (int q = 0; q < kXPer; ++q) {
+      const int e = tid + q * kThreads;
+      const int r = e / (16 * DT), c = e % (16 * DT);
+      if (r < R) x[r * ldx + c] = xr[q];
+    }
+  };
+
+  long src0 = -1, src1 = -1;
+  if (tid < R) {
+    src0 = row_src(g, tid);
+    src1 = row_src(g + G, tid);
+  }
+  // this wave's weights, in flight while the first block's rows are fetched
+  const int n = 16 * w + i;  // the lane's unit in both hidden layers
+  float w1[DT][4], w2[NT][4], w2t[kW2Lds ? 1 : NT][4];
+#pragma unroll
+  for (int q = 0; q < NT; ++q) {
+    const float4 t = *reinterpret_cast<const float4*>(net.w[1] + n * H + 16 * q + 4 * kk);
+    w2[q][0] = t.x;
+    w2[q][1] = t.y;
+    w2[q][2] = t.z;
+    w2[q][3] = t.w;
+  }
+#pragma unroll
+  for (int q = 0; q < DT; ++q)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const int k = 16 * q + 4 * kk + e;
+      w1[q][e] = k < D ? net.w[0][n * D + k] : 0.0f;
+    }
+  if constexpr (kW2Lds) {
+    // (the wave's own rows, from the registers just loaded)
+#pragma unroll
+    for (int q = 0; q < NT; ++q)
+      *reinterpret_cast<float4*>(s_w2 + n * ld + 16 * q + 4 * kk) =
+          make_float4(w2[q][0], w2[q][1], w2[q][2], w2[q][3]);
+  } else {
+#pragma unroll
+    for (int q = 0; q < NT; ++q)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) w2t[q][e] = net.w[1][(16 * q + 4 * kk + e) * H + n];
+  }
+  const float b1 = net.b[0][n], b2 = net.b[1][n];
+  if (tid < R) {
+    s_row[0][tid] = src0;
+    s_row[1][tid] = src1;
+  }
+  for (int e = tid; e < 16 * MT * (H / 4); e += kThreads) {
+    const int m = e / (H / 4), c = 4 * (e % (H / 4));
+    *reinterpret_cast<float4*>(s_w3 + m * ld + c) =
+        m < M3 ? *reinterpret_cast<const float4*>(net.w[2] + m * H + c)
+               : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+  }
+  if (tid < R) {
+#pragma unroll
+    for (int k = 0; k < kMlpSums; ++k) s_acc[k][tid] = 0.0;
+  }
+  // (the critic writes only the first 16 output columns)
+  for (int e = tid; e < R * ldz; e += kThreads) s_z[e] = 0.0f;
+  if (tid < 16 * MT) s_b3[tid] = tid < M3 ? net.b[2][tid] : 0.0f;
+  lds_barrier();
+  load_x(s_row[0]);
+  store_x(s_x[0]);
+  lds_barrier();
+
+  double gw1[DT][4], gw2[NT][4], gw3[MT][4];
+  double gb1 = 0.0, gb2 = 0.0, gb3 = 0.0;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+#pragma unroll
+    for (int q = 0; q < DT; ++q) gw1[q][r] = 0.0;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) gw2[q][r] = 0.0;
+#pragma unroll
+    for (int q = 0; q < MT; ++q) gw3[q][r] = 0.0;
+  }
+  const v4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+  // sum over 16 q + 4 kk + e of row i of an LDS operand times registers
+  auto product = [&](const float* in, int ldin, auto& wr, int q, v4f c) {
+    const float4 t = *reinterpret_cast<const float4*>(in + i * ldin + 16 * q + 4 * kk);
+    c = mfma4(t.x, wr[q][0], c);
+    c = mfma4(t.y, wr[q][1], c);
+    c = mfma4(t.z, wr[q][2], c);
+    return mfma4(t.w, wr[q][3], c);
+  };
+
+  // the same with the columns n of an LDS matrix (row stride ld)
+  auto product_t = [&](const float* in, int ldin, const float* wt, int q, v4f c) {
+    const float4 t = *reinterpret_cast<const float4*>(in + i * ldin + 16 * q + 4 * kk);
+    const float* wr = wt + (16 * q + 4 * kk) * ld + n;
+    c = mfma4(t.x, wr[0], c);
+    c = mfma4(t.y, wr[ld], c);
+    c = mfma4(t.z, wr[2 * ld], c);
+    return mfma4(t.w, wr[3 * ld], c);
+  };
+
+  int buf = 0;
+  for (long b = g; b < nblk; b += G, buf ^= 1) {
+    const float* x = s_x[buf];
+    const bool more = b + G < nblk;
+    // the next block's rows, the indices of the one after it, and (wave 0, a
+    // quad of lanes per row) this block's loss inputs
+    long src2 = -1;
+    RowIn rin = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
+    int raw_act = 0;
+    bool valid = false;
+    if (more) {
+      load_x(s_row[buf ^ 1]);
+      if (tid < R) src2 = row_src(b + 2 * G, tid);
+    }
+    if (w == 0) {
+      const long src = s_row[buf][lane / 4];
+      valid = src >= 0;
+      const long sc = in_range(src) ? src : 0;
+      if (critic) {
+        rin.ret = a.ret[sc];
+        rin.vo = a.use_vclip ? a.old_val[sc] : 0.0f;
+      } else {
+        rin.old_lp = a.old_lp[sc];
+        rin.adv = a.adv[sc];
+        const long act = a.act64 ? (long)reinterpret_cast<const int64_t*>(a.actions)[sc]
+                                 : (long)reinterpret_cast<const int32_t*>(a.actions)[sc];
+        raw_act = act >= 0 && act < M3 ? (int)act : -1;
+      }
+    }
+    // layer 1
+    v4f c = zero;
+#pragma unroll
+    for (int q = 0; q < DT; ++q) c = product(x, ldx, w1, q, c);
+    float h1[4], h2[4], g2[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      h1[r] = act_fwd<kAct>(c[r] + b1);
+      s_h1[(4 * kk + r) * ld + n] = h1[r];
+    }
+    lds_barrier();
+    // layer 2
+    c = zero;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) c = product(s_h1, ld, w2, q, c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      h2[r] = act_fwd<kAct>(c[r] + b2);
+      s_h2[(4 * kk + r) * ld + n] = h2[r];
+    }
+    lds_barrier();
+    // layer 3: wave t forms output tile t (outputs past M3 come out 0)
+    for (int t = w; t < mt; t += NT) {
+      v4f z = zero;
+      const float* wr = s_w3 + (16 * t + i) * ld;
+#pragma unroll
+      for (int q = 0; q < NT; ++q) {
+        const float4 hv = *reinterpret_cast<const float4*>(s_h2 + i * ld + 16 * q + 4 * kk);
+        const float4 wv = *reinterpret_cast<const float4*>(wr + 16 * q + 4 * kk);
+        z = mfma4(hv.x, wv.x, z);
+        z = mfma4(hv.y, wv.y, z);
+        z = mfma4(hv.z, wv.z, z);
+        z = mfma4(hv.w, wv.w, z);
+      }
+      const float b3 = s_b3[16 * t + i];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) s_z[(4 * kk + r) * ldz + 16 * t + i] = z[r] + b3;
+    }
+    lds_barrier();
+    // loss rows: outputs -> their gradients in place (the value terms do not
+    // depend on the log-prob, which is given its old value here)
+    if (w == 0) {
+      const int q4 = lane % 4;
+      float* zr = s_z + (lane / 4) * ldz;
+      if (critic) {
+        rin.v = zr[0];
+        const RowOut out = ppo_row_math(a, rin, rin.old_lp);
+        if (q4 == 0) {
+          zr[0] = valid ? out.dval : 0.0f;
+          if (valid) s_acc[1][lane / 4] += (double)out.vl;
+        }
+      } else {
+        float H_ent;
+        const RowOut out = cat_quad_grad<MT>(a, zr, M3, raw_act, a.ec * a.inv_b, rin, valid, H_ent);
+        if (q4 == 0 && valid) {
+          s_acc[0][lane / 4] += (double)out.pol;
+          s_acc[2][lane / 4] += (double)H_ent;
+          s_acc[3][lane / 4] += (double)out.kl;
+          s_acc[4][lane / 4] += (double)out.clipped;
+        }
+      }
+    }
+    lds_barrier();
+    // gradient into the second hidden layer, dW3, db3
+    c = zero;
+#pragma unroll
+    for (int q = 0; q < MT; ++q) c = product_t(s_z, ldz, s_w3, q, c);
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      g2[r] = act_grad<kAct>(c[r], h2[r]);
+      s_g2[(4 * kk + r) * ld + n] = g2[r];
+    }
+    gb2 += (double)((g2[0] + g2[1]) + (g2[2] + g2[3]));
+    if (more) store_x(s_x[buf ^ 1]);
+    if (tid < R) s_row[buf][tid] = src2;
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < MT; ++q) {
+      v4f t = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t = mfma4(s_z[(4 * kk + r) * ldz + 16 * q + i], h2[r], t);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gw3[q][r] += (double)t[r];
+    }
+    if (tid < 16 * MT) {
+      float t = 0.0f;
+#pragma unroll
+      for (int r = 0; r < R; ++r) t += s_z[r * ldz + tid];
+      gb3 += (double)t;
+    }
+    // gradient into the first hidden layer
+    c = zero;
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      if constexpr (kW2Lds) c = product_t(s_g2, ld, s_w2, q, c);
+      else c = product(s_g2, ld, w2t, q, c);
+    }
+    float g1[4];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) g1[r] = act_grad<kAct>(c[r], h1[r]);
+    gb1 += (double)((g1[0] + g1[1]) + (g1[2] + g1[3]));
+    // dW2, dW1
+#pragma unroll
+    for (int q = 0; q < NT; ++q) {
+      v4f t = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t = mfma4(s_g2[(4 * kk + r) * ld + 16 * q + i], h1[r], t);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gw2[q][r] += (double)t[r];
+    }
+#pragma unroll
+    for (int q = 0; q < DT; ++q) {
+      v4f t = zero;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) t = mfma4(g1[r], x[(4 * kk + r) * ldx + 16 * q + i], t);
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gw1[q][r] += (double)t[r];
+    }
+    // (what the next block overwrites before its first barrier, s_h1, was
+    // last read two barriers ago; s_x and s_row are double-buffered)
   }
 
-  float* gp = a.gpart + blk * a.P;
-  if (critic)
-    net_backward<H, kAct, kBlock>(net, a.oc, gp, s_v, 1, 1, s_x, D, s_h1, s_h2, s_g1, s_g2);
-  else
-    net_backward<H, kAct, kBlock>(net, a.oa, gp, s_z, kZld, A, s_x, D, s_h1, s_h2, s_g1, s_g2);
+  // loss sums over the 16 rows of all blocks (s_acc is wave 0's own)
+  if (w == 0) {
+    double acc[kMlpSums];
+#pragma unroll
+    for (int k = 0; k < kMlpSums; ++k) acc[k] = wave_sum(lane < R ? s_acc[k][lane % R] : 0.0);
+    if (lane == 0) {
+      if (critic) {
+        a.spart[1 * G + g] = acc[1];
+      } else {
+        a.spart[0 * G + g] = acc[0];
+#pragma unroll
+        for (int k = 2; k < kMlpSums; ++k) a.spart[(long)k * G + g] = acc[k];
+      }
+    }
+  }
+  float* gp = a.gpart + g * a.P;
+#pragma unroll
+  for (int q = 0; q < NT; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) gp[o.w[1] + (16 * q + 4 * kk + r) * H + n] = (float)gw2[q][r];
+#pragma unroll
+  for (int q = 0; q < DT; ++q) {
+    const int k = 16 * q + i;
+    if (k < D) {
+#pragma unroll
+      for (int r = 0; r < 4; ++r) gp[o.w[0] + (16 * w + 4 * kk + r) * D + k] = (float)gw1[q][r];
+    }
+  }
+#pragma unroll
+  for (int q = 0; q < MT; ++q)
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+      const int m = 16 * q + 4 * kk + r;
+      if (m < M3) gp[o.w[2] + m * H + n] = (float)gw3[q][r];
+    }
+  gb1 += __shfl_xor(gb1, 16, kWave);
+  gb2 += __shfl_xor(gb2, 16, kWave);
+  gb1 += __shfl_xor(gb1, 32, kWave);
+  gb2 += __shfl_xor(gb2, 32, kWave);
+  if (kk == 0) {
+    gp[o.b[0] + n] = (float)gb1;
+    gp[o.b[1] + n] = (float)gb2;
+  }
+  if (tid < M3) gp[o.b[2] + tid] = (float)gb3;
 }
 
 // Action selection through both networks (ppo.py:65-79 for N observations):
@@ -958,6 +1164,13 @@ NetOffsets net_offsets(long base, int D, int H, int O) {
   return o;
 }
 
+// Workgroups per network of the gradient kernel, at most: both networks' fill
+// the chip once (H / 16 waves each).  Measured on MI355X, us per call, at
+// half / this / twice the number: 32,768 rows H = 128 196 / 115 / 123, H = 64
+// 74 / 55 / 61, H = 32 43 / 30 / 39, H = 16 26 / 25 / 36.
+constexpr long grad_groups(int H) { return 128L * 128 / H; }
+
+
 struct MlpLayout {
   long P, nblocks, rblocks;
   int threads;  // of the gradient kernel's workgroups
@@ -968,8 +1181,8 @@ struct MlpLayout {
 MlpLayout mlp_layout(long B, int D, int H, int A) {
   MlpLayout l;
   l.P = mlp_params(D, H, A) + mlp_params(D, H, 1);
-  l.threads = H == 128 ? grad_block<128>() : kMlpBlock;
-  l.nblocks = (B + kMlpRows - 1) / kMlpRows;
+  l.threads = H / 16 * kWave;
+  l.nblocks = std::min((B + kMlpRows - 1) / kMlpRows, grad_groups(H));
   const NetOffsets o[2] = {net_offsets(0, D, H, A), net_offsets(mlp_params(D, H, A), D, H, 1)};
   const int outs[2] = {A, 1};
   l.tblk[0] = 0;
@@ -989,13 +1202,22 @@ MlpLayout mlp_layout(long B, int D, int H, int A) {
   return l;
 }
 
+template <int H, int kAct>
+const void* mlp_kernel_tiles(int D, int A) {
+  if (D <= 16)
+    return A <= 16 ? (const void*)mlp_cat_grad_kernel<H, kAct, 1, 1>
+                   : (const void*)mlp_cat_grad_kernel<H, kAct, 1, 2>;
+  return A <= 16 ? (const void*)mlp_cat_grad_kernel<H, kAct, 4, 1>
+                 : (const void*)mlp_cat_grad_kernel<H, kAct, 4, 2>;
+}
+
 template <int kAct>
-const void* mlp_kernel_act(int H) {
+const void* mlp_kernel_act(int H, int D, int A) {
   switch (H) {
-    case 16: return (const void*)mlp_cat_grad_kernel<16, kAct>;
-    case 32: return (const void*)mlp_cat_grad_kernel<32, kAct>;
-    case 64: return (const void*)mlp_cat_grad_kernel<64, kAct>;
-    case 128: return (const void*)mlp_cat_grad_kernel<128, kAct>;
+    case 16: return mlp_kernel_tiles<16, kAct>(D, A);
+    case 32: return mlp_kernel_tiles<32, kAct>(D, A);
+    case 64: return mlp_kernel_tiles<64, kAct>(D, A);
+    case 128: return mlp_kernel_tiles<128, kAct>(D, A);
     default: return nullptr;
   }
 }
@@ -1088,8 +1310,8 @@ int mlp_setup(const ppo_mlp3_f32* actor, const ppo_mlp3_f32* critic, int32_t obs
   if (B < 0 || n < 0) return PPO_ERR_INVALID_ARG;
   if (obs_dim <= 0 || obs_dim > kMlpMaxIn || A <= 0 || A > kMlpMaxA) return PPO_ERR_UNSUPPORTED;
   if (activation != PPO_ACT_RELU && activation != PPO_ACT_TANH) return PPO_ERR_INVALID_ARG;
-  const void* k = activation == PPO_ACT_TANH ? mlp_kernel_act<PPO_ACT_TANH>(hidden)
-                                             : mlp_kernel_act<PPO_ACT_RELU>(hidden);
+  const void* k = activation == PPO_ACT_TANH ? mlp_kernel_act<PPO_ACT_TANH>(hidden, obs_dim, A)
+                                             : mlp_kernel_act<PPO_ACT_RELU>(hidden, obs_dim, A);
   if (!k) return PPO_ERR_UNSUPPORTED;
   if (!mlp_net_ok(actor) || !mlp_net_ok(critic) || !params || !scalars_out)
     return PPO_ERR_INVALID_ARG;
@@ -1148,17 +1370,29 @@ int mlp_setup(const ppo_mlp3_f32* actor, const ppo_mlp3_f32* critic, int32_t obs
   return PPO_OK;
 }
 
-// The gradient kernel (two workgroups per 16-row block) and the reduction.
+// Waves of the reduction's workgroups.  Few partial rows need few loads in
+// flight.  From kRedWideRows on, 16 waves, but 8 where that many 1024-thread
+// workgroups would run in two rounds (H = 128: 590 workgroups, 128 rows, 9.6 ->
+// 6.5 us).  The 8-wave form never joins the Adam update: with 590 workgroups
+// meeting at its barrier the joint kernel takes 23 us, the two launches 14.5.
+int reduce_waves(const MlpLayout& l) {
+  if (l.nblocks < kRedWideRows) return 4;
+  return l.rblocks > 512 ? 8 : 16;
+}
+
+// The gradient kernel (two workgroups, one per network, per partial row) and the
+// reduction.
 int mlp_launch(const void* kern, MlpArgs& a, const MlpLayout& l, hipStream_t stream) {
   void* args[] = {&a};
   int st = hip_status(hipLaunchKernel(kern, dim3((unsigned)(2 * l.nblocks)), dim3(l.threads),
                                       args, 0, stream));
   if (st) return st;
-  const bool wide = l.nblocks >= kRedWideRows;
-  return hip_status(hipLaunchKernel(wide ? (const void*)mlp_grad_reduce_kernel<16, 16>
-                                         : (const void*)mlp_grad_reduce_kernel<4, 8>,
-                                    dim3((unsigned)l.rblocks), dim3(wide ? 1024 : 256), args, 0,
-                                    stream));
+  const int waves = reduce_waves(l);
+  const void* reduce = waves == 16  ? (const void*)mlp_grad_reduce_kernel<16, 16>
+                       : waves == 8 ? (const void*)mlp_grad_reduce_kernel<8, 16>
+                                    : (const void*)mlp_grad_reduce_kernel<4, 8>;
+  return hip_status(hipLaunchKernel(reduce, dim3((unsigned)l.rblocks), dim3(waves * kWave), args,
+                                    0, stream));
 }
 
 }  // namespace
@@ -1214,12 +1448,12 @@ extern "C" int ppo_mlp_cat_step_f32(const ppo_mlp3_f32* actor, const ppo_mlp3_f3
   hipStream_t stream = reinterpret_cast<hipStream_t>(stream_ptr);
   // one launch for the reduction and the update when its grid is resident
   // (PPO_AMD_MLP_FUSED_ADAM=0 in the environment keeps two launches)
-  const bool wide = l.nblocks >= kRedWideRows;
-  const void* fused = wide ? (const void*)mlp_reduce_adam_kernel<16, 16>
-                           : (const void*)mlp_reduce_adam_kernel<4, 8>;
-  const int fused_threads = wide ? 1024 : 256;
+  const int waves = reduce_waves(l);
+  const void* fused = waves == 16 ? (const void*)mlp_reduce_adam_kernel<16, 16>
+                                  : (const void*)mlp_reduce_adam_kernel<4, 8>;
+  const int fused_threads = waves * kWave;
   const char* env = getenv("PPO_AMD_MLP_FUSED_ADAM");
-  if (!(env && env[0] == '0') && l.rblocks <= 0x7fffffffL &&
+  if (!(env && env[0] == '0') && waves != 8 && l.rblocks <= 0x7fffffffL &&
       resident_blocks(fused, fused_threads, 0, 0) >= l.rblocks) {
     MlpAdamArgs u = {};
     for (int j = 0; j < kMlpTensors; ++j) {
