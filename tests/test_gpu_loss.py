@@ -601,6 +601,59 @@ def test_cat_past_2_31_elements(dev):
     torch.testing.assert_close(scalars.double().cpu(), weighted, rtol=2e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("B", [1, 3, 70_001])
+def test_backward_scales_saved_gradients(dev, B):
+    """The losses' backward: the fused kernel's gradients times the incoming
+    one, bit for bit, whichever way autograd may still need the saved ones."""
+    logits, actions, old_lp, adv, ret, val, _ = (x.to(dev) for x in cat_inputs(B, 5, seed=B))
+    _, dl, dv = ppo_amd.ppo_loss_discrete_fused(logits, actions, old_lp, adv, ret, val)
+
+    def leaves():
+        x, v = logits.clone().requires_grad_(), val.clone().requires_grad_()
+        return x, v, ppo_amd.ppo_loss_discrete(x, actions, old_lp, adv, ret, v)[0]
+
+    def check(x, v, scale):
+        assert torch.equal(x.grad, dl * scale) and torch.equal(v.grad, dv * scale)
+
+    for scale in (1.0, 0.25, -3.0):
+        x, v, loss = leaves()
+        (loss if scale == 1.0 else loss * scale).backward()
+        check(x, v, scale)
+        # a graph kept for a second pass, and accumulation into .grad
+        x, v, loss = leaves()
+        (loss * scale).backward(retain_graph=True)
+        check(x, v, scale)
+        x.grad = v.grad = None
+        loss.backward(retain_graph=True)
+        check(x, v, 1.0)
+        loss.backward()
+        check(x, v, 2.0)
+        with pytest.raises(RuntimeError, match="second time"):
+            loss.backward()
+    # saved gradients that someone else holds stay as they were
+    x, v, loss = leaves()
+    held = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: held.append(t) or t, lambda t: t):
+        x2, v2, loss2 = leaves()
+    kept = [t.clone() for t in held]
+    (loss2 * 4.0).backward()
+    check(x2, v2, 4.0)
+    assert held and all(torch.equal(a, b) for a, b in zip(held, kept))
+    with torch.autograd.graph.save_on_cpu():
+        x3, v3, loss3 = leaves()
+    (loss3 * 4.0).backward()
+    check(x3, v3, 4.0)
+    # in-place on the loss, and a gradient of the gradient by the incoming one
+    loss /= 4.0
+    loss.backward()
+    check(x, v, 0.25)
+    x, v, loss = leaves()
+    g = torch.tensor(2.0, device=dev, requires_grad=True)
+    (gx,) = torch.autograd.grad(loss, x, grad_outputs=g, create_graph=True)
+    (gg,) = torch.autograd.grad(gx.sum(), g)
+    torch.testing.assert_close(gg, dl.sum())
+
+
 def test_empty_batches_raise_like_the_reference(dev):
     """A minibatch of no rows: the reference's Categorical / Normal on an
     empty batch raises (torch cannot validate a [0, A] tensor, and the means

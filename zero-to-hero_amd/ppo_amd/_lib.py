@@ -177,6 +177,25 @@ def load() -> ctypes.CDLL:
     return _lib
 
 
+_native = None
+
+
+def native():
+    """The extension module ppo_amd._native (host path in C++); raise if absent."""
+    global _native
+    if _native is None:
+        load()
+        try:
+            from . import _native as mod
+        except ImportError as e:
+            raise RuntimeError(
+                "ppo_amd._native is not built. Build it with `python -m ppo_amd.build` "
+                "(or __graft_entry__.build())."
+            ) from e
+        _native = mod
+    return _native
+
+
 class PPOLibraryError(RuntimeError):
     """A non-zero return code from libppo_amd."""
 

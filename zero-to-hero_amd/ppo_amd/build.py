@@ -1,4 +1,5 @@
-"""Build libppo_amd.so for gfx950 in-tree (python -m ppo_amd.build)."""
+"""Build libppo_amd.so (gfx950) and the extension _native.so in-tree (python -m
+ppo_amd.build)."""
 
 from __future__ import annotations
 

@@ -19,6 +19,7 @@ Reference functions replaced (mrhooray/zero-to-hero, rl/deep/agents/ppo.py):
 from __future__ import annotations
 
 import ctypes
+import sys
 from typing import Optional
 
 import torch
@@ -687,22 +688,62 @@ def ppo_loss_discrete_fused(
     return scalars, dlogits, dvalues
 
 
+def _save_grads(ctx, scalars: torch.Tensor, *grads: torch.Tensor):
+    """Forward's end: saves the gradients the fused kernel wrote and returns
+    (loss, scalars).  The loss is a 0-d tensor on the first scalar's storage
+    rather than an indexed view, whose backward would build and fill a [6]
+    gradient; the scalars are reported values."""
+    ctx.save_for_backward(*grads)
+    # (saved-tensor hooks hand backward tensors that may be someone else's)
+    ctx.hooked = torch._C._autograd._top_saved_tensors_default_hooks(False) is not None
+    ctx.set_materialize_grads(False)
+    ctx.mark_non_differentiable(scalars)
+    loss = torch.empty(0, dtype=scalars.dtype, device=scalars.device)
+    loss.set_(scalars.untyped_storage(), scalars.storage_offset(), ())
+    return loss, scalars
+
+
+# References to a saved gradient inside _scaled_grads when nothing else holds
+# it: the saved variable, the tuple and the list, the loop variable, getrefcount's
+# argument.
+_SOLE_REFS = 5
+
+
+def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
+    """Backward: every saved gradient times the loss's incoming gradient.
+
+    Where the graph is released after this pass (no retain_graph, no
+    create_graph) and nothing else can see the saved gradients -- no
+    saved-tensor hooks, no other reference to them -- they are scaled in place
+    and returned themselves; the launch then touches nothing if the incoming
+    gradient is 1, as it is for loss.backward().  Otherwise they are scaled into
+    new tensors, and under create_graph by torch's own operators, which keep
+    the dependence on the incoming gradient."""
+    saved = ctx.saved_tensors
+    if grad_loss is None:
+        return (None,) * len(saved)
+    if torch.is_grad_enabled():
+        return tuple(t * grad_loss for t in saved)
+    grads = list(saved)
+    own = (not ctx.hooked and not torch._C._autograd._get_current_graph_task_keep_graph()
+           and all(sys.getrefcount(t) == _SOLE_REFS for t in grads))
+    outs = grads if own else [torch.empty_like(t) for t in grads]
+    _lib.check("scale_grads", _lib.native().scale_grads(grads, outs, grad_loss))
+    return tuple(outs)
+
+
 class _DiscreteLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, logits, values, actions, old_log_probs, advantages, returns,
                 old_values, clip_ratio, vf_clip, value_coef, entropy_coef, validate_args):
-        scalars, dlogits, dvalues = ppo_loss_discrete_fused(
+        return _save_grads(ctx, *ppo_loss_discrete_fused(
             logits.detach(), actions, old_log_probs, advantages, returns, values.detach(),
             old_values, clip_ratio, vf_clip, value_coef, entropy_coef, validate_args,
-        )
-        ctx.save_for_backward(dlogits, dvalues)
-        return scalars
+        ))
 
     @staticmethod
-    def backward(ctx, grad_scalars):
-        dlogits, dvalues = ctx.saved_tensors
-        g = grad_scalars[0]
-        return (dlogits * g, dvalues * g) + (None,) * 10
+    def backward(ctx, grad_loss, _):
+        return _scaled_grads(ctx, grad_loss) + (None,) * 10
 
 
 def ppo_loss_discrete(
@@ -726,11 +767,11 @@ def ppo_loss_discrete(
     incoming gradient); `stats` holds the component scalars, which are
     reported values, not differentiable outputs.
     """
-    scalars = _DiscreteLoss.apply(
+    loss, scalars = _DiscreteLoss.apply(
         logits, values, actions, old_log_probs, advantages, returns, old_values,
         clip_ratio, vf_clip, value_coef, entropy_coef, validate_args,
     )
-    return scalars[0], _stats_dict(scalars)
+    return loss, _stats_dict(scalars)
 
 
 def ppo_loss_gaussian_fused(
@@ -792,18 +833,14 @@ class _GaussianLoss(torch.autograd.Function):
     @staticmethod
     def forward(ctx, mu, log_std, values, actions, old_log_probs, advantages, returns,
                 old_values, clip_ratio, vf_clip, value_coef, entropy_coef):
-        scalars, dmu, dlog_std, dvalues = ppo_loss_gaussian_fused(
+        return _save_grads(ctx, *ppo_loss_gaussian_fused(
             mu.detach(), log_std.detach(), actions, old_log_probs, advantages, returns,
             values.detach(), old_values, clip_ratio, vf_clip, value_coef, entropy_coef,
-        )
-        ctx.save_for_backward(dmu, dlog_std, dvalues)
-        return scalars
+        ))
 
     @staticmethod
-    def backward(ctx, grad_scalars):
-        dmu, dlog_std, dvalues = ctx.saved_tensors
-        g = grad_scalars[0]
-        return (dmu * g, dlog_std * g, dvalues * g) + (None,) * 9
+    def backward(ctx, grad_loss, _):
+        return _scaled_grads(ctx, grad_loss) + (None,) * 9
 
 
 def ppo_loss_gaussian(
@@ -822,11 +859,11 @@ def ppo_loss_gaussian(
 ) -> tuple[torch.Tensor, LossStats]:
     """Differentiable PPO loss of a Normal(mu, exp(log_std)) policy; gradients
     reach mu, log_std and values.  See ppo_loss_discrete for the contract."""
-    scalars = _GaussianLoss.apply(
+    loss, scalars = _GaussianLoss.apply(
         mu, log_std, values, actions, old_log_probs, advantages, returns, old_values,
         clip_ratio, vf_clip, value_coef, entropy_coef,
     )
-    return scalars[0], _stats_dict(scalars)
+    return loss, _stats_dict(scalars)
 
 
 # ---------------------------------------------------------------------------
