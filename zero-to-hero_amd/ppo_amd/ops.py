@@ -124,6 +124,27 @@ def _call(name: str, device: torch.device, stream: int, *args) -> None:
         _lib.check(name, code)
 
 
+def _native_failed(name: str, code: int, device: torch.device, stream: int) -> None:
+    """A library call of the native host path returned `code`."""
+    _WORKSPACES.drop(device, stream)
+    _lib.check(name, code)
+
+
+_NATIVE = None
+
+
+def _native():
+    """The native host path (csrc/native.cpp).  Its functions return None for
+    any call but the ordinary one, which then takes the checks here."""
+    global _NATIVE
+    if _NATIVE is None:
+        mod = _lib.native()
+        mod.init(_WORKSPACES, LossStats, _native_failed, list(_lib.SCALAR_NAMES),
+                 torch.nn.Sequential, torch.nn.Linear, torch.nn.ReLU, torch.nn.Tanh)
+        _NATIVE = mod
+    return _NATIVE
+
+
 def check_waits(device: Optional[torch.device] = None) -> None:
     """Synchronises torch's current stream on `device` (default: the current
     device) and raises PPOLibraryError with code PPO_ERR_WAIT_TIMEOUT if a
@@ -292,6 +313,10 @@ def gae(
     rewards, with returns = advantages + values (ppo.py:124); written into
     `out` = (advantages, returns) when given.
     """
+    if out is None:
+        got = _native().gae(rewards, values, dones, last_value, gamma, lam)
+        if got is not None:
+            return got
     device, T, N = _gae_inputs(rewards, values, dones, last_value)
     adv, ret = _outputs(out, 2, rewards, (rewards, values, dones, last_value))
     if T * N == 0:
@@ -331,6 +356,10 @@ def gae_normalize(
     ones would be (the resident pass then skips one store per element), the
     returned tuple holds that tensor first and third, and `out` is
     (normalized_advantages, returns)."""
+    if out is None and keep_raw:
+        got = _native().gae_normalize(rewards, values, dones, last_value, gamma, lam, eps)
+        if got is not None:
+            return got if return_stats else got[:3]
     device, T, N = _gae_inputs(rewards, values, dones, last_value)
     inputs = (rewards, values, dones, last_value)
     if keep_raw:
@@ -652,6 +681,12 @@ def ppo_loss_discrete_fused(
     torch.distributions.Categorical's support check does (this syncs);
     without it, such a row's log-prob is NaN.
     """
+    if not validate_args:
+        got = _native().loss_discrete_fused(
+            logits, actions, old_log_probs, advantages, returns, values, old_values, clip_ratio,
+            vf_clip, value_coef, entropy_coef)
+        if got is not None:
+            return got
     _require(logits, "logits", (torch.float32,))
     device = logits.device
     if logits.dim() != 2:
@@ -767,6 +802,12 @@ def ppo_loss_discrete(
     incoming gradient); `stats` holds the component scalars, which are
     reported values, not differentiable outputs.
     """
+    if not validate_args:
+        got = _native().loss_discrete(
+            logits, actions, old_log_probs, advantages, returns, values, old_values, clip_ratio,
+            vf_clip, value_coef, entropy_coef)
+        if got is not None:
+            return got
     loss, scalars = _DiscreteLoss.apply(
         logits, values, actions, old_log_probs, advantages, returns, old_values,
         clip_ratio, vf_clip, value_coef, entropy_coef, validate_args,
@@ -794,6 +835,11 @@ def ppo_loss_gaussian_fused(
     and entropy summed over D.  Returns (scalars[6], dmu[B,D], dlog_std[D],
     dvalues[B]).
     """
+    got = _native().loss_gaussian_fused(
+        mu, log_std, actions, old_log_probs, advantages, returns, values, old_values, clip_ratio,
+        vf_clip, value_coef, entropy_coef)
+    if got is not None:
+        return got
     _require(mu, "mu", (torch.float32,))
     device = mu.device
     if mu.dim() != 2:
@@ -859,6 +905,11 @@ def ppo_loss_gaussian(
 ) -> tuple[torch.Tensor, LossStats]:
     """Differentiable PPO loss of a Normal(mu, exp(log_std)) policy; gradients
     reach mu, log_std and values.  See ppo_loss_discrete for the contract."""
+    got = _native().loss_gaussian(
+        mu, log_std, actions, old_log_probs, advantages, returns, values, old_values, clip_ratio,
+        vf_clip, value_coef, entropy_coef)
+    if got is not None:
+        return got
     loss, scalars = _GaussianLoss.apply(
         mu, log_std, values, actions, old_log_probs, advantages, returns, old_values,
         clip_ratio, vf_clip, value_coef, entropy_coef,
@@ -1010,6 +1061,11 @@ def ppo_mlp_cat_grads(
     `.grad` is overwritten with d loss / d parameter (allocated if None).
     Returns the loss scalars (0-d device tensors).  Both networks must satisfy
     mlp_fusable(); follow with ClippedAdam.step()."""
+    got = _native().mlp_grads(
+        policy, value, observations, actions, old_log_probs, advantages, returns, old_values,
+        index, clip_ratio, vf_clip, value_coef, entropy_coef, scalars_out)
+    if got is not None:
+        return got
     device, stream, ws, scalars, head, keep = _mlp_minibatch_args(
         policy, value, observations, actions, old_log_probs, advantages, returns, old_values,
         index, clip_ratio, vf_clip, value_coef, entropy_coef, scalars_out)
@@ -1081,6 +1137,10 @@ def mlp_act_categorical(
     log_probs [N], values [N]); the *_out tensors are written in place when
     given, and observations_out (e.g. a rollout buffer row) receives a copy
     of the observations."""
+    got = _native().mlp_act(policy, value, observations, uniforms, generator, observations_out,
+                            actions_out, log_probs_out, values_out)
+    if got is not None:
+        return got
     if not mlp_fusable(policy, value):
         raise ValueError("policy/value are not MLPs the fused kernel supports (see mlp_fusable)")
     lp, act = mlp_structure(policy)
