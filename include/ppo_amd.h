@@ -178,6 +178,7 @@ int ppo_gae_norm_f32(const float* rewards, const float* values,
 #define PPO_GAE_ROUTE_STRIP 2     /* strip walk (+ normalise pass)             */
 #define PPO_GAE_ROUTE_SPAN 3      /* span passes + carry scan (+ normalise)    */
 #define PPO_GAE_ROUTE_TILES 4     /* tile passes + carry scan                  */
+#define PPO_GAE_ROUTE_COLUMN 5    /* one launch, a workgroup per few envs      */
 int ppo_gae_route(int64_t T, int64_t N, int normalize, int has_values);
 
 /* ------------------------------------------------------------------------ */

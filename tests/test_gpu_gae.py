@@ -514,6 +514,64 @@ def _resident_case(dev, T, N, p, norm, seed, last=True, fill=0xAB):
     return exact, adv, adv_n
 
 
+# The column pass: one and several workgroups, 4, 8 and 16 envs per workgroup, 2
+# to 16 steps per thread, a last column and a last segment in part, single
+# elements, and one element past each bound (which takes another pass)
+COLUMN_SHAPES = [
+    (1, 1), (1, 5), (3, 4), (127, 8), (128, 17), (256, 16), (257, 33), (512, 16), (513, 16),
+    (1000, 8), (1024, 9), (1000, 255), (1000, 257), (1025, 64), (2048, 3), (2047, 65), (2048, 2047),
+    (2049, 7), (255, 4096), (60, 4097), (200, 8192), (16, 8192), (500, 4100),
+]
+
+
+@pytest.mark.parametrize("p", [0.0, 0.02])
+@pytest.mark.parametrize("T,N", COLUMN_SHAPES)
+def test_gae_column_pass(dev, T, N, p):
+    """Against the oracle with and without the normaliser, in place, with a
+    buffer of random bytes as workspace, on misaligned arrays, without values,
+    and with infinities late in the horizon."""
+    r, v, d, lv = (x.to(dev) for x in _inputs(T, N, p, T + N, True))
+    print(f"gae column T={T} N={N} p={p} routes {_route(T, N, True)} {_route(T, N, False)}",
+          flush=True)
+    a_ref, _ = ref.gae_c(r.cpu().numpy(), v.cpu().numpy(), d.cpu().numpy(), lv.cpu().numpy(),
+                         0.99, 0.95)
+    for norm in (False, True):
+        adv, ret, adv_n = _gae_abi(dev, r, v, d, lv, 0.99, 0.95, norm=norm, fill=0xAB)
+        assert_gae_close(adv.cpu().numpy(), a_ref)
+        assert torch.equal(ret, adv + v)
+        if norm and T * N > 1:
+            n_ref = ref.normalize_reference(torch.from_numpy(a_ref).reshape(-1)).reshape(T, N)
+            torch.testing.assert_close(adv_n.cpu(), n_ref, rtol=1e-5, atol=1e-6)
+        elif norm:
+            assert torch.equal(adv_n, adv)
+
+    def shifted(x):
+        buf = torch.empty(x.numel() + 1, dtype=x.dtype, device=dev)
+        buf[1:] = x.reshape(-1)
+        return buf[1:].view(x.shape)
+
+    args = [shifted(x) for x in (r, v, d, lv)]
+    got = ppo_amd.gae_normalize(*args, 0.99, 0.95)
+    assert_gae_close(got[0].cpu().numpy(), a_ref)
+    in_place, ret_ip, _ = ppo_amd.gae_normalize(*args, 0.99, 0.95, keep_raw=False)
+    torch.testing.assert_close(in_place, got[2], rtol=1e-5, atol=1e-6)
+    assert torch.equal(ret_ip, got[1])
+    disc = ppo_amd.discounted_returns(r, dones=d, gamma=0.99).cpu().numpy()
+    d_ref, _ = ref.gae_c(r.cpu().numpy(), np.zeros((T, N), np.float32), d.cpu().numpy(), None,
+                         0.99, 1.0)
+    assert_gae_close(disc, d_ref)
+    r[T // 2, 0] = float("inf")
+    v[T // 3, N // 2] = float("nan")
+    lv[N - 1] = float("-inf")
+    a_ref, _ = ref.gae_c(r.cpu().numpy(), v.cpu().numpy(), d.cpu().numpy(), lv.cpu().numpy(),
+                         0.99, 0.95)
+    got = _gae_abi(dev, r, v, d, lv, 0.99, 0.95)[0].cpu().numpy()
+    for f in (np.isnan, np.isposinf, np.isneginf):
+        np.testing.assert_array_equal(f(got), f(a_ref))
+    fin = np.isfinite(a_ref)
+    assert_gae_close(got[fin], a_ref[fin])
+
+
 @pytest.mark.parametrize("norm", [True, False])
 @pytest.mark.parametrize("T,N,p", RESIDENT_SHAPES)
 def test_gae_resident_matches_oracle(dev, T, N, p, norm):

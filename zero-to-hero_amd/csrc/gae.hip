@@ -269,6 +269,7 @@ SpanPlan span_plan(long T, long N, long blocks) {
 #endif
 constexpr int kResBlock = PPO_GAE_RES_BLOCK;
 constexpr long kResMaxTiles = 256;  // one workgroup per CU on MI355X
+constexpr int kColBlock = 1024;      // threads of the column pass
 
 struct ResPlan {
   int E, L;          // E = 0: not applicable
@@ -286,18 +287,22 @@ struct ResPlan {
 // measured 38.2-38.5 us per call in the north-star step against 39.1-39.3 us
 // for 64-env tiles; 256-env tiles were slower, their look-back folding 15
 // tiles per column, so 128-env tiles are taken only up to 8 tiles per column).  Rollouts that
-// give fewer than 128 tiles (too little parallelism), or more than 16 tiles
-// per env column without filling the device, take the other paths: measured
-// on MI355X, e.g. T x N = 1024 x 512 (16-64 tiles) 28 us against 24 us on the
-// tile passes, while 2048 x 4096 runs 45 us against 55 us, 4096 x 2048 45 us
-// against 72 and 32768 x 256 (64 tiles per column, 256 tiles) 57 us against 67.
+// give fewer than `min_tiles` tiles, or more than 16 tiles per env column
+// without filling the device, take the other paths: measured on MI355X, 2048 x
+// 4096 runs 45 us against 55 us, 4096 x 2048 45 us against 72 and 32768 x 256 (64
+// tiles per column, 256 tiles) 57 us against 67.  From 128 tiles on the resident
+// pass comes first; with fewer (kResFewTiles) it follows the column pass, where
+// that declines or is slower (gae_route): 2048 x 256 with the normaliser
+// 13.3 us against 15.4 of columns and 19.4 of the span passes, 8192 x 16 13.2
+// against 18.4.
 // Without the normaliser, rollouts too long for one round (more than 256
 // tiles of 16 steps per thread) run in rounds of 256 tiles, from the end of
 // the horizon backwards (at most kResMaxRounds), each round handing the
 // advantage at its left edge to the next.
 constexpr long kResMaxRounds = 8;
+constexpr long kResManyTiles = 128, kResFewTiles = 2;
 
-ResPlan res_plan(long T, long N, bool norm) {
+ResPlan res_plan(long T, long N, bool norm, long min_tiles) {
   ResPlan best = {0, 0, 0, 0, 0, 0, 0};
   if (!PPO_GAE_RES || T <= 0 || N <= 0 || T * N >= (1L << 30)) return best;
   const int Es[4] = {128, 64, 32, 16};
@@ -324,7 +329,7 @@ ResPlan res_plan(long T, long N, bool norm) {
       }
     }
   }
-  if (best.E && (best.tiles() < 128 || (best.nt > 16 && best.tiles() < kResMaxTiles)))
+  if (best.E && (best.tiles() < min_tiles || (best.nt > 16 && best.tiles() < kResMaxTiles)))
     best.E = 0;
   if (best.E || norm) return best;
   // rounds: the widest tile of at most 64 envs dividing N, 16 steps per thread
@@ -352,6 +357,48 @@ ResPlan res_plan(long T, long N, bool norm) {
   return best;
 }
 
+// Column pass (gae_column_kernel): E envs per 1024-thread workgroup, L steps per
+// thread, the whole horizon in one workgroup.
+struct ColPlan {
+  int E, L;  // E = 0: not applicable
+  long wgs;
+};
+
+// A workgroup touches every row of the horizon once per array whatever E is (16,
+// 32 or 64 bytes of it), so its time grows with T: taken to T = 2048 (2048 x 64
+// with the normaliser 13 us, 4096 x 64 28 us against 19 of the span passes).
+// Narrow columns give more workgroups, wide ones longer row pieces: 16 envs to
+// 256 steps, then 4, or 8 where 4 would give more than 64 workgroups (1000 x 64
+// 10.2 against 11.6 us, 1000 x 1023 17.2 against 16.5; 2048 x 2047 without the
+// normaliser 31 against 21).  A rollout that one workgroup holds needs no exchange
+// (512 x 16 with the normaliser 7.9 us with 16 envs, 9.6 with 8).  The exchange
+// needs the grid resident at once (256 workgroups).  Where the tile or strip
+// passes have enough rows in flight they win: past 512 columns (512 x 20001 without
+// the normaliser 124 us against 76), with most threads idle (16 x 30000 13 against
+// 7), and past 1024 steps of more than 64 envs (2000 x 129 20.0 against 18.1, 1500 x
+// 257 19.7 against 18.4, 2048 x 1300 without the normaliser 28 against 25) unless
+// the normaliser's extra passes (2048 x 700 22 against 60) or an N that no vector
+// width divides (2048 x 2047 21 against 36) cost them more.
+ColPlan col_plan(long T, long N, bool norm) {
+  const ColPlan none = {0, 0, 0};
+  if (T <= 0 || N <= 0 || T > 2048 || T * N >= (1L << 30)) return none;
+  auto steps = [&](int E) { return (T * E + kColBlock - 1) / kColBlock; };
+  int E = T <= 256 ? 16 : (N > 256 ? 8 : 4);
+  if (norm) {
+    for (int e : {16, 8, 4})
+      if (N <= e && steps(e) <= 8) E = e;
+    while ((N + E - 1) / E > kResMaxTiles) {
+      if (E == 16 || steps(2 * E) > 16) return none;
+      E *= 2;
+    }
+  }
+  const long wgs = (N + E - 1) / E, per = steps(E);
+  if (wgs > 2 * kResMaxTiles || (wgs > kResMaxTiles && T * E < kColBlock)) return none;
+  if (T > 1024 && N > 64 && (norm ? N < (N % 4 ? 768 : 384) : N <= 1024 || N % 4 == 0))
+    return none;
+  return {E, per <= 2 ? 2 : (per <= 4 ? 4 : (per <= 8 ? 8 : 16)), wgs};
+}
+
 // 64-bit slot words of the resident pass: the start barrier's counter (a
 // block of 32 words), per tile E composites (a, P) of two words each, per
 // round one carry per env (the advantage at the round's left edge), then
@@ -366,7 +413,10 @@ size_t res_slot_words(const ResPlan& rp) {
          (size_t)rp.grid() * kResPartWords;
 }
 size_t res_slot_words_max(long T, long N) {
-  return std::max(res_slot_words(res_plan(T, N, true)), res_slot_words(res_plan(T, N, false)));
+  const ColPlan cp = col_plan(T, N, true);
+  return std::max({res_slot_words(res_plan(T, N, true, kResFewTiles)),
+                   res_slot_words(res_plan(T, N, false, kResFewTiles)),
+                   cp.wgs > 1 ? kResSlotBase + (size_t)cp.wgs * kResPartWords : 0});
 }
 
 struct GaeLayout {
@@ -2150,20 +2200,18 @@ const void* res_kernel(const ResPlan& rp, bool stats, bool has_v) {
 // The environment variable PPO_AMD_GAE_RESIDENT=0 turns the resident pass
 // off (every rollout then takes the strip walk, span or tile passes), so that
 // those paths can be tested on shapes the resident pass would take.
-bool resident_ok(long T, long N, bool norm, bool has_v) {
+bool resident_ok(long T, long N, bool norm, bool has_v, long min_tiles) {
   const char* env = getenv("PPO_AMD_GAE_RESIDENT");
   if (env && env[0] == '0') return false;
-  const ResPlan rp = res_plan(T, N, norm);
+  const ResPlan rp = res_plan(T, N, norm, min_tiles);
   if (rp.E == 0) return false;
   const void* kern = res_kernel(rp, norm, has_v);
   return kern && resident_blocks(kern, kResBlock, 0, 0) >= rp.grid();
 }
 
-// Launches the resident pass when the plan applies and the whole grid fits
-// on the device at once; returns -1 (nothing launched) otherwise.
+// Launches the resident pass (resident_ok).
 int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
-  if (!resident_ok(T, N, norm, a.v != nullptr)) return -1;
-  const ResPlan rp = res_plan(T, N, norm);
+  const ResPlan rp = res_plan(T, N, norm, kResFewTiles);
   const void* kern = res_kernel(rp, norm, a.v != nullptr);
   a.res_nc = rp.nc;
   a.res_nt = rp.nt;
@@ -2175,6 +2223,238 @@ int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
   void* args[] = {&a};
   return hip_status(
       hipLaunchKernel(kern, dim3((unsigned)rp.grid()), dim3(kResBlock), args, 0, stream));
+}
+
+// ---------------------------------------------------------------------------
+// Column pass: one launch for rollouts whose horizon fits one workgroup.  A
+// 1024-thread workgroup owns E envs for the whole horizon (1024 / E segments of L
+// steps, one env per thread, rows in registers from load to store, any N and
+// any alignment), so no carry crosses workgroups; with the normaliser the
+// workgroups exchange only their fp64 (n, sum, sum of squares) through the
+// slots of grid_sync.hpp (a single workgroup exchanges nothing) and write the
+// normalised advantages from the registers.
+//
+// What bounds it: latency -- one round of loads, the scan, the exchange, the
+// stores.  Measured on MI355X against the 3 or 4 launches of the span and tile
+// passes (T x N, us of device time per call, with / without the normaliser):
+//   128 x 8      15.0 -> 5.3 / 5.9 -> 3.6      1000 x 64    18.2 -> 10.3 / 11.6 -> 5.6
+//   1000 x 1023  21.4 -> 16.4 / 16.2 -> 10.8   2048 x 64    18.4 -> 13.1 / 11.4 -> 8.0
+//   200 x 2048   19.2 -> 10.3 / 14.4 -> 4.9    2048 x 2047  45.5 -> 30.2 / 36.0 -> 21.4
+// ---------------------------------------------------------------------------
+constexpr int kColWaves = kColBlock / kWave;
+
+template <int E, int L, bool kStats, bool kHasV>
+__global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
+  constexpr int SW = kWave / E;  // segments per wave
+  __shared__ double2 s_wc[kColWaves][E];
+  __shared__ float s_norm[2];
+  __shared__ unsigned s_tag;
+  __shared__ uint64_t s_epoch;
+  const int tid = threadIdx.x;
+  const int lane = tid % kWave, w = tid / kWave, j = lane / E, e = tid % E;
+  // neighbouring columns, which share cache lines, on one XCD
+  const long nwg = gridDim.x;
+  const long col = nwg % kXcds == 0 ? (long)blockIdx.x % kXcds * (nwg / kXcds) + blockIdx.x / kXcds
+                                    : (long)blockIdx.x;
+  const bool multi = kStats && nwg > 1;
+  uint64_t* part = a.slots + kResSlotBase;  // [grid][kResPartWords]
+  int fail = 0;
+  if (multi && w == 0) {
+    uint64_t epoch;
+    const unsigned tag = launch_tag(&a.hdr->epoch, a.nonce, epoch);
+    if (tid == 0) {
+      s_tag = tag;
+      s_epoch = epoch;
+    }
+    sync_start(a.slots, part + (size_t)blockIdx.x * kResPartWords, (int)kResPartWords, tag);
+  }
+  const long env = col * E + e;
+  const long T = a.T;
+  const unsigned n32 = (unsigned)a.N, env32 = (unsigned)(env < a.N ? env : a.N - 1);
+  const long t0 = (long)(tid / E) * L;
+  const int nvalid = env >= a.N || t0 >= T ? 0 : (T - t0 < L ? (int)(T - t0) : L);
+  // (rows past the horizon re-read the last one)
+  auto row = [&](long t) { return (unsigned)(t < T ? t : T - 1) * n32 + env32; };
+  float r[L], v[L];
+  unsigned d[L];
+  const bool inner = t0 + L < T;
+  const float* nsrc = inner ? (kHasV ? a.v + row(t0 + L) : a.r + env32)
+                            : (a.lastv ? a.lastv + env32 : a.r + env32);
+  float nv = *nsrc;
+  if (!(inner ? kHasV : a.lastv != nullptr)) nv = 0.0f;
+#pragma unroll
+  for (int i = L - 1; i >= 0; --i) {
+    const unsigned off = row(t0 + i);
+    r[i] = a.r[off];
+    v[i] = kHasV ? a.v[off] : 0.0f;
+    d[i] = a.d[off];
+  }
+  const double gl0 = mul(a.gl, 0.0);
+
+  // segment composites (a, P), then the reverse scan over the workgroup (the
+  // composites only carry the advantage between segments: fused multiply-adds)
+  double ia = 0.0, ip = 1.0;
+  {
+    double nvd = nv;
+#pragma unroll
+    for (int i = L - 1; i >= 0; --i) {
+      if (i < nvalid) {
+        const bool done = d[i] != 0u;
+        const double vd = v[i];
+        const double dl = __builtin_fma(a.gamma * nvd, done ? 0.0 : 1.0, (double)r[i]) - vd;
+        const double cc = done ? gl0 : a.gl;
+        ia = __builtin_fma(cc, ia, dl);
+        ip = ip * cc;
+        nvd = vd;
+      }
+    }
+  }
+#pragma unroll
+  for (int off = 1; off < SW; off <<= 1) {
+    const double pa = __shfl_down(ia, E * off);
+    const double pp = __shfl_down(ip, E * off);
+    if (j + off < SW) {
+      ia = ia + ip * pa;
+      ip = prod_nz(ip, pp);
+    }
+  }
+  double na = __shfl_down(ia, E), np = __shfl_down(ip, E);
+  if (j + 1 >= SW) {
+    na = 0.0;
+    np = 1.0;
+  }
+  if (j == 0) s_wc[w][e] = make_double2(ia, ip);
+  lds_barrier();
+  double C = 0.0;
+  for (int ww = kColWaves - 1; ww > w; --ww) {
+    const double2 c = s_wc[ww][e];
+    C = c.x + c.y * C;
+  }
+
+  // exact recurrence from the segment's carry.  (The empty asm hides that the
+  // rows are unchanged: the compiler would keep their fp64 copies and deltas
+  // from above alive, and at 16 steps spill them.)
+#pragma unroll
+  for (int i = 0; i < L; ++i) asm volatile("" : "+v"(r[i]), "+v"(v[i]), "+v"(d[i]));
+  double acc[3] = {(double)nvalid, 0.0, 0.0};
+  {
+    double x = na + np * C, nvd = nv;
+#pragma unroll
+    for (int i = L - 1; i >= 0; --i) {
+      if (i < nvalid) {
+        const bool done = d[i] != 0u;
+        const double vd = v[i];
+        const double dl = sub(add((double)r[i], mul(mul(a.gamma, nvd), done ? 0.0 : 1.0)), vd);
+        x = add(dl, mul(done ? gl0 : a.gl, x));
+        nvd = vd;
+        r[i] = (float)x;  // the advantage replaces the reward
+        const unsigned off = row(t0 + i);
+        if (!kStats || a.adv != a.adv_n) a.adv[off] = r[i];
+        if (a.ret) a.ret[off] = r[i] + v[i];
+        if constexpr (kStats) {
+          const double xf = r[i];
+          acc[1] += xf;
+          acc[2] += xf * xf;
+        }
+      }
+    }
+  }
+  if constexpr (kStats) {
+    block_sum_lds<3>(acc);
+    if (multi) {
+      if (tid == 0) {
+        uint64_t* pp = part + (size_t)blockIdx.x * kResPartWords;
+        slot_put(pp + 0, acc[0]);
+        slot_put(pp + 1, acc[1]);
+        slot_put(pp + 2, acc[2]);
+        if (!res_wait(a.slots, s_tag, gridDim.x, a.wc.spin)) fail = 1;
+        if (blockIdx.x == 0) epoch_advance(&a.hdr->epoch, s_epoch);
+      }
+      lds_barrier();
+      // every workgroup reads all partials in one order: the same bits in each
+      acc[0] = acc[1] = acc[2] = 0.0;
+      for (long u = tid; u < nwg; u += kColBlock) {
+        uint64_t* pp = part + (size_t)u * kResPartWords;
+        acc[0] += slot_get(pp + 0, a.wc.spin, fail);
+        acc[1] += slot_get(pp + 1, a.wc.spin, fail);
+        acc[2] += slot_get(pp + 2, a.wc.spin, fail);
+      }
+      block_sum_lds<3>(acc);
+    }
+    if (tid == 0) {
+      const NormParams np_ = norm_params_of(acc, a.eps);
+      s_norm[0] = np_.mean_used;
+      s_norm[1] = np_.denom;
+      if (blockIdx.x == 0) {
+        a.hdr->stats[0] = np_.mean_used;
+        a.hdr->stats[1] = np_.std;
+        a.hdr->stats[2] = np_.denom;
+        if (a.stats_out) {
+          a.stats_out[0] = np_.mean;
+          a.stats_out[1] = np_.std;
+        }
+      }
+    }
+    lds_barrier();
+    const float mean = s_norm[0], denom = s_norm[1];
+#pragma unroll
+    for (int i = 0; i < L; ++i) {
+      asm volatile("" : "+v"(r[i]));  // (as above: the rows' fp64 copies)
+      if (i < nvalid) a.adv_n[row(t0 + i)] = (r[i] - mean) / denom;
+    }
+    // A wait that gave up (grid not co-resident): NaN over everything this
+    // workgroup wrote, and the device's wait-status word.
+    if (multi && __syncthreads_or(fail)) {
+      if (tid == 0) wait_report(a.wc.status);
+      const float qnan = __builtin_nanf("");
+      for (int i = 0; i < nvalid; ++i) {
+        a.adv[row(t0 + i)] = qnan;
+        if (a.ret) a.ret[row(t0 + i)] = qnan;
+        a.adv_n[row(t0 + i)] = qnan;
+      }
+    }
+  }
+}
+
+template <int E>
+const void* column_kernel_e(int L, bool stats, bool has_v) {
+#define PPO_COL(L_)                                                          \
+  (stats ? (has_v ? (const void*)gae_column_kernel<E, L_, true, true>         \
+                  : (const void*)gae_column_kernel<E, L_, true, false>)       \
+         : (has_v ? (const void*)gae_column_kernel<E, L_, false, true>        \
+                  : (const void*)gae_column_kernel<E, L_, false, false>))
+  return L == 16 ? PPO_COL(16) : (L == 8 ? PPO_COL(8) : (L == 4 ? PPO_COL(4) : PPO_COL(2)));
+#undef PPO_COL
+}
+
+const void* column_kernel(const ColPlan& cp, bool stats, bool has_v) {
+  if (cp.E == 16) return column_kernel_e<16>(cp.L, stats, has_v);
+  if (cp.E == 8) return column_kernel_e<8>(cp.L, stats, has_v);
+  return column_kernel_e<4>(cp.L, stats, has_v);
+}
+
+// Whether a column pass runs here: the normaliser's exchange needs the whole
+// grid resident at once (and no PPO_AMD_GAE_RESIDENT=0, which asks for passes
+// that wait for nothing).
+bool column_ok(long T, long N, bool norm, bool has_v) {
+  const ColPlan cp = col_plan(T, N, norm);
+  if (!cp.E) return false;
+  if (!norm || cp.wgs == 1) return true;
+  const char* env = getenv("PPO_AMD_GAE_RESIDENT");
+  if (env && env[0] == '0') return false;
+  return resident_blocks(column_kernel(cp, norm, has_v), kColBlock, 0, 0) >= cp.wgs;
+}
+
+int launch_column(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
+  const ColPlan cp = col_plan(T, N, norm);
+  if (norm && cp.wgs > 1) {
+    a.nonce = next_nonce();
+    const int st = wait_ctl(a.wc);
+    if (st) return st;
+  }
+  void* args[] = {&a};
+  return hip_status(hipLaunchKernel(column_kernel(cp, norm, a.v != nullptr),
+                                    dim3((unsigned)cp.wgs), dim3(kColBlock), args, 0, stream));
 }
 
 // Pass kernels by (VW, L, solo) geometry.
@@ -2285,6 +2565,23 @@ bool span_route(long T, long N, bool norm) {
          strip_plan(make_plan(T, N, 4)).E == 0 && (norm || (N < 64 && T * N >= (1L << 20)));
 }
 
+// The passes of a rollout: `vec` where N and the buffers allow 16-byte accesses
+// (all_vec: the normalised advantages too).
+int gae_route(long T, long N, bool norm, bool has_v, bool vec, bool all_vec) {
+  // aligned rollouts of many tiles that all fit on the device at once: one
+  // read of the rollout, one write of each output
+  if (all_vec && resident_ok(T, N, norm, has_v, kResManyTiles)) return PPO_GAE_ROUTE_RESIDENT;
+  const bool column = column_ok(T, N, norm, has_v);
+  // fewer tiles: long horizons, or many columns of a horizon past 1024
+  if (all_vec && (!column || (T > 1024 && N > 64)) &&
+      resident_ok(T, N, norm, has_v, kResFewTiles))
+    return PPO_GAE_ROUTE_RESIDENT;
+  if (column) return PPO_GAE_ROUTE_COLUMN;
+  if (vec && span_route(T, N, norm)) return PPO_GAE_ROUTE_SPAN;
+  const GaePlan p = make_plan(T, N, vec && !narrow_scalar(T, N, norm) ? 4 : 1);
+  return strip_plan(p).E > 0 ? PPO_GAE_ROUTE_STRIP : PPO_GAE_ROUTE_TILES;
+}
+
 int gae_impl(const float* rewards, const float* values, const uint8_t* dones,
              const float* last_value, int64_t T, int64_t N, double gamma, double lam, double eps,
              float* adv_out, float* ret_out, float* adv_norm_out, float* stats_out, bool norm,
@@ -2327,15 +2624,13 @@ int gae_impl(const float* rewards, const float* values, const uint8_t* dones,
   a.adv_n = adv_norm_out;
   a.slots = reinterpret_cast<uint64_t*>(ws + l.slots);
 
-  // Aligned rollouts whose tiles all fit on the device at once take the
-  // resident pass (one read of the rollout, one write of each output).
-  if (vec && (!norm || aligned(adv_norm_out, 16))) {
-    const int st = launch_resident(T, N, a, norm, stream);
-    if (st >= 0) return st;
+  switch (gae_route(T, N, norm, values != nullptr, vec,
+                    vec && (!norm || aligned(adv_norm_out, 16)))) {
+    case PPO_GAE_ROUTE_RESIDENT: return launch_resident(T, N, a, norm, stream);
+    case PPO_GAE_ROUTE_COLUMN: return launch_column(T, N, a, norm, stream);
+    case PPO_GAE_ROUTE_SPAN: return launch_span(T, N, a, norm, stream);
+    default: return launch_gae(p, a, norm, stream);
   }
-
-  if (vec && span_route(T, N, norm)) return launch_span(T, N, a, norm, stream);
-  return launch_gae(p, a, norm, stream);
 }
 
 }  // namespace
@@ -2347,10 +2642,7 @@ extern "C" int ppo_gae_route(int64_t T, int64_t N, int normalize, int has_values
   const bool norm = normalize != 0;
   if (N > (1L << 31) || T > (1L << 40) || T * N > (1L << 50)) return PPO_GAE_ROUTE_NONE;
   const bool vec = N % 4 == 0;
-  if (vec && resident_ok(T, N, norm, has_values != 0)) return PPO_GAE_ROUTE_RESIDENT;
-  if (vec && span_route(T, N, norm)) return PPO_GAE_ROUTE_SPAN;
-  const GaePlan p = make_plan(T, N, vec && !narrow_scalar(T, N, norm) ? 4 : 1);
-  return strip_plan(p).E > 0 ? PPO_GAE_ROUTE_STRIP : PPO_GAE_ROUTE_TILES;
+  return gae_route(T, N, norm, has_values != 0, vec, vec);
 }
 
 extern "C" size_t ppo_gae_workspace_bytes(int64_t T, int64_t N) {

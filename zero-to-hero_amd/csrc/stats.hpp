@@ -21,9 +21,8 @@ struct NormParams {
   float mean, std;         // what is reported
 };
 
-__device__ inline NormParams norm_params(const double* partials, long count, double eps) {
-  double tot[3];
-  sum_partials(partials, count, tot);
+// From the totals (n, sum x, sum x^2).
+__device__ inline NormParams norm_params_of(const double (&tot)[3], double eps) {
   const double n = tot[0];
   const double mean = tot[1] / n;
   NormParams r;
@@ -39,6 +38,12 @@ __device__ inline NormParams norm_params(const double* partials, long count, dou
     r.denom = 1.0f;
   }
   return r;
+}
+
+__device__ inline NormParams norm_params(const double* partials, long count, double eps) {
+  double tot[3];
+  sum_partials(partials, count, tot);
+  return norm_params_of(tot, eps);
 }
 
 // Enqueue the one-block kernel that turns `count` (n, sum, sum of squares)

@@ -55,7 +55,7 @@ class Mlp3(ctypes.Structure):
     ]
 
 
-GAE_ROUTES = {0: "none", 1: "resident", 2: "strip", 3: "span", 4: "tiles"}
+GAE_ROUTES = {0: "none", 1: "resident", 2: "strip", 3: "span", 4: "tiles", 5: "column"}
 
 PPO_ACT_RELU = 0
 PPO_ACT_TANH = 1
