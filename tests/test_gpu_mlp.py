@@ -262,6 +262,20 @@ def test_vecppo_fused_mlp_matches_unfused(dev, graphs):
         torch.testing.assert_close(s_f[k], s_u[k], rtol=1e-4, atol=1e-6)
 
 
+@pytest.mark.parametrize("H", [64, 128])
+def test_mlp_act_wide_and_narrow_forms_agree(dev, H):
+    """8193 rows take the narrow form, 8192 and fewer the wide one: the same
+    tiles in the same order, so the same bits."""
+    pol, val, _, gpu = _case(dev, 8193, 9, H, 6, "tanh", seed=H)
+    pol, val = pol.to(dev), val.to(dev)
+    u = torch.rand(8193, generator=torch.Generator().manual_seed(H)).to(dev)
+    full = ppo_amd.mlp_act_categorical(pol, val, gpu["obs"], uniforms=u)
+    for n in (1, 16, 17, 8192):
+        part = ppo_amd.mlp_act_categorical(pol, val, gpu["obs"][:n], uniforms=u[:n])
+        for a, b in zip(full, part):
+            assert torch.equal(a[:n], b)
+
+
 @pytest.mark.parametrize("H,A,act", [(64, 2, "tanh"), (128, 5, "relu"), (32, 18, "tanh")])
 def test_mlp_act_matches_torch_forward_and_sampler(dev, H, A, act):
     """ppo_mlp_act_cat_f32 (both forwards + the inverse-CDF draw in one

@@ -748,16 +748,17 @@ struct ActArgs {
   float* logits;
 };
 
-// Threads of the one-workgroup act launch (at most kMlpRows rows, where the
-// chain of dependent loads and barriers is the kernel's time): a wave per
-// 16-column tile of both networks' hidden layers (2 H / 16 tiles), so that no
-// wave works through several tiles one after another; at least kMlpBlock.
+// Threads of the wide act launch (at most kActWideRows rows, where the chain of
+// dependent loads and barriers is the kernel's time): a wave per 16-column tile
+// of both networks' hidden layers (2 H / 16 tiles), so that no wave works through
+// several tiles one after another; at least kMlpBlock.
+constexpr long kActWideRows = 8192;
 template <int H>
 constexpr int act_wide_block() {
   return 2 * (H / 16) * kWave > kMlpBlock ? 2 * (H / 16) * kWave : kMlpBlock;
 }
 
-// kBlock threads: kMlpBlock, or act_wide_block<H>() for one workgroup.
+// kBlock threads: kMlpBlock, or act_wide_block<H>().
 template <int H, int kAct, int kBlock = kMlpBlock>
 __global__ void __launch_bounds__(kBlock) mlp_act_cat_kernel(ActArgs a) {
   constexpr int R = kMlpRows;
@@ -1520,8 +1521,12 @@ int launch_act(const ppo_mlp3_f32* actor, const ppo_mlp3_f32* critic, int32_t ob
   if (a.N < 0) return PPO_ERR_INVALID_ARG;
   if (obs_dim <= 0 || obs_dim > kMlpMaxIn || A <= 0 || A > kMlpMaxA) return PPO_ERR_UNSUPPORTED;
   if (activation != PPO_ACT_RELU && activation != PPO_ACT_TANH) return PPO_ERR_INVALID_ARG;
-  // (one workgroup: the wide form, measured on MI355X at H = 128: 9.6 -> 8.4 us)
-  const bool wide = a.N <= kMlpRows;
+  // The wide form while its workgroups (8 or 16 waves) leave CUs to spare: the
+  // chain of layers bounds a launch then.  Measured on MI355X, us per call, 4 waves
+  // and wide: H = 64, 4096 rows 8.0 and 7.2 (D = 60, A = 18 13.7 and 11.2), 8192
+  // rows 9.7 and 9.0, 16,384 rows 12.7 and 12.4 (D = 60 21.4 and 22.0); H = 128, 4096
+  // rows 11.2 and 10.0, 16,384 rows 25.6 and 26.8.
+  const bool wide = a.N <= kActWideRows;
   const void* kern = activation == PPO_ACT_TANH ? act_kernel_act<PPO_ACT_TANH>(hidden, wide)
                                                 : act_kernel_act<PPO_ACT_RELU>(hidden, wide);
   if (!kern) return PPO_ERR_UNSUPPORTED;
