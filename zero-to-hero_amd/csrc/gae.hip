@@ -407,6 +407,10 @@ constexpr size_t kResSlotBase = kSyncWords;
 // per workgroup: n, sum and sum of squares of its advantages, and the centred
 // sum of squares of the exact second pass (gae_resident_kernel, step 4)
 constexpr size_t kResPartWords = 4;
+// column pass of up to kColTagged workgroups, per workgroup: n, sum and sum of
+// squares as tagged words
+constexpr long kColTagged = 64;
+constexpr size_t kColPartWords = 6;
 size_t res_slot_words(const ResPlan& rp) {
   if (!rp.E) return 0;
   return kResSlotBase + (size_t)rp.tiles() * 2 * rp.E + (size_t)rp.rounds * rp.nc * rp.E +
@@ -416,7 +420,8 @@ size_t res_slot_words_max(long T, long N) {
   const ColPlan cp = col_plan(T, N, true);
   return std::max({res_slot_words(res_plan(T, N, true, kResFewTiles)),
                    res_slot_words(res_plan(T, N, false, kResFewTiles)),
-                   cp.wgs > 1 ? kResSlotBase + (size_t)cp.wgs * kResPartWords : 0});
+                   cp.wgs <= kColTagged ? (size_t)cp.wgs * kColPartWords
+                                        : kResSlotBase + (size_t)cp.wgs * kResPartWords});
 }
 
 struct GaeLayout {
@@ -2231,7 +2236,7 @@ int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
 // steps, one env per thread, rows in registers from load to store, any N and
 // any alignment), so no carry crosses workgroups; with the normaliser the
 // workgroups exchange only their fp64 (n, sum, sum of squares) through the
-// slots of grid_sync.hpp (a single workgroup exchanges nothing) and write the
+// words of grid_sync.hpp (a single workgroup exchanges nothing) and write the
 // normalised advantages from the registers.
 //
 // What bounds it: latency -- one round of loads, the scan, the exchange, the
@@ -2248,8 +2253,7 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
   constexpr int SW = kWave / E;  // segments per wave
   __shared__ double2 s_wc[kColWaves][E];
   __shared__ float s_norm[2];
-  __shared__ unsigned s_tag;
-  __shared__ uint64_t s_epoch;
+  __shared__ CallTag s_tag;
   const int tid = threadIdx.x;
   const int lane = tid % kWave, w = tid / kWave, j = lane / E, e = tid % E;
   // neighbouring columns, which share cache lines, on one XCD
@@ -2257,16 +2261,19 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
   const long col = nwg % kXcds == 0 ? (long)blockIdx.x % kXcds * (nwg / kXcds) + blockIdx.x / kXcds
                                     : (long)blockIdx.x;
   const bool multi = kStats && nwg > 1;
-  uint64_t* part = a.slots + kResSlotBase;  // [grid][kResPartWords]
+  // up to kColTagged workgroups exchange tagged words, more of them slots behind
+  // a start barrier (us of device time, tagged and slots: 128 x 64, 4 workgroups,
+  // 7.2 and 8.6; 2048 x 64, 16 workgroups, 12.4 and 13.1; 1000 x 1023, 128
+  // workgroups, 17.7 and 16.5)
+  const bool tagged = nwg <= kColTagged;
+  uint64_t* part = a.slots + kResSlotBase;  // (slots) [grid][kResPartWords]
   int fail = 0;
-  if (multi && w == 0) {
-    uint64_t epoch;
-    const unsigned tag = launch_tag(&a.hdr->epoch, a.nonce, epoch);
-    if (tid == 0) {
-      s_tag = tag;
-      s_epoch = epoch;
-    }
-    sync_start(a.slots, part + (size_t)blockIdx.x * kResPartWords, (int)kResPartWords, tag);
+  uint64_t epoch = 0;  // (thread 0)
+  unsigned nonce = 0;  // (thread 0) the start barrier's tag
+  if (multi && tagged && tid == 0) s_tag = call_tag(&a.hdr->epoch, a.nonce, epoch);
+  if (multi && !tagged && w == 0) {
+    nonce = launch_tag(&a.hdr->epoch, a.nonce, epoch);
+    sync_start(a.slots, part + (size_t)blockIdx.x * kResPartWords, (int)kResPartWords, nonce);
   }
   const long env = col * E + e;
   const long T = a.T;
@@ -2362,24 +2369,34 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
   if constexpr (kStats) {
     block_sum_lds<3>(acc);
     if (multi) {
-      if (tid == 0) {
-        uint64_t* pp = part + (size_t)blockIdx.x * kResPartWords;
-        slot_put(pp + 0, acc[0]);
-        slot_put(pp + 1, acc[1]);
-        slot_put(pp + 2, acc[2]);
-        if (!res_wait(a.slots, s_tag, gridDim.x, a.wc.spin)) fail = 1;
-        if (blockIdx.x == 0) epoch_advance(&a.hdr->epoch, s_epoch);
-      }
-      lds_barrier();
-      // every workgroup reads all partials in one order: the same bits in each
-      acc[0] = acc[1] = acc[2] = 0.0;
-      for (long u = tid; u < nwg; u += kColBlock) {
-        uint64_t* pp = part + (size_t)u * kResPartWords;
-        acc[0] += slot_get(pp + 0, a.wc.spin, fail);
-        acc[1] += slot_get(pp + 1, a.wc.spin, fail);
-        acc[2] += slot_get(pp + 2, a.wc.spin, fail);
+      // (every workgroup reads all partials in one order: the same bits in each)
+      if (tagged) {
+        const CallTag tag = s_tag;
+        if (tid == 0) {
+          uint64_t* pp = a.slots + (size_t)blockIdx.x * kColPartWords;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) tagged_put(pp + 2 * k, acc[k], tag);
+        }
+        acc[0] = acc[1] = acc[2] = 0.0;
+        if (tid < nwg)
+          tagged_get<3>(a.slots + (size_t)tid * kColPartWords, tag, a.wc.spin, fail, acc);
+      } else {
+        if (tid == 0) {
+          uint64_t* pp = part + (size_t)blockIdx.x * kResPartWords;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) slot_put(pp + k, acc[k]);
+          if (!res_wait(a.slots, nonce, gridDim.x, a.wc.spin)) fail = 1;
+        }
+        lds_barrier();
+        acc[0] = acc[1] = acc[2] = 0.0;
+        if (tid < nwg) {
+          uint64_t* pp = part + (size_t)tid * kResPartWords;
+#pragma unroll
+          for (int k = 0; k < 3; ++k) acc[k] = slot_get(pp + k, a.wc.spin, fail);
+        }
       }
       block_sum_lds<3>(acc);
+      if (blockIdx.x == 0 && tid == 0) epoch_advance(&a.hdr->epoch, epoch);
     }
     if (tid == 0) {
       const NormParams np_ = norm_params_of(acc, a.eps);

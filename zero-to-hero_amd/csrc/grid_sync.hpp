@@ -156,6 +156,59 @@ __device__ inline void epoch_advance(uint64_t* epoch, uint64_t e) {
   __hip_atomic_store(epoch, e + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
+// Tagged words: a double that travels between workgroups as two 64-bit words,
+// each half of it beside half of the call's tag, so that a reader knows a value
+// of this call from whatever the words held before: no emptying, no start
+// barrier, one hop from the store to the reader.  The tag is a hash of the
+// workspace's call counter and the host's nonce; its halves are odd, so a
+// zeroed word never carries one.  (For few readers: where 128 or more workgroups
+// poll one another's words, a start barrier and slots measured faster.  Sleeping
+// longer between polls only adds to the wait.)  Every workgroup reads the counter before it
+// publishes, and workgroup 0 advances it (epoch_advance) once it has read every
+// workgroup's words.
+struct CallTag {
+  unsigned lo, hi;
+};
+
+__device__ inline CallTag call_tag(const uint64_t* epoch, unsigned nonce, uint64_t& e) {
+  e = __hip_atomic_load(epoch, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  uint64_t h = (e * 0x9E3779B97F4A7C15ULL + nonce) * 0xD6E8FEB86659FD93ULL;
+  h ^= h >> 32;
+  return {(unsigned)h | 1u, (unsigned)(h >> 32) | 1u};
+}
+
+__device__ __forceinline__ void tagged_put(uint64_t* p, double x, CallTag t) {
+  const uint64_t b = __builtin_bit_cast(uint64_t, x);
+  __hip_atomic_store(p, b << 32 | t.lo, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __hip_atomic_store(p + 1, (b & 0xFFFFFFFF00000000ULL) | t.hi, __ATOMIC_RELAXED,
+                     __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Polls the words of K doubles together, up to `spin` times; when a tag is
+// still missing they read as NaN and `fail` is set (spin 0: gives up at once).
+template <int K>
+__device__ __forceinline__ void tagged_get(uint64_t* p, CallTag t, long spin, int& fail,
+                                           double (&x)[K]) {
+  for (long it = 0; it < spin; ++it) {
+    uint64_t w[2 * K];
+#pragma unroll
+    for (int k = 0; k < 2 * K; ++k) w[k] = slot_peek(p + k);
+    bool ok = true;
+#pragma unroll
+    for (int k = 0; k < 2 * K; ++k) ok = ok && (unsigned)w[k] == (k % 2 ? t.hi : t.lo);
+    if (ok) {
+#pragma unroll
+      for (int k = 0; k < K; ++k)
+        x[k] = __builtin_bit_cast(double, (w[2 * k + 1] & 0xFFFFFFFF00000000ULL) | w[2 * k] >> 32);
+      return;
+    }
+    __builtin_amdgcn_s_sleep(1);
+  }
+  fail = 1;
+#pragma unroll
+  for (int k = 0; k < K; ++k) x[k] = __builtin_nan("");
+}
+
 // A different tag for every launch (zero is skipped).
 inline unsigned next_nonce() {
   static std::atomic<unsigned> calls{0x5bd1e995u};

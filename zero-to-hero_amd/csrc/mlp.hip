@@ -1009,23 +1009,24 @@ __global__ void __launch_bounds__(kWaves * kWave) mlp_grad_reduce_kernel(MlpArgs
 // when the reduction grid is resident on the device at once).  Each
 // workgroup sums its parameters' gradient partials as
 // mlp_grad_reduce_kernel does and publishes the sum of squares of the fp32
-// gradients to a slot (grid_sync.hpp: value-tagged 64-bit words, cleared by
-// the owner before a start barrier); then every workgroup reads all slots
-// and forms the per-tensor norms, the total norm and the clip coefficient
+// gradients as tagged words (grid_sync.hpp); then every workgroup reads all of
+// them and forms the per-tensor norms, the total norm and the clip coefficient
 // in the order adam_update_kernel uses (wave w takes tensors w, w + kWaves,
 // ...; lane l sums a tensor's partials l, l + 64, ... in fp64, then the wave
 // tree; adam_coef_from_norms), and updates its parameters from registers.
 // The results are bit-identical to the reduction + adam_update_kernel
-// launches, with one dependent launch fewer per minibatch.
+// launches, with one dependent launch fewer per minibatch.  What bounds it: two
+// dependent trips to memory (the partials, the other workgroups' words); behind
+// slots emptied before a start barrier there was a third (whole step, us: 256 rows
+// 4-64-64-2 18.1 -> 17.5, 128 rows 4-128-128-2 25.4 -> 22.9).
 struct MlpAdamArgs {
   float* p[kMlpTensors];
   float* m[kMlpTensors];
   float* v[kMlpTensors];
   AdamScalars s;
   float* norm_out;
-  uint64_t* sync;  // start barrier (kSyncWords words)
-  uint64_t* sq;    // per reduction workgroup: its sum-of-squares slot
-  uint64_t* epoch; // the workspace header's call counter (launch_tag)
+  uint64_t* sq;    // per reduction workgroup: its sum of squares (tagged words)
+  uint64_t* epoch; // the workspace header's call counter (call_tag)
   unsigned nonce;
   WaitCtl wc;      // poll limit and the device's wait-status word
 };
@@ -1046,19 +1047,19 @@ __global__ void __launch_bounds__(kWaves * kWave) mlp_reduce_adam_kernel(MlpArgs
   const long li = valid ? local : 0;
   const long pc = a.toff[j] + li;
   // wave 0: this workgroup's parameters and moments (they do not depend on
-  // the norm), the step count (read before arriving: workgroup 0 advances it
-  // only once every workgroup has arrived), its slot emptied, arrival
+  // the norm) and the step count (read before publishing: workgroup 0 advances
+  // it only once every workgroup has published)
   float pr = 0.0f, mr = 0.0f, vr = 0.0f;
   int64_t step0 = 0;
-  unsigned tag = 0;  // (wave 0)
-  uint64_t epoch = 0;
+  __shared__ CallTag s_tag;
+  uint64_t epoch = 0;  // (wave 0)
   if (w == 0) {
     pr = u.p[j][li];
     mr = u.m[j][li];
     vr = u.v[j][li];
     if (a.step_counter) step0 = *a.step_counter;
-    tag = launch_tag(u.epoch, u.nonce, epoch);
-    sync_start(u.sync, u.sq + blk, 1, tag);
+    const CallTag tag = call_tag(u.epoch, u.nonce, epoch);
+    if (lane == 0) s_tag = tag;
   }
   double s = 0.0;
   for (long b0 = w; b0 < a.nblocks; b0 += kRedLoads * kWaves) {
@@ -1081,7 +1082,10 @@ __global__ void __launch_bounds__(kWaves * kWave) mlp_reduce_adam_kernel(MlpArgs
     for (int k = 1; k < kWaves; ++k) t += s_sum[k][lane];
     g = (float)t;
     const double sq = wave_sum(valid ? (double)g * (double)g : 0.0);
-    if (lane == 0) slot_put(u.sq + blk, sq);
+    if (lane == 0) {
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the step count and the counter are read
+      tagged_put(u.sq + 2 * blk, sq, s_tag);
+    }
   }
   if (blk == 0) {
     double tot[kMlpSums];
@@ -1102,31 +1106,24 @@ __global__ void __launch_bounds__(kWaves * kWave) mlp_reduce_adam_kernel(MlpArgs
       a.scalars[PPO_SCALAR_LOSS] = (pol + a.vc * vl) - a.ec * ent;
     }
   }
-  // A wait that gives up (grid not co-resident) may leave slots unread or
-  // read before their owner emptied them: this workgroup then writes none of
-  // its parameters, moments or gradients (and workgroup 0 neither the step
+  // A wait that gives up (grid not co-resident): this workgroup then writes none
+  // of its parameters, moments or gradients (and workgroup 0 neither the step
   // counter; the norm output reads NaN), and raises the wait-status word.
   int fail = 0;
-  if (threadIdx.x == 0) {
-    if (!res_wait(u.sync, tag, gridDim.x, u.wc.spin)) fail = 1;
-    if (blk == 0) epoch_advance(u.epoch, epoch);
-  }
-  // (after the barrier every workgroup has arrived and emptied its slot)
-  if (__syncthreads_or(fail)) {
-    if (threadIdx.x == 0) {
-      wait_report(u.wc.status);
-      if (blk == 0 && u.norm_out) *u.norm_out = __builtin_nanf("");
-    }
-    return;
-  }
+  const CallTag tag = s_tag;  // (every wave is past the barrier after the partial sums)
   for (int kk = w; kk < kMlpTensors; kk += kWaves) {
     double acc = 0.0;
-    for (long c = a.tblk[kk] + lane; c < a.tblk[kk + 1]; c += kWave)
-      acc += slot_get(u.sq + c, u.wc.spin, fail);
+    for (long c = a.tblk[kk] + lane; c < a.tblk[kk + 1]; c += kWave) {
+      double x[1];
+      tagged_get<1>(u.sq + 2 * c, tag, u.wc.spin, fail, x);
+      acc += x[0];
+    }
     const double sk = wave_sum(acc);
     if (lane == 0) s_norm[kk] = (float)sqrt(sk);
   }
-  if (__syncthreads_or(fail)) {
+  const int failed = __syncthreads_or(fail);
+  if (blk == 0 && threadIdx.x == 0) epoch_advance(u.epoch, epoch);
+  if (failed) {
     if (threadIdx.x == 0) {
       wait_report(u.wc.status);
       if (blk == 0 && u.norm_out) *u.norm_out = __builtin_nanf("");
@@ -1176,7 +1173,7 @@ struct MlpLayout {
   long P, nblocks, rblocks;
   int threads;  // of the gradient kernel's workgroups
   long tblk[kMlpTensors + 1], toff[kMlpTensors], tnum[kMlpTensors];
-  size_t gpart, spart, sqpart, sync, total;
+  size_t gpart, spart, sqpart, total;
 };
 
 MlpLayout mlp_layout(long B, int D, int H, int A) {
@@ -1198,8 +1195,7 @@ MlpLayout mlp_layout(long B, int D, int H, int A) {
   l.gpart = kHeaderBytes;
   l.spart = l.gpart + align_up((size_t)l.nblocks * l.P * sizeof(float), 256);
   l.sqpart = l.spart + align_up((size_t)kMlpSums * l.nblocks * sizeof(double), 256);
-  l.sync = l.sqpart + align_up((size_t)l.rblocks * sizeof(double), 256);
-  l.total = l.sync + kSyncWords * sizeof(uint64_t);
+  l.total = l.sqpart + align_up((size_t)l.rblocks * 2 * sizeof(uint64_t), 256);
   return l;
 }
 
@@ -1466,7 +1462,6 @@ extern "C" int ppo_mlp_cat_step_f32(const ppo_mlp3_f32* actor, const ppo_mlp3_f3
     }
     u.s = make_adam_scalars(adam);
     u.norm_out = grad_norm_out;
-    u.sync = reinterpret_cast<uint64_t*>(static_cast<char*>(workspace) + l.sync);
     u.sq = reinterpret_cast<uint64_t*>(a.sqpart);
     u.epoch = &reinterpret_cast<WsHeader*>(workspace)->epoch;
     u.nonce = next_nonce();
