@@ -262,6 +262,19 @@ def test_vecppo_fused_mlp_matches_unfused(dev, graphs):
         torch.testing.assert_close(s_f[k], s_u[k], rtol=1e-4, atol=1e-6)
 
 
+@pytest.mark.parametrize("H", [16, 32, 64, 128])
+@pytest.mark.parametrize("A", [1, 16, 17, 32])
+def test_mlp_act_draws_as_the_sampling_kernel(dev, H, A):
+    """The fused launch's draw on its own logits: sample_categorical's bits."""
+    pol, val, _, gpu = _case(dev, 37, 64, H, A, "relu", seed=H + A)
+    pol, val = pol.to(dev), val.to(dev)
+    u = torch.rand(37, generator=torch.Generator().manual_seed(A)).to(dev)
+    act, lp, v = ppo_amd.mlp_act_categorical(pol, val, gpu["obs"], uniforms=u)
+    logits, v_ref = ppo_amd.mlp_forward_categorical(pol, val, gpu["obs"])
+    act_ref, lp_ref = ppo_amd.sample_categorical(logits, u)
+    assert torch.equal(act, act_ref) and torch.equal(lp, lp_ref) and torch.equal(v, v_ref)
+
+
 @pytest.mark.parametrize("H", [64, 128])
 def test_mlp_act_wide_and_narrow_forms_agree(dev, H):
     """8193 rows take the narrow form, 8192 and fewer the wide one: the same

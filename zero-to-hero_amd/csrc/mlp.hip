@@ -792,10 +792,26 @@ __global__ void __launch_bounds__(kBlock) mlp_act_cat_kernel(ActArgs a) {
     if (tid < R && row0 + tid < a.N) a.val[row0 + tid] = s_v[tid];
     return;
   }
+  // The draw's exponentials by all threads, its running sums by a lane per row
+  // (sample_cat_row's bits).  By a lane per row alone, 2 A exponentials in turn,
+  // 4096 rows of 60-64-64-18 took 11.2 us; so 10.2.  (In the observations' LDS: more
+  // of it costs H = 128 a workgroup per CU, 16,384 rows 25 -> 37 us.)
+  static_assert(kZld + 1 <= kXld, "the draw's exponentials and maxima fit there");
+  float* s_e = s_x;
+  float* s_m = s_x + R * kZld;
+  for (int e = tid; e < R * a.A; e += kBlock) {
+    const int r = e / a.A, j = e - r * a.A;
+    const float* zr = s_z + r * kZld;
+    float m = -INFINITY;
+    for (int k = 0; k < a.A; ++k) m = fmaxf(m, zr[k]);
+    s_e[r * kZld + j] = expf(zr[j] - m);
+    if (j == 0) s_m[r] = m;
+  }
+  lds_barrier();
   if (tid < R && row0 + tid < a.N) {
     int act;
     float lp;
-    sample_cat_row(s_z + tid * kZld, a.A, u, act, lp);
+    sample_cat_exps(s_e + tid * kZld, s_z + tid * kZld, s_m[tid], a.A, u, act, lp);
     a.act[row0 + tid] = act;
     a.logp[row0 + tid] = lp;
     a.val[row0 + tid] = s_v[tid];

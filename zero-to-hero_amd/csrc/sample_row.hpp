@@ -34,4 +34,24 @@ __device__ __forceinline__ void sample_cat_row(const float* zr, int A, float u, 
   logp = (zr[a] - m) - logf(s);
 }
 
+// The same draw from the row's exponentials e_j = expf(z_j - m), formed
+// beforehand (by many lanes): the same sums in the same order.
+__device__ __forceinline__ void sample_cat_exps(const float* er, const float* zr, float m, int A,
+                                                float u, int& action, float& logp) {
+  float s = 0.0f;
+  for (int j = 0; j < A; ++j) s += er[j];
+  const float target = u * s;
+  float c = 0.0f;
+  int a = -1, last_pos = 0;
+  for (int j = 0; j < A; ++j) {
+    const float e = er[j];
+    c += e;
+    if (e > 0.0f) last_pos = j;
+    if (a < 0 && target < c) a = j;
+  }
+  if (a < 0) a = last_pos;
+  action = a;
+  logp = (zr[a] - m) - logf(s);
+}
+
 }  // namespace ppo
