@@ -654,6 +654,38 @@ def test_backward_scales_saved_gradients(dev, B):
     torch.testing.assert_close(gg, dl.sum())
 
 
+@pytest.mark.parametrize("validate", [False, True])
+def test_backward_of_batched_gradients(dev, validate):
+    """Incoming gradients that have no storage of their own to scale by
+    (is_grads_batched) and dispatch modes: torch's products, bit for bit."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    class Seen(TorchDispatchMode):
+        names = []
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            self.names.append(str(func))
+            return func(*args, **(kwargs or {}))
+
+    logits, actions, old_lp, adv, ret, val, _ = (x.to(dev) for x in cat_inputs(33, 5, seed=3))
+    _, dl, dv = ppo_amd.ppo_loss_discrete_fused(logits, actions, old_lp, adv, ret, val)
+    scales = torch.tensor([1.0, -0.5, 3.0], device=dev)
+
+    def leaves():
+        x, v = logits.clone().requires_grad_(), val.clone().requires_grad_()
+        return x, v, ppo_amd.ppo_loss_discrete(x, actions, old_lp, adv, ret, v,
+                                               validate_args=validate)[0]
+
+    x, v, loss = leaves()
+    gx, gv = torch.autograd.grad(loss, (x, v), grad_outputs=scales, is_grads_batched=True)
+    assert torch.equal(gx, dl * scales.view(3, 1, 1)) and torch.equal(gv, dv * scales.view(3, 1))
+    x, v, loss = leaves()
+    with Seen() as seen:
+        loss.backward()
+    assert torch.equal(x.grad, dl) and torch.equal(v.grad, dv)
+    assert any("mul" in n for n in seen.names)
+
+
 def test_empty_batches_raise_like_the_reference(dev):
     """A minibatch of no rows: the reference's Categorical / Normal on an
     empty batch raises (torch cannot validate a [0, A] tensor, and the means

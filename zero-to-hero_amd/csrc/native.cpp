@@ -56,22 +56,29 @@ void need(bool ok) {
 }
 
 // Modes and transforms that want to see torch operators: not for this path.
-void need_plain_mode() {
-  need(!at::impl::torch_function_mode_enabled() &&
-       !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
-       !c10::impl::tls_is_dispatch_key_included(
-           c10::DispatchKey::FuncTorchDynamicLayerFrontMode));
+bool plain_mode() {
+  return !at::impl::torch_function_mode_enabled() &&
+         !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
+         !c10::impl::tls_is_dispatch_key_included(
+             c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
 }
+
+void need_plain_mode() { need(plain_mode()); }
+
+// Keys of tensors that stand for another tensor, or for none: no storage of
+// their own to read.
+constexpr c10::DispatchKeySet kWrapped({c10::DispatchKey::Python, c10::DispatchKey::Batched,
+                                        c10::DispatchKey::FuncTorchBatched,
+                                        c10::DispatchKey::FuncTorchGradWrapper,
+                                        c10::DispatchKey::Functionalize,
+                                        c10::DispatchKey::Negative, c10::DispatchKey::Conjugate,
+                                        c10::DispatchKey::ZeroTensor});
 
 // A torch.Tensor (or Parameter) itself: no subclass, no wrapper, dense GPU
 // storage, contiguous.
 const Tensor& plain(PyObject* o, at::ScalarType type) {
   need(THPVariable_CheckExact(o));
   const Tensor& t = THPVariable_Unpack(o);
-  static constexpr c10::DispatchKeySet kWrapped(
-      {c10::DispatchKey::Python, c10::DispatchKey::FuncTorchBatched,
-       c10::DispatchKey::FuncTorchGradWrapper, c10::DispatchKey::Functionalize,
-       c10::DispatchKey::Negative, c10::DispatchKey::Conjugate, c10::DispatchKey::ZeroTensor});
   need(t.defined() && t.is_cuda() && t.layout() == at::kStrided &&
        !t.key_set().has_any(kWrapped) && t.scalar_type() == type && t.is_contiguous());
   return t;
@@ -306,6 +313,15 @@ Loss loss_gaussian_launch(PyObject* const* a) {  // mu, log_std, actions, rows..
   return l;
 }
 
+// A loss's incoming gradient that the scale kernel can read on `device`.  Batched
+// gradients (is_grads_batched), fake tensors and dispatch modes see torch's
+// products instead.
+bool plain_scale(const Tensor& g, const at::Device& device) {
+  return plain_mode() && g.is_cuda() && g.layout() == at::kStrided &&
+         !g.key_set().has_any(kWrapped) && g.scalar_type() == at::kFloat && g.numel() == 1 &&
+         g.device() == device;
+}
+
 // The losses' node: saved gradients times the loss's incoming gradient (the
 // rules of ops._scaled_grads).
 struct LossNode : public torch::autograd::Function<LossNode> {
@@ -324,8 +340,7 @@ struct LossNode : public torch::autograd::Function<LossNode> {
     const size_t n = grads.size();
     if (!g[0].defined()) return variable_list(n + 1);
     const Tensor& scale = g[0];
-    if (at::GradMode::is_enabled() || scale.scalar_type() != at::kFloat || scale.numel() != 1 ||
-        scale.device() != grads[0].device()) {
+    if (at::GradMode::is_enabled() || !plain_scale(scale, grads[0].device())) {
       for (Tensor& t : grads) t = t * scale;
     } else {
       // sole owners: the saved variable and `grads`
@@ -602,11 +617,13 @@ PyMethodDef kMethods[] = {
 #undef PPO_ENTRY
 
 // dst[k] = src[k] * scale (a one-element fp32 tensor) in one launch; all
-// contiguous fp32 on one device.  Returns the library's status code.
+// contiguous fp32 on one device.  Returns the library's status code, or -1 for a
+// scale that the kernel cannot read.
 int scale_grads(const std::vector<Tensor>& src, const std::vector<Tensor>& dst,
                 const Tensor& scale) {
   TORCH_CHECK(!src.empty() && src.size() == dst.size() && src.size() <= ppo::kMaxScaleArrays,
               "scale_grads takes 1 to ", ppo::kMaxScaleArrays, " tensors");
+  if (!plain_scale(scale, src[0].device())) return -1;
   ppo::ScaleArray a[ppo::kMaxScaleArrays];
   for (size_t k = 0; k < src.size(); ++k) {
     TORCH_CHECK(src[k].scalar_type() == at::kFloat && dst[k].scalar_type() == at::kFloat &&
@@ -616,8 +633,6 @@ int scale_grads(const std::vector<Tensor>& src, const std::vector<Tensor>& dst,
                 "scale_grads takes contiguous fp32 tensors of one size on one device");
     a[k] = {in(src[k]), out(dst[k]), src[k].numel()};
   }
-  TORCH_CHECK(scale.is_cuda() && scale.scalar_type() == at::kFloat && scale.numel() == 1,
-              "scale must be a one-element fp32 GPU tensor");
   return ppo::launch_scale(a, (int)src.size(), in(scale), current_stream(scale.device()));
 }
 

@@ -752,8 +752,9 @@ def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
     saved-tensor hooks, no other reference to them -- they are scaled in place
     and returned themselves; the launch then touches nothing if the incoming
     gradient is 1, as it is for loss.backward().  Otherwise they are scaled into
-    new tensors, and under create_graph by torch's own operators, which keep
-    the dependence on the incoming gradient."""
+    new tensors, and by torch's own operators under create_graph, which keep
+    the dependence on the incoming gradient, and for an incoming gradient
+    without storage of its own (batched gradients, fake tensors)."""
     saved = ctx.saved_tensors
     if grad_loss is None:
         return (None,) * len(saved)
@@ -763,7 +764,10 @@ def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
     own = (not ctx.hooked and not torch._C._autograd._get_current_graph_task_keep_graph()
            and all(sys.getrefcount(t) == _SOLE_REFS for t in grads))
     outs = grads if own else [torch.empty_like(t) for t in grads]
-    _lib.check("scale_grads", _lib.native().scale_grads(grads, outs, grad_loss))
+    code = _lib.native().scale_grads(grads, outs, grad_loss)
+    if code < 0:
+        return tuple(t * grad_loss for t in saved)
+    _lib.check("scale_grads", code)
     return tuple(outs)
 
 
