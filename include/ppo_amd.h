@@ -56,9 +56,10 @@ const char* ppo_amd_strerror(int code);
 
 /*
  * Status of the bounded in-kernel waits (no counterpart in the reference: its
- * update runs on the CPU in one thread).  Four launches hold workgroups that
+ * update runs on the CPU in one thread).  Five launches hold workgroups that
  * wait for one another inside the launch: the resident GAE pass
- * (ppo_gae_f32 / ppo_gae_norm_f32, PPO_GAE_ROUTE_RESIDENT), the Gaussian loss
+ * (ppo_gae_f32 / ppo_gae_norm_f32, PPO_GAE_ROUTE_RESIDENT), the column GAE
+ * pass with the normaliser (PPO_GAE_ROUTE_COLUMN), the Gaussian loss
  * with its in-kernel finish (ppo_loss_gauss_f32), the categorical loss, which
  * also finishes in-kernel (ppo_loss_cat_f32 and its _noalloc form: every batch
  * on the wave-tile kernels, whose workgroup 0 only collects, batches of at
@@ -171,7 +172,8 @@ int ppo_gae_norm_f32(const float* rewards, const float* values,
  * of the PPO_GAE_ROUTE_* values (diagnostics and tests; no counterpart in the
  * reference).  has_values = 0 means values == NULL.  Misaligned buffers take
  * the scalar tile passes whatever this returns.  The environment variable
- * PPO_AMD_GAE_RESIDENT=0 turns the resident pass off.
+ * PPO_AMD_GAE_RESIDENT=0 turns off the resident pass and the column pass
+ * wherever its workgroups exchange statistics.
  */
 #define PPO_GAE_ROUTE_NONE 0      /* empty or oversized rollout                */
 #define PPO_GAE_ROUTE_RESIDENT 1  /* one launch, whole rollout in registers    */

@@ -366,7 +366,7 @@ struct ColPlan {
 
 // A workgroup touches every row of the horizon once per array whatever E is (16,
 // 32 or 64 bytes of it), so its time grows with T: taken to T = 2048 (2048 x 64
-// with the normaliser 13 us, 4096 x 64 28 us against 19 of the span passes).
+// with the normaliser 12 us, 4096 x 64 28 us against 19 of the span passes).
 // Narrow columns give more workgroups, wide ones longer row pieces: 16 envs to
 // 256 steps, then 4, or 8 where 4 would give more than 64 workgroups (1000 x 64
 // 10.2 against 11.6 us, 1000 x 1023 17.2 against 16.5; 2048 x 2047 without the
@@ -2243,7 +2243,7 @@ int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
 // stores.  Measured on MI355X against the 3 or 4 launches of the span and tile
 // passes (T x N, us of device time per call, with / without the normaliser):
 //   128 x 8      15.0 -> 5.3 / 5.9 -> 3.6      1000 x 64    18.2 -> 10.3 / 11.6 -> 5.6
-//   1000 x 1023  21.4 -> 16.4 / 16.2 -> 10.8   2048 x 64    18.4 -> 13.1 / 11.4 -> 8.0
+//   1000 x 1023  21.4 -> 16.4 / 16.2 -> 10.8   2048 x 64    18.4 -> 12.4 / 11.4 -> 8.0
 //   200 x 2048   19.2 -> 10.3 / 14.4 -> 4.9    2048 x 2047  45.5 -> 30.2 / 36.0 -> 21.4
 // ---------------------------------------------------------------------------
 constexpr int kColWaves = kColBlock / kWave;

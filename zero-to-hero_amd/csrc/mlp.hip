@@ -949,7 +949,8 @@ __global__ void __launch_bounds__(kMlpBlock) mlp_cartpole_rollout_kernel(Rollout
 // read from HBM at a stride of the whole parameter count, so the kernel is
 // latency-bound: for >= 128 partial rows, 16 waves x 16 loads put a
 // 4096-row minibatch's 256 rows in flight at once (update of T=2048 x N=64 in
-// minibatches of 4096: 4.69 -> 4.37 ms); fewer rows keep 4 waves x 8 loads.
+// minibatches of 4096: 4.69 -> 4.37 ms); fewer rows keep 4 waves x 8 loads
+// (reduce_waves: 8 where the grid is too large for one round of 16).
 // With sqpart the workgroup also leaves the fp64 sum of the squares of the
 // fp32 gradients it wrote (clip_grad_norm_'s per-tensor sums, in pieces).
 // Workgroup 0 also forms the loss scalars.
@@ -1183,7 +1184,6 @@ NetOffsets net_offsets(long base, int D, int H, int O) {
 // half / this / twice the number: 32,768 rows H = 128 196 / 115 / 123, H = 64
 // 74 / 55 / 61, H = 32 43 / 30 / 39, H = 16 26 / 25 / 36.
 constexpr long grad_groups(int H) { return 128L * 128 / H; }
-
 
 struct MlpLayout {
   long P, nblocks, rblocks;
