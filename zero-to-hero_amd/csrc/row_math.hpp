@@ -140,11 +140,11 @@ __device__ __forceinline__ RowOut cat_row_grad(const P& a, float* zr, int A, int
 #pragma unroll
   for (int j = 0; j < MAXA; ++j)
     if (j < MINA || j < A) {
-      const float d = t[j] - m;
       // (a NaN logit, or an infinite one: inf - inf, is NaN in e and so in s
-      // and in the row's whole gradient)
-      const float ej = __builtin_amdgcn_exp2f(d * kLog2e);
-      const float tj = fmaxf(d, -FLT_MAX);
+      // and in the row's whole gradient; a maximum that keeps it is one
+      // instruction, fmaxf beside the exponential of the difference two)
+      const float tj = __builtin_elementwise_maximum(t[j] - m, -FLT_MAX);
+      const float ej = __builtin_amdgcn_exp2f(tj * kLog2e);
       t[j] = tj;
       e[j] = ej;
       s += ej;
