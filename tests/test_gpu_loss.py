@@ -655,6 +655,37 @@ def test_backward_scales_saved_gradients(dev, B):
 
 
 @pytest.mark.parametrize("validate", [False, True])
+@pytest.mark.parametrize("kind", ["strided", "expanded", "half", "double"])
+def test_backward_of_tensors_that_hooks_replaced(dev, kind, validate):
+    """Saved-tensor hooks may hand backward another tensor than the kernel saved:
+    a row of a padded pool, an expanded one, another type.  The gradient is torch's
+    product of that tensor and the incoming gradient, bit for bit."""
+
+    def unpack(t):
+        if kind == "strided":
+            pool = torch.full((t.shape[0], 7, *t.shape[1:]), 9.0, device=dev)
+            pool[:, 3] = t
+            return pool[:, 3]
+        if kind == "expanded":
+            return t[:1].expand_as(t)
+        return t.half() if kind == "half" else t.double()
+
+    B, A = 100, 5
+    logits, actions, old_lp, adv, ret, val, _ = (x.to(dev) for x in cat_inputs(B, A, seed=B))
+    _, dl, dv = ppo_amd.ppo_loss_discrete_fused(logits, actions, old_lp, adv, ret, val)
+    for scale in (1.0, -3.0):
+        x, v = logits.clone().requires_grad_(), val.clone().requires_grad_()
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            loss = ppo_amd.ppo_loss_discrete(x, actions, old_lp, adv, ret, v,
+                                             validate_args=validate)[0]
+        print(f"hooked backward kind={kind} validate={validate} scale={scale}", flush=True)
+        (loss * scale).backward()
+        g = torch.tensor(scale, device=dev)
+        assert torch.equal(x.grad, (unpack(dl) * g).float())
+        assert torch.equal(v.grad, (unpack(dv) * g).float())
+
+
+@pytest.mark.parametrize("validate", [False, True])
 def test_backward_of_batched_gradients(dev, validate):
     """Incoming gradients that have no storage of their own to scale by
     (is_grads_batched) and dispatch modes: torch's products, bit for bit."""

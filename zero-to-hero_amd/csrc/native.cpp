@@ -313,13 +313,36 @@ Loss loss_gaussian_launch(PyObject* const* a) {  // mu, log_std, actions, rows..
   return l;
 }
 
-// A loss's incoming gradient that the scale kernel can read on `device`.  Batched
-// gradients (is_grads_batched), fake tensors and dispatch modes see torch's
-// products instead.
-bool plain_scale(const Tensor& g, const at::Device& device) {
-  return plain_mode() && g.is_cuda() && g.layout() == at::kStrided &&
-         !g.key_set().has_any(kWrapped) && g.scalar_type() == at::kFloat && g.numel() == 1 &&
-         g.device() == device;
+// A tensor that the scale kernel can read: dense fp32 with storage of its own on
+// `device`.
+bool plain_f32(const Tensor& t, const at::Device& device) {
+  return t.is_cuda() && t.layout() == at::kStrided && !t.key_set().has_any(kWrapped) &&
+         t.scalar_type() == at::kFloat && t.is_contiguous() && t.device() == device;
+}
+
+// Whether the scale kernel may multiply `grads` by `scale`.  Batched gradients
+// (is_grads_batched), fake tensors and dispatch modes see torch's products
+// instead, and so do saved tensors that a hook replaced by views, other types or
+// other devices' tensors.
+bool plain_scale(const variable_list& grads, const Tensor& scale) {
+  if (!plain_mode() || scale.numel() != 1 || !plain_f32(scale, scale.device())) return false;
+  for (const Tensor& t : grads)
+    if (!plain_f32(t, scale.device())) return false;
+  return true;
+}
+
+// grads[k] * scale in one launch, into the tensors themselves (`own`) or new ones.
+variable_list scaled(const variable_list& grads, const Tensor& scale, bool own) {
+  variable_list dst = grads;
+  ppo::ScaleArray a[ppo::kMaxScaleArrays];
+  for (size_t k = 0; k < grads.size(); ++k) {
+    if (!own) dst[k] = at::empty_like(grads[k]);
+    a[k] = {in(grads[k]), out(dst[k]), dst[k].numel()};
+  }
+  const int code =
+      ppo::launch_scale(a, (int)grads.size(), in(scale), current_stream(scale.device()));
+  TORCH_CHECK(code == PPO_OK, "scaling the loss gradients failed with code ", code);
+  return dst;
 }
 
 // The losses' node: saved gradients times the loss's incoming gradient (the
@@ -328,7 +351,7 @@ struct LossNode : public torch::autograd::Function<LossNode> {
   static Tensor forward(AutogradContext* ctx, at::TensorList, const Loss* l) {
     ctx->save_for_backward(l->grads);
     ctx->set_materialize_grads(false);
-    // (saved-tensor hooks hand backward tensors that may be someone else's)
+    // (saved-tensor hooks hand backward whatever they like)
     ctx->saved_data["hooked"] = at::SavedTensorDefaultHooks::get_hooks().has_value();
     // a 0-d tensor on the scalars' storage: an indexed view's backward would
     // build and fill a [6] gradient
@@ -340,22 +363,14 @@ struct LossNode : public torch::autograd::Function<LossNode> {
     const size_t n = grads.size();
     if (!g[0].defined()) return variable_list(n + 1);
     const Tensor& scale = g[0];
-    if (at::GradMode::is_enabled() || !plain_scale(scale, grads[0].device())) {
+    if (at::GradMode::is_enabled() || ctx->saved_data["hooked"].toBool() ||
+        !plain_scale(grads, scale)) {
       for (Tensor& t : grads) t = t * scale;
     } else {
       // sole owners: the saved variable and `grads`
-      bool own = !ctx->saved_data["hooked"].toBool() &&
-                 !torch::autograd::get_current_graph_task_keep_graph();
+      bool own = !torch::autograd::get_current_graph_task_keep_graph();
       for (const Tensor& t : grads) own = own && t.use_count() == 2;
-      variable_list dst = grads;
-      ppo::ScaleArray a[ppo::kMaxScaleArrays];
-      for (size_t k = 0; k < n; ++k) {
-        if (!own) dst[k] = at::empty_like(grads[k]);
-        a[k] = {in(grads[k]), out(dst[k]), dst[k].numel()};
-      }
-      const int code = ppo::launch_scale(a, (int)n, in(scale), current_stream(scale.device()));
-      TORCH_CHECK(code == PPO_OK, "scaling the loss gradients failed with code ", code);
-      grads = std::move(dst);
+      grads = scaled(grads, scale, own);
     }
     grads.resize(n + 1);  // (the launch's results are no differentiable input)
     return grads;
@@ -616,24 +631,13 @@ PyMethodDef kMethods[] = {
     {nullptr, nullptr, 0, nullptr}};
 #undef PPO_ENTRY
 
-// dst[k] = src[k] * scale (a one-element fp32 tensor) in one launch; all
-// contiguous fp32 on one device.  Returns the library's status code, or -1 for a
-// scale that the kernel cannot read.
-int scale_grads(const std::vector<Tensor>& src, const std::vector<Tensor>& dst,
-                const Tensor& scale) {
-  TORCH_CHECK(!src.empty() && src.size() == dst.size() && src.size() <= ppo::kMaxScaleArrays,
-              "scale_grads takes 1 to ", ppo::kMaxScaleArrays, " tensors");
-  if (!plain_scale(scale, src[0].device())) return -1;
-  ppo::ScaleArray a[ppo::kMaxScaleArrays];
-  for (size_t k = 0; k < src.size(); ++k) {
-    TORCH_CHECK(src[k].scalar_type() == at::kFloat && dst[k].scalar_type() == at::kFloat &&
-                    src[k].is_contiguous() && dst[k].is_contiguous() &&
-                    src[k].numel() == dst[k].numel() && src[k].device() == scale.device() &&
-                    dst[k].device() == scale.device(),
-                "scale_grads takes contiguous fp32 tensors of one size on one device");
-    a[k] = {in(src[k]), out(dst[k]), src[k].numel()};
-  }
-  return ppo::launch_scale(a, (int)src.size(), in(scale), current_stream(scale.device()));
+// grads[k] * scale in one launch (into the tensors themselves with `own`), or
+// None for tensors that torch's products have to take.
+py::object scale_grads(const variable_list& grads, const Tensor& scale, bool own) {
+  TORCH_CHECK(!grads.empty() && grads.size() <= ppo::kMaxScaleArrays, "scale_grads takes 1 to ",
+              ppo::kMaxScaleArrays, " tensors");
+  if (!plain_scale(grads, scale)) return py::none();
+  return py::cast(scaled(grads, scale, own));
 }
 
 void init(py::object pool, py::object stats, py::object fail, const std::vector<std::string>& names,

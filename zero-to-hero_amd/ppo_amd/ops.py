@@ -729,7 +729,7 @@ def _save_grads(ctx, scalars: torch.Tensor, *grads: torch.Tensor):
     rather than an indexed view, whose backward would build and fill a [6]
     gradient; the scalars are reported values."""
     ctx.save_for_backward(*grads)
-    # (saved-tensor hooks hand backward tensors that may be someone else's)
+    # (saved-tensor hooks hand backward whatever they like)
     ctx.hooked = torch._C._autograd._top_saved_tensors_default_hooks(False) is not None
     ctx.set_materialize_grads(False)
     ctx.mark_non_differentiable(scalars)
@@ -748,27 +748,25 @@ def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
     """Backward: every saved gradient times the loss's incoming gradient.
 
     Where the graph is released after this pass (no retain_graph, no
-    create_graph) and nothing else can see the saved gradients -- no
-    saved-tensor hooks, no other reference to them -- they are scaled in place
-    and returned themselves; the launch then touches nothing if the incoming
-    gradient is 1, as it is for loss.backward().  Otherwise they are scaled into
-    new tensors, and by torch's own operators under create_graph, which keep
-    the dependence on the incoming gradient, and for an incoming gradient
-    without storage of its own (batched gradients, fake tensors)."""
+    create_graph) and nothing else holds the saved gradients, they are scaled
+    in place and returned themselves; the launch then touches nothing if the
+    incoming gradient is 1, as it is for loss.backward().  Otherwise they are
+    scaled into new tensors, and by torch's own operators under create_graph,
+    which keep the dependence on the incoming gradient, for saved tensors that
+    a hook replaced (views, other types), and for an incoming gradient without
+    storage of its own (batched gradients, fake tensors)."""
     saved = ctx.saved_tensors
     if grad_loss is None:
         return (None,) * len(saved)
-    if torch.is_grad_enabled():
+    if torch.is_grad_enabled() or ctx.hooked:
         return tuple(t * grad_loss for t in saved)
     grads = list(saved)
-    own = (not ctx.hooked and not torch._C._autograd._get_current_graph_task_keep_graph()
+    own = (not torch._C._autograd._get_current_graph_task_keep_graph()
            and all(sys.getrefcount(t) == _SOLE_REFS for t in grads))
-    outs = grads if own else [torch.empty_like(t) for t in grads]
-    code = _lib.native().scale_grads(grads, outs, grad_loss)
-    if code < 0:
+    got = _lib.native().scale_grads(grads, grad_loss, own)
+    if got is None:
         return tuple(t * grad_loss for t in saved)
-    _lib.check("scale_grads", code)
-    return tuple(outs)
+    return tuple(got)
 
 
 class _DiscreteLoss(torch.autograd.Function):
