@@ -717,6 +717,35 @@ def test_backward_of_batched_gradients(dev, validate):
     assert any("mul" in n for n in seen.names)
 
 
+@pytest.mark.parametrize("kind", ["cat", "gauss"])
+def test_traced_loss_follows_its_inputs(dev, kind):
+    """torch.jit.trace records the loss as an autograd function of its inputs:
+    called with others, the trace gives their loss and gradients."""
+    if kind == "cat":
+        make = lambda seed: [x.to(dev) for x in cat_inputs(200, 5, seed=seed)[:6]]  # noqa: E731
+        fn, leaf = ppo_amd.ppo_loss_discrete, (0, 5)
+    else:
+        make = lambda seed: [x.to(dev) for x in gauss_inputs(200, 6, seed=seed)[:7]]  # noqa: E731
+        fn, leaf = ppo_amd.ppo_loss_gaussian, (0, 1, 6)
+
+    def leaves(seed):
+        args = make(seed)
+        for k in leaf:
+            args[k].requires_grad_()
+        return args
+
+    print(f"traced loss {kind}", flush=True)
+    traced = torch.jit.trace(lambda *a: fn(*a)[0], tuple(leaves(1)), check_trace=False)
+    for seed in (2, 3):
+        got, want = leaves(seed), leaves(seed)
+        a, b = traced(*got), fn(*want)[0]
+        assert torch.equal(a, b)
+        a.backward()
+        b.backward()
+        for k in leaf:
+            assert torch.equal(got[k].grad, want[k].grad)
+
+
 def test_empty_batches_raise_like_the_reference(dev):
     """A minibatch of no rows: the reference's Categorical / Normal on an
     empty batch raises (torch cannot validate a [0, A] tensor, and the means

@@ -24,6 +24,7 @@
 #include <torch/csrc/autograd/custom_function.h>
 #include <torch/csrc/autograd/graph_task.h>
 #include <torch/csrc/autograd/python_variable.h>
+#include <torch/csrc/jit/frontend/tracer.h>
 #include <torch/csrc/utils/pybind.h>
 
 #include "ppo_amd.h"
@@ -55,9 +56,10 @@ void need(bool ok) {
   if (!ok) throw NotPlain{};
 }
 
-// Modes and transforms that want to see torch operators: not for this path.
+// Modes, transforms and traces that want to see torch operators or autograd
+// functions: not for this path.
 bool plain_mode() {
-  return !at::impl::torch_function_mode_enabled() &&
+  return !torch::jit::tracer::isTracing() && !at::impl::torch_function_mode_enabled() &&
          !c10::impl::TorchDispatchModeTLS::any_modes_set() &&
          !c10::impl::tls_is_dispatch_key_included(
              c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
