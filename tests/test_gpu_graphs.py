@@ -138,3 +138,32 @@ def test_clipped_adam_step_in_graph_replays(dev):
         for a, b in zip(p_got, p_ref):
             torch.testing.assert_close(a.detach(), b.detach(), rtol=2e-6, atol=1e-7)
     assert opt_got.step_count() == 5
+
+
+@pytest.mark.parametrize("validate", [False, True])
+def test_captured_backward_replays_alone(dev, validate):
+    """The losses' backward captured in a graph of its own, replayed several times
+    per forward with other incoming gradients: each replay gives the saved
+    gradients times its own one, bit for bit, with eager work in between."""
+    g = torch.Generator().manual_seed(7)
+    B, A = 3000, 5
+    logits = torch.randn(B, A, generator=g).to(dev).requires_grad_()
+    val = torch.randn(B, generator=g).to(dev).requires_grad_()
+    actions = torch.randint(0, A, (B,), generator=g, dtype=torch.int32).to(dev)
+    rows = [torch.randn(B, generator=g).to(dev) for _ in range(3)]
+    _, dl, dv = ppo_amd.ppo_loss_discrete_fused(logits.detach(), actions, *rows, val.detach())
+    scale = torch.ones((), device=dev)
+    s = torch.cuda.Stream(dev)
+    s.wait_stream(torch.cuda.current_stream(dev))
+    with torch.cuda.stream(s):
+        loss, _ = ppo_amd.ppo_loss_discrete(logits, actions, *rows, val, validate_args=validate)
+    torch.cuda.synchronize(dev)
+    print(f"captured backward validate={validate}", flush=True)
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=s):
+        gl, gv = torch.autograd.grad(loss, (logits, val), grad_outputs=scale)
+    for x in (2.0, -0.5, 1.0, 4.0):
+        scale.fill_(x)
+        graph.replay()
+        torch.cuda.synchronize(dev)
+        assert torch.equal(gl, dl * x) and torch.equal(gv, dv * x), x

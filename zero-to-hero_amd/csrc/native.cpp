@@ -18,6 +18,7 @@
 #include <ATen/SavedTensorHooks.h>
 #include <c10/core/impl/LocalDispatchKeySet.h>
 #include <c10/core/impl/TorchDispatchModeTLS.h>
+#include <c10/hip/HIPGraphsC10Utils.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/Device.h>
 #include <torch/csrc/Generator.h>
@@ -334,7 +335,10 @@ bool plain_scale(const variable_list& grads, const Tensor& scale) {
 }
 
 // grads[k] * scale in one launch, into the tensors themselves (`own`) or new ones.
+// A captured launch always writes new ones: the graph may be replayed more often
+// than the forward that fills the saved ones.
 variable_list scaled(const variable_list& grads, const Tensor& scale, bool own) {
+  own = own && c10::hip::currentStreamCaptureStatusMayInitCtx() == c10::hip::CaptureStatus::None;
   variable_list dst = grads;
   ppo::ScaleArray a[ppo::kMaxScaleArrays];
   for (size_t k = 0; k < grads.size(); ++k) {

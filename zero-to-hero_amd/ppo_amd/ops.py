@@ -748,7 +748,8 @@ def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
     """Backward: every saved gradient times the loss's incoming gradient.
 
     Where the graph is released after this pass (no retain_graph, no
-    create_graph) and nothing else holds the saved gradients, they are scaled
+    create_graph), no HIP graph is being captured (its replays may outnumber
+    the forward's) and nothing else holds the saved gradients, they are scaled
     in place and returned themselves; the launch then touches nothing if the
     incoming gradient is 1, as it is for loss.backward().  Otherwise they are
     scaled into new tensors, and by torch's own operators under create_graph,
