@@ -654,6 +654,32 @@ def test_backward_scales_saved_gradients(dev, B):
     torch.testing.assert_close(gg, dl.sum())
 
 
+@pytest.mark.parametrize("holder", ["none", "object", "tensor"])
+def test_backward_in_place_needs_sole_ownership(dev, holder):
+    """The Python node (validate_args takes it) scales the saved gradients in place
+    only if nobody else holds them, whether by the Python object or by another
+    owner of its tensor."""
+    logits, actions, old_lp, adv, ret, val, _ = (x.to(dev) for x in cat_inputs(100, 5, seed=4))
+    _, dl, dv = ppo_amd.ppo_loss_discrete_fused(logits, actions, old_lp, adv, ret, val)
+    x, v = logits.requires_grad_(), val.requires_grad_()
+    loss = ppo_amd.ppo_loss_discrete(x, actions, old_lp, adv, ret, v, validate_args=True)[0]
+    held = loss.grad_fn.saved_tensors
+    ptrs = [t.data_ptr() for t in held]
+    other = []
+    if holder == "tensor":  # (a graph node of torch's own: no Python reference)
+        other = [(torch.ones_like(t, requires_grad=True) * t) for t in held]
+    if holder != "object":
+        held = None
+    (loss * 4.0).backward()
+    assert torch.equal(x.grad, dl * 4.0) and torch.equal(v.grad, dv * 4.0)
+    assert [x.grad.data_ptr() == ptrs[0], v.grad.data_ptr() == ptrs[1]] == [holder == "none"] * 2
+    if holder == "object":
+        assert torch.equal(held[0], dl) and torch.equal(held[1], dv)
+    for o, want in zip(other, (dl, dv)):
+        (g,) = torch.autograd.grad(o.sum(), o.grad_fn.next_functions[0][0].variable)
+        assert torch.equal(g, want)
+
+
 @pytest.mark.parametrize("validate", [False, True])
 @pytest.mark.parametrize("kind", ["strided", "expanded", "half", "double"])
 def test_backward_of_tensors_that_hooks_replaced(dev, kind, validate):
@@ -717,6 +743,7 @@ def test_backward_of_batched_gradients(dev, validate):
     assert any("mul" in n for n in seen.names)
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning")
 @pytest.mark.parametrize("kind", ["cat", "gauss"])
 def test_traced_loss_follows_its_inputs(dev, kind):
     """torch.jit.trace records the loss as an autograd function of its inputs:

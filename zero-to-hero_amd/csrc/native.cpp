@@ -637,11 +637,36 @@ PyMethodDef kMethods[] = {
     {nullptr, nullptr, 0, nullptr}};
 #undef PPO_ENTRY
 
-// grads[k] * scale in one launch (into the tensors themselves with `own`), or
-// None for tensors that torch's products have to take.
-py::object scale_grads(const variable_list& grads, const Tensor& scale, bool own) {
-  TORCH_CHECK(!grads.empty() && grads.size() <= ppo::kMaxScaleArrays, "scale_grads takes 1 to ",
+// The reference counts of a tensor with one owner in C++ (as a saved variable is)
+// and one reference to its Python object (as the tuple of saved tensors holds),
+// which depend on whether the tensor itself keeps its Python object alive.
+struct SoleOwners {
+  Py_ssize_t object;
+  size_t tensor;
+  SoleOwners() {
+    const Tensor t = at::empty({0}, at::kCPU);
+    const py::object o = py::reinterpret_steal<py::object>(wrap(t));
+    object = Py_REFCNT(o.ptr());
+    tensor = t.use_count();
+  }
+};
+
+// ops._scaled_grads: every tensor of the tuple that ctx.saved_tensors gave times
+// `scale`, in one launch, or None for tensors that torch's products have to take.
+// In place where the graph is released and nobody else holds them (SoleOwners).
+py::object scale_grads(const py::tuple& saved, const Tensor& scale) {
+  TORCH_CHECK(saved.size() > 0 && saved.size() <= ppo::kMaxScaleArrays, "scale_grads takes 1 to ",
               ppo::kMaxScaleArrays, " tensors");
+  static const SoleOwners sole;
+  bool own = !torch::autograd::get_current_graph_task_keep_graph();
+  variable_list grads;
+  for (size_t k = 0; k < saved.size(); ++k) {
+    PyObject* o = PyTuple_GET_ITEM(saved.ptr(), k);
+    if (!THPVariable_CheckExact(o)) return py::none();
+    const Tensor& t = THPVariable_Unpack(o);
+    own = own && Py_REFCNT(o) == sole.object && t.use_count() == sole.tensor;
+    grads.push_back(t);
+  }
   if (!plain_scale(grads, scale)) return py::none();
   return py::cast(scaled(grads, scale, own));
 }

@@ -19,7 +19,6 @@ Reference functions replaced (mrhooray/zero-to-hero, rl/deep/agents/ppo.py):
 from __future__ import annotations
 
 import ctypes
-import sys
 from typing import Optional
 
 import torch
@@ -738,12 +737,6 @@ def _save_grads(ctx, scalars: torch.Tensor, *grads: torch.Tensor):
     return loss, scalars
 
 
-# References to a saved gradient inside _scaled_grads when nothing else holds
-# it: the saved variable, the tuple and the list, the loop variable, getrefcount's
-# argument.
-_SOLE_REFS = 5
-
-
 def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
     """Backward: every saved gradient times the loss's incoming gradient.
 
@@ -761,10 +754,7 @@ def _scaled_grads(ctx, grad_loss: Optional[torch.Tensor]) -> tuple:
         return (None,) * len(saved)
     if torch.is_grad_enabled() or ctx.hooked:
         return tuple(t * grad_loss for t in saved)
-    grads = list(saved)
-    own = (not torch._C._autograd._get_current_graph_task_keep_graph()
-           and all(sys.getrefcount(t) == _SOLE_REFS for t in grads))
-    got = _lib.native().scale_grads(grads, grad_loss, own)
+    got = _lib.native().scale_grads(saved, grad_loss)
     if got is None:
         return tuple(t * grad_loss for t in saved)
     return tuple(got)
