@@ -15,6 +15,7 @@ import pytest
 import torch
 
 import ppo_amd
+from ppo_amd import ops
 from oracle import ppo_oracle as ref
 
 pytestmark = pytest.mark.gpu
@@ -678,6 +679,26 @@ def test_backward_in_place_needs_sole_ownership(dev, holder):
     for o, want in zip(other, (dl, dv)):
         (g,) = torch.autograd.grad(o.sum(), o.grad_fn.next_functions[0][0].variable)
         assert torch.equal(g, want)
+
+
+@pytest.mark.parametrize("kind,leaf", [("cat", 0), ("cat", 5), ("gauss", 0), ("gauss", 1),
+                                       ("gauss", 6)])
+def test_forward_mode_input_is_refused_before_a_second_launch(dev, monkeypatch, kind, leaf):
+    """A differentiable input with a forward-mode tangent: the autograd function's
+    error (it has no jvp), the kernel launched at most once."""
+    import torch.autograd.forward_ad as fwad
+
+    fn = ppo_amd.ppo_loss_discrete if kind == "cat" else ppo_amd.ppo_loss_gaussian
+    args = [x.to(dev) for x in (cat_inputs(64, 5, seed=1)[:6] if kind == "cat"
+                                else gauss_inputs(64, 6, seed=1)[:7])]
+    calls = []
+    get = ops._WORKSPACES.get
+    monkeypatch.setattr(ops._WORKSPACES, "get", lambda *a: calls.append(a) or get(*a))
+    with fwad.dual_level():
+        args[leaf] = fwad.make_dual(args[leaf], torch.ones_like(args[leaf]))
+        with pytest.raises(RuntimeError, match="jvp"):
+            fn(*args)
+    assert len(calls) <= 1
 
 
 @pytest.mark.parametrize("validate", [False, True])

@@ -384,7 +384,6 @@ struct LossNode : public torch::autograd::Function<LossNode> {
 };
 
 PyObject* with_autograd(const Loss& l) {
-  for (const Tensor& t : l.inputs) need(!t._fw_grad(0).defined());
   const Tensor loss = LossNode::apply(at::TensorList(l.inputs), &l);
   py::object stats = loss_stats(l.scalars);
   py::tuple r(2);
@@ -393,8 +392,22 @@ PyObject* with_autograd(const Loss& l) {
   return r.release().ptr();
 }
 
-PyObject* loss_discrete(PyObject* const* a) { return with_autograd(loss_discrete_launch(a)); }
-PyObject* loss_gaussian(PyObject* const* a) { return with_autograd(loss_gaussian_launch(a)); }
+// Forward-mode tangents are for ops' autograd functions (to refuse), before
+// anything is launched.
+void need_no_tangent(PyObject* o) {
+  need(THPVariable_CheckExact(o) && !THPVariable_Unpack(o)._fw_grad(0).defined());
+}
+
+PyObject* loss_discrete(PyObject* const* a) {  // logits, actions, rows...
+  need_no_tangent(a[0]);
+  need_no_tangent(a[5]);
+  return with_autograd(loss_discrete_launch(a));
+}
+
+PyObject* loss_gaussian(PyObject* const* a) {  // mu, log_std, actions, rows...
+  for (int k : {0, 1, 6}) need_no_tangent(a[k]);
+  return with_autograd(loss_gaussian_launch(a));
+}
 
 PyObject* loss_discrete_fused(PyObject* const* a) {
   const Loss l = loss_discrete_launch(a);
