@@ -315,3 +315,16 @@ def test_mlp_act_matches_torch_forward_and_sampler(dev, H, A, act):
     torch.testing.assert_close(lp1.cpu()[clear], lp2.cpu()[clear], rtol=1e-5, atol=1e-5)
     torch.testing.assert_close(v1, v2, rtol=1e-5, atol=1e-5)
     assert torch.equal(obs_out, obs)
+
+
+@pytest.mark.parametrize("size", ["8", 1 << 80])
+def test_layer_sizes_that_are_no_sizes_raise(dev, size):
+    """A Linear whose in_features is no integer, or none that fits 64 bits, gets
+    the Python checks' error."""
+    pol, val = (MLP(8, 64, o, "tanh").to(dev) for o in (4, 1))
+    pol.net[0].in_features = size
+    obs, rows = torch.zeros(16, 8, device=dev), torch.zeros(16, device=dev)
+    with pytest.raises(ValueError, match="not MLPs"):
+        ppo_amd.mlp_act_categorical(pol, val, obs)
+    with pytest.raises(ValueError, match="not MLPs"):
+        ppo_amd.ppo_mlp_cat_grads(pol, val, obs, rows.int(), rows, rows, rows)

@@ -50,7 +50,8 @@ struct Python {
            *weight = nullptr, *bias = nullptr, *in_features = nullptr, *out_features = nullptr;
 } P;
 
-// Thrown for a call that is not the ordinary one.
+// Thrown for a call that is not the ordinary one (entry clears a Python error that
+// a look at its arguments has set).
 struct NotPlain {};
 
 void need(bool ok) {
@@ -102,10 +103,13 @@ const Tensor& plain_rows(PyObject* o, const at::Device& device, int64_t n) {
 double number(PyObject* o) {
   need(PyFloat_CheckExact(o) || PyLong_CheckExact(o));
   const double x = PyFloat_AsDouble(o);
-  if (x == -1.0 && PyErr_Occurred()) {
-    PyErr_Clear();
-    throw NotPlain{};
-  }
+  need(x != -1.0 || !PyErr_Occurred());
+  return x;
+}
+
+int64_t integer(PyObject* o) {
+  const int64_t x = PyLong_AsLongLong(o);
+  need(x != -1 || !PyErr_Occurred());
   return x;
 }
 
@@ -471,8 +475,7 @@ struct Net {
            PyDict_GetItemWithError(d, P.bias) == nullptr);
       w[l] = &plain(item(params, P.weight), at::kFloat);
       b[l] = &plain(item(params, P.bias), at::kFloat);
-      const int64_t i = PyLong_AsLongLong(item(d, P.in_features)),
-                    o = PyLong_AsLongLong(item(d, P.out_features));
+      const int64_t i = integer(item(d, P.in_features)), o = integer(item(d, P.out_features));
       need(w[l]->dim() == 2 && w[l]->size(0) == o && w[l]->size(1) == i && b[l]->dim() == 1 &&
            b[l]->size(0) == o && (l == 0 || dim[l] == i) && b[l]->device() == w[0]->device() &&
            w[l]->device() == w[0]->device());
@@ -626,6 +629,7 @@ PyObject* entry(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     need_plain_mode();
     return kFn(args);
   } catch (const NotPlain&) {
+    PyErr_Clear();
     Py_RETURN_NONE;
   } catch (py::error_already_set& e) {
     e.restore();
