@@ -331,3 +331,46 @@ def test_wait_poller_reports_previous_iteration(dev, giveup):
     poller.flush(dev)
     for a, b in zip(good, again):
         assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("call", ["gae", "act"])
+def test_full_queue_stops_no_other_thread(dev, call):
+    """A thread whose calls fill the hardware queue behind a long kernel waits for
+    room outside the GIL: other Python threads run meanwhile."""
+    import threading
+    import time
+
+    r, v, d, lv = (x.to(dev) for x in _rollout(128, 8, 0.01, 1))
+    pol, val, (obs, *_) = _mlp_case(dev, 32, 5)
+    pol, val, u = pol.to(dev), val.to(dev), torch.rand(32, device=dev)
+    if call == "gae":
+        run = lambda: ops.gae(r, v, d, lv)  # noqa: E731
+    else:
+        run = lambda: ops.mlp_act_categorical(pol, val, obs, u)  # noqa: E731
+    run()
+    torch.cuda.synchronize(dev)
+    t = time.perf_counter()
+    torch.cuda._sleep(50_000_000)
+    torch.cuda.synchronize(dev)
+    cycles = int(50_000_000 * 1.0 / (time.perf_counter() - t))  # about a second
+    longest = [0.0]
+
+    def flood():
+        end = time.perf_counter() + 1.2
+        while (now := time.perf_counter()) < end:
+            run()
+            longest[0] = max(longest[0], time.perf_counter() - now)
+
+    torch.cuda._sleep(cycles)
+    th = threading.Thread(target=flood)
+    th.start()
+    gap, last = 0.0, time.perf_counter()
+    while th.is_alive():
+        time.sleep(0.002)
+        now = time.perf_counter()
+        gap, last = max(gap, now - last), now
+    torch.cuda.synchronize(dev)
+    print(f"full queue {call}: longest call {longest[0]:.3f} s, gap {gap:.3f} s", flush=True)
+    if longest[0] < 0.3:
+        pytest.skip("the queue did not fill")
+    assert gap < 0.5 * longest[0]

@@ -131,6 +131,14 @@ Tensor workspace(const at::Device& device, void* stream, size_t nbytes) {
   return THPVariable_Unpack(r);
 }
 
+// Allocations and the library call, outside the GIL: other Python threads run
+// while this one waits for memory or for room in a full hardware queue.
+template <typename F>
+int unlocked(F f) {
+  py::gil_scoped_release no_gil;
+  return f();
+}
+
 // Raises PPOLibraryError (ops._native_failed) for a non-zero status.
 void check(const char* name, int code, const at::Device& device, void* stream) {
   if (code == PPO_OK) return;
@@ -209,24 +217,31 @@ struct Rollout {
 
 PyObject* gae(PyObject* const* a) {
   const Rollout x(a);
-  const Tensor adv = at::empty(x.r->sizes(), x.r->options()), ret = at::empty_like(adv);
-  check("ppo_gae_f32",
-        ppo_gae_f32(in(*x.r), in(*x.v), x.dones(), x.last(), x.T, x.N, x.gamma, x.lam, out(adv),
-                    out(ret), x.ws.data_ptr(), x.ws.numel(), x.stream),
-        x.r->device(), x.stream);
+  Tensor adv, ret;
+  const int code = unlocked([&] {
+    adv = at::empty(x.r->sizes(), x.r->options());
+    ret = at::empty_like(adv);
+    return ppo_gae_f32(in(*x.r), in(*x.v), x.dones(), x.last(), x.T, x.N, x.gamma, x.lam,
+                       out(adv), out(ret), x.ws.data_ptr(), x.ws.numel(), x.stream);
+  });
+  check("ppo_gae_f32", code, x.r->device(), x.stream);
   return tuple_of({adv, ret});
 }
 
 PyObject* gae_normalize(PyObject* const* a) {  // ..., eps
   const Rollout x(a);
   const double eps = number(a[6]);
-  const Tensor adv = at::empty(x.r->sizes(), x.r->options()), ret = at::empty_like(adv),
-               adv_n = at::empty_like(adv), stats = at::empty({2}, x.r->options());
-  check("ppo_gae_norm_f32",
-        ppo_gae_norm_f32(in(*x.r), in(*x.v), x.dones(), x.last(), x.T, x.N, x.gamma, x.lam, eps,
-                         out(adv), out(ret), out(adv_n), out(stats), x.ws.data_ptr(),
-                         x.ws.numel(), x.stream),
-        x.r->device(), x.stream);
+  Tensor adv, ret, adv_n, stats;
+  const int code = unlocked([&] {
+    adv = at::empty(x.r->sizes(), x.r->options());
+    ret = at::empty_like(adv);
+    adv_n = at::empty_like(adv);
+    stats = at::empty({2}, x.r->options());
+    return ppo_gae_norm_f32(in(*x.r), in(*x.v), x.dones(), x.last(), x.T, x.N, x.gamma, x.lam,
+                            eps, out(adv), out(ret), out(adv_n), out(stats), x.ws.data_ptr(),
+                            x.ws.numel(), x.stream);
+  });
+  check("ppo_gae_norm_f32", code, x.r->device(), x.stream);
   return tuple_of({adv, ret, adv_n, stats});
 }
 
@@ -281,15 +296,16 @@ Loss loss_discrete_launch(PyObject* const* a) {  // logits, actions, rows...
   const Tensor ws = workspace(dev, stream, ppo_loss_cat_workspace_bytes(B, A));
   at::AutoDispatchBelowADInplaceOrView below;
   Loss l;
-  const Tensor dz = at::empty({B, A}, z.options()), dv = at::empty({B}, z.options());
-  l.scalars = at::empty({PPO_NUM_SCALARS}, z.options());
-  check("ppo_loss_cat_f32",
-        ppo_loss_cat_f32(in(z), B, A, act.const_data_ptr(), at_ == at::kLong, in(*r.old_lp),
-                         in(*r.adv), in(*r.ret), in(*r.val), r.old_values(), &r.p, out(dz),
-                         out(dv), out(l.scalars), ws.data_ptr(), ws.numel(), stream),
-        dev, stream);
+  const int code = unlocked([&] {
+    const Tensor dz = at::empty({B, A}, z.options()), dv = at::empty({B}, z.options());
+    l.scalars = at::empty({PPO_NUM_SCALARS}, z.options());
+    l.grads = {dz, dv};
+    return ppo_loss_cat_f32(in(z), B, A, act.const_data_ptr(), at_ == at::kLong, in(*r.old_lp),
+                            in(*r.adv), in(*r.ret), in(*r.val), r.old_values(), &r.p, out(dz),
+                            out(dv), out(l.scalars), ws.data_ptr(), ws.numel(), stream);
+  });
+  check("ppo_loss_cat_f32", code, dev, stream);
   l.inputs = {z, *r.val};
-  l.grads = {dz, dv};
   return l;
 }
 
@@ -307,16 +323,17 @@ Loss loss_gaussian_launch(PyObject* const* a) {  // mu, log_std, actions, rows..
   const Tensor ws = workspace(dev, stream, ppo_loss_gauss_workspace_bytes(B, D));
   at::AutoDispatchBelowADInplaceOrView below;
   Loss l;
-  const Tensor dmu = at::empty({B, D}, mu.options()), dls = at::empty({D}, mu.options()),
-               dv = at::empty({B}, mu.options());
-  l.scalars = at::empty({PPO_NUM_SCALARS}, mu.options());
-  check("ppo_loss_gauss_f32",
-        ppo_loss_gauss_f32(in(mu), in(ls), B, D, in(act), in(*r.old_lp), in(*r.adv), in(*r.ret),
-                           in(*r.val), r.old_values(), &r.p, out(dmu), out(dls), out(dv),
-                           out(l.scalars), ws.data_ptr(), ws.numel(), stream),
-        dev, stream);
+  const int code = unlocked([&] {
+    const Tensor dmu = at::empty({B, D}, mu.options()), dls = at::empty({D}, mu.options()),
+                 dv = at::empty({B}, mu.options());
+    l.scalars = at::empty({PPO_NUM_SCALARS}, mu.options());
+    l.grads = {dmu, dls, dv};
+    return ppo_loss_gauss_f32(in(mu), in(ls), B, D, in(act), in(*r.old_lp), in(*r.adv),
+                              in(*r.ret), in(*r.val), r.old_values(), &r.p, out(dmu), out(dls),
+                              out(dv), out(l.scalars), ws.data_ptr(), ws.numel(), stream);
+  });
+  check("ppo_loss_gauss_f32", code, dev, stream);
   l.inputs = {mu, ls, *r.val};
-  l.grads = {dmu, dls, dv};
   return l;
 }
 
@@ -521,13 +538,16 @@ struct Pair {
   int activation() const { return actor.tanh ? PPO_ACT_TANH : PPO_ACT_RELU; }
 };
 
-// An output argument (or None: allocated).
-Tensor out_or_new(PyObject* o, at::IntArrayRef sizes, at::ScalarType type,
-                  const at::Device& dev) {
-  if (o == Py_None) return at::empty(sizes, at::TensorOptions().dtype(type).device(dev));
+// An output argument (None: undefined, for new_if_none).
+Tensor given(PyObject* o, at::IntArrayRef sizes, at::ScalarType type, const at::Device& dev) {
+  if (o == Py_None) return {};
   const Tensor& t = plain(o, type, dev);
   need(t.sizes() == sizes);
   return t;
+}
+
+void new_if_none(Tensor& t, at::IntArrayRef sizes, at::ScalarType type, const at::Device& dev) {
+  if (!t.defined()) t = at::empty(sizes, at::TensorOptions().dtype(type).device(dev));
 }
 
 // policy, value, observations, uniforms, generator, observations_out,
@@ -545,27 +565,27 @@ PyObject* mlp_act(PyObject* const* a) {
     obs_out = out(t);
   }
   at::AutoDispatchBelowADInplaceOrView below;
-  const Tensor act = out_or_new(a[6], {N}, at::kInt, dev),
-               lp = out_or_new(a[7], {N}, at::kFloat, dev),
-               val = out_or_new(a[8], {N}, at::kFloat, dev);
-  Tensor u;
+  Tensor act = given(a[6], {N}, at::kInt, dev), lp = given(a[7], {N}, at::kFloat, dev),
+         val = given(a[8], {N}, at::kFloat, dev), u;
+  std::optional<at::Generator> gen;
   if (a[3] != Py_None) {
     u = plain_rows(a[3], dev, N);
-  } else {
-    std::optional<at::Generator> gen;
-    if (a[4] != Py_None) {
-      need(THPGenerator_Check(a[4]));
-      gen = THPGenerator_Unwrap(a[4]);
-    }
-    u = at::rand({N}, gen, obs.options());
+  } else if (a[4] != Py_None) {
+    need(THPGenerator_Check(a[4]));
+    gen = THPGenerator_Unwrap(a[4]);
   }
   const ppo_mlp3_f32 pa = nets.actor.pointers(false), pc = nets.critic.pointers(false);
   void* stream = current_stream(dev);
-  check("ppo_mlp_act_cat_f32",
-        ppo_mlp_act_cat_f32(&pa, &pc, (int32_t)nets.actor.D, (int32_t)nets.actor.H,
-                            (int32_t)nets.actor.O, nets.activation(), in(obs), N, in(u), obs_out,
-                            act.data_ptr<int32_t>(), out(lp), out(val), stream),
-        dev, stream);
+  const int code = unlocked([&] {
+    new_if_none(act, {N}, at::kInt, dev);
+    new_if_none(lp, {N}, at::kFloat, dev);
+    new_if_none(val, {N}, at::kFloat, dev);
+    if (!u.defined()) u = at::rand({N}, gen, obs.options());
+    return ppo_mlp_act_cat_f32(&pa, &pc, (int32_t)nets.actor.D, (int32_t)nets.actor.H,
+                               (int32_t)nets.actor.O, nets.activation(), in(obs), N, in(u),
+                               obs_out, act.data_ptr<int32_t>(), out(lp), out(val), stream);
+  });
+  check("ppo_mlp_act_cat_f32", code, dev, stream);
   py::tuple r(3);
   const Tensor* ts[] = {&act, &lp, &val};
   for (int k = 0; k < 3; ++k) {
@@ -603,16 +623,18 @@ PyObject* mlp_grads(PyObject* const* a) {
   need(B > 0);
   const ppo_mlp3_f32 pa = nets.actor.pointers(true), pc = nets.critic.pointers(true);
   at::AutoDispatchBelowADInplaceOrView below;
-  const Tensor scalars = out_or_new(a[13], {PPO_NUM_SCALARS}, at::kFloat, dev);
+  Tensor scalars = given(a[13], {PPO_NUM_SCALARS}, at::kFloat, dev);
   const int32_t D = (int32_t)nets.actor.D, H = (int32_t)nets.actor.H, A = (int32_t)nets.actor.O;
   void* stream = current_stream(dev);
   const Tensor ws = workspace(dev, stream, ppo_mlp_cat_grad_workspace_bytes(B, D, H, A));
-  check("ppo_mlp_cat_grad_f32",
-        ppo_mlp_cat_grad_f32(&pa, &pc, D, H, A, nets.activation(), in(obs), n, idx, B,
-                             act.const_data_ptr(), type == at::kLong, in(old_lp), in(adv),
-                             in(ret), old_val, &p, out(scalars), ws.data_ptr(), ws.numel(),
-                             stream),
-        dev, stream);
+  const int code = unlocked([&] {
+    new_if_none(scalars, {PPO_NUM_SCALARS}, at::kFloat, dev);
+    return ppo_mlp_cat_grad_f32(&pa, &pc, D, H, A, nets.activation(), in(obs), n, idx, B,
+                                act.const_data_ptr(), type == at::kLong, in(old_lp), in(adv),
+                                in(ret), old_val, &p, out(scalars), ws.data_ptr(), ws.numel(),
+                                stream);
+  });
+  check("ppo_mlp_cat_grad_f32", code, dev, stream);
   return loss_stats(scalars).release().ptr();
 }
 
@@ -685,7 +707,11 @@ py::object scale_grads(const py::tuple& saved, const Tensor& scale) {
     grads.push_back(t);
   }
   if (!plain_scale(grads, scale)) return py::none();
-  return py::cast(scaled(grads, scale, own));
+  {
+    py::gil_scoped_release no_gil;
+    grads = scaled(grads, scale, own);
+  }
+  return py::cast(grads);
 }
 
 void init(py::object pool, py::object stats, py::object fail, const std::vector<std::string>& names,
