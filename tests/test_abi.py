@@ -6,6 +6,7 @@ function here launches a kernel."""
 import ctypes
 import os
 import re
+import subprocess
 
 import pytest
 
@@ -108,3 +109,14 @@ def test_host_side_errors_before_launch():
 def test_error_mapping():
     with pytest.raises(_lib.PPOLibraryError, match="workspace"):
         _lib.check("ppo_gae_f32", 2)
+
+
+@pytest.mark.parametrize("out", [None, "_trace.so"])
+def test_make_builds_the_extension_beside_the_library_only(tmp_path, out):
+    """`make OUT=...` (the trace build of bench.py --gae-phases) builds that library
+    alone: the extension links to the library beside it."""
+    cmd = ["make", "-n", "-B", "-C", os.path.join(ROOT, "zero-to-hero_amd", "csrc"),
+           f"OBJDIR={tmp_path}"] + ([] if out is None else [f"OUT={out}"])
+    plan = subprocess.run(cmd, check=True, capture_output=True, text=True).stdout
+    assert ("_native.so" in plan) == (out is None)
+    assert f"-o {out or '../ppo_amd/libppo_amd.so'}" in plan
