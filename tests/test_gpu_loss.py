@@ -344,6 +344,37 @@ def test_cat_masked_logits(dev, A):
     assert (dl[mask] == 0).all()
 
 
+@pytest.mark.parametrize("low", [-float("inf"), float(torch.finfo(torch.float32).min)])
+@pytest.mark.parametrize("offset", [0, 1])
+@pytest.mark.parametrize("A", [2, 3, 4, 8, 18, 20, 23, 33, 64, 100, 300, 1000, 1030])
+def test_cat_masked_logits_of_a_heavy_entropy_term(dev, A, offset, low):
+    """entropy_coef > B: a masked logit's factor in the gradient must not overflow
+    against its probability of 0.  Finite gradients, 0 at the masked logits, and
+    the 64-bit gradient of the unmasked ones."""
+    B, ec = 3, 40.0
+    g = torch.Generator().manual_seed(A)
+    logits = torch.randn(B, A, generator=g)
+    mask = torch.rand(B, A, generator=g) < 0.4
+    mask[:, 0], mask[:, A - 1] = False, True
+    logits = logits.masked_fill(mask, low)
+    act = torch.zeros(B, dtype=torch.int64)
+    old_lp = torch.log_softmax(logits, 1)[:, 0].clone()
+    adv, ret, val = (torch.randn(B, generator=g) for _ in range(3))
+    buf = torch.empty(B * A + offset, device=dev)
+    buf[offset:] = logits.reshape(-1).to(dev)
+    scalars, dl, _ = ppo_amd.ppo_loss_discrete_fused(
+        buf[offset:].view(B, A), act.to(dev), *(x.to(dev) for x in (old_lp, adv, ret, val)),
+        entropy_coef=ec)
+    z = logits.double().masked_fill(mask, 0.0).requires_grad_()
+    lp = torch.log_softmax(z.masked_fill(mask, -1e6), 1)  # (exp(-1e6) is 0)
+    ratio = (lp[:, 0] - old_lp.double()).exp()
+    a64 = adv.double()
+    pol = -torch.min(ratio * a64, ratio.clamp(0.8, 1.2) * a64).mean()
+    (pol + ec * (lp.exp() * lp).sum(1).mean()).backward()
+    assert torch.isfinite(scalars).all() and (dl.cpu()[mask] == 0).all()
+    assert_grad_close(dl, z.grad.float())
+
+
 @pytest.mark.parametrize("scale", [30.0, 100.0])
 @pytest.mark.parametrize("A", [2, 18, 33])
 def test_cat_peaked_logits(dev, A, scale):

@@ -438,7 +438,7 @@ __device__ __forceinline__ ActT row_action_raw(const LossArgs& a, long row) {
 // independently, each with the next tile's loads in flight during the
 // current tile's math.  Each lane reads its row into registers once and
 // evaluates, per logit,
-//     t_j = max(z_j - m, -FLT_MAX),  e_j = exp(t_j),  s += e_j,  S += e_j t_j
+//     t_j = max(z_j - m, kLowestShift),  e_j = exp(t_j),  s += e_j,  S += e_j t_j
 //     dlogit_j = (e_j / s) * (ec/B * t_j + K),  K = ec/B * (H - log s) - g_lp
 // which is the gradient of the LDS-pass form rearranged (log p_j = t_j -
 // log s); the 1[j == a] * g_lp term is added by one LDS read-modify-write per
@@ -734,7 +734,7 @@ __global__ void __launch_bounds__(kBlock) loss_cat_lanes_kernel(LossArgs a, long
           // (a NaN logit, or an infinite one: t = inf - inf, is NaN in e and
           // so in s and in the row's whole gradient)
           float e = __builtin_amdgcn_exp2f(t * kLog2e);
-          const float tc = fmaxf(t, -FLT_MAX);
+          const float tc = fmaxf(t, kLowestShift);
           if constexpr (VW == 1) x[i][c] = tc;
           else x[i][c][k] = tc;
           if constexpr (kRagged) e = col[c] + k >= own[c] ? e : 0.0f;

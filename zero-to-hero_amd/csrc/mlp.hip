@@ -317,7 +317,7 @@ __device__ __forceinline__ RowOut cat_quad_grad(const P& a, float* zr, int A, in
       ta += 16 * c + 4 * q + k == ai ? d : 0.0f;
       // (a NaN logit is NaN in e and so in s and in the row's whole gradient)
       e[c][k] = in_row ? __builtin_amdgcn_exp2f(d * kLog2e) : 0.0f;
-      t[c][k] = fmaxf(d, -FLT_MAX);
+      t[c][k] = fmaxf(d, kLowestShift);
       s += e[c][k];
       S = fmaf(e[c][k], t[c][k], S);
     }

@@ -124,6 +124,12 @@ __device__ __forceinline__ RowOut ppo_row_math(const P& a, const RowIn& in, floa
 // the action index, -1 when outside [0, A) (the log-prob is then NaN).
 // Returns the row's loss terms; H receives the row's entropy.  MINA <= A <=
 // MAXA: only logits from MINA on are tested against A.
+
+// Lowest z_j - m that the row formulas multiply by (masked logits are -inf or the
+// type's lowest value): its exponential is 0 in fp32, as below -104, and its
+// product with ge is finite, so such a logit's gradient is 0.
+constexpr float kLowestShift = -1024.0f;
+
 template <int MAXA, int MINA = 0, typename P>
 __device__ __forceinline__ RowOut cat_row_grad(const P& a, float* zr, int A, int ai, float ge,
                                                const RowIn& in, float& H) {
@@ -143,7 +149,7 @@ __device__ __forceinline__ RowOut cat_row_grad(const P& a, float* zr, int A, int
       // (a NaN logit, or an infinite one: inf - inf, is NaN in e and so in s
       // and in the row's whole gradient; a maximum that keeps it is one
       // instruction, fmaxf beside the exponential of the difference two)
-      const float tj = __builtin_elementwise_maximum(t[j] - m, -FLT_MAX);
+      const float tj = __builtin_elementwise_maximum(t[j] - m, kLowestShift);
       const float ej = __builtin_amdgcn_exp2f(tj * kLog2e);
       t[j] = tj;
       e[j] = ej;
