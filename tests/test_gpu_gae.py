@@ -521,6 +521,8 @@ COLUMN_SHAPES = [
     (1, 1), (1, 5), (3, 4), (127, 8), (128, 17), (256, 16), (257, 33), (512, 16), (513, 16),
     (1000, 8), (1024, 9), (1000, 255), (1000, 257), (1025, 64), (2048, 3), (2047, 65), (2048, 2047),
     (2049, 7), (255, 4096), (60, 4097), (200, 8192), (16, 8192), (500, 4100),
+    # workgroup counts of every remainder by the 8 XCDs
+    (300, 2049), (300, 2057), (300, 2065), (300, 2073), (300, 2081), (300, 2089), (300, 2097),
 ]
 
 
