@@ -56,10 +56,9 @@ const char* ppo_amd_strerror(int code);
 
 /*
  * Status of the bounded in-kernel waits (no counterpart in the reference: its
- * update runs on the CPU in one thread).  Five launches hold workgroups that
+ * update runs on the CPU in one thread).  Four launches hold workgroups that
  * wait for one another inside the launch: the resident GAE pass
- * (ppo_gae_f32 / ppo_gae_norm_f32, PPO_GAE_ROUTE_RESIDENT), the column GAE
- * pass with the normaliser (PPO_GAE_ROUTE_COLUMN), the Gaussian loss
+ * (ppo_gae_f32 / ppo_gae_norm_f32, PPO_GAE_ROUTE_RESIDENT), the Gaussian loss
  * with its in-kernel finish (ppo_loss_gauss_f32), the categorical loss, which
  * also finishes in-kernel (ppo_loss_cat_f32 and its _noalloc form: every batch
  * on the wave-tile kernels, whose workgroup 0 only collects, batches of at
@@ -171,16 +170,15 @@ int ppo_gae_norm_f32(const float* rewards, const float* values,
  * a T x N rollout with 16-byte-aligned buffers on the current device, as one
  * of the PPO_GAE_ROUTE_* values (diagnostics and tests; no counterpart in the
  * reference).  has_values = 0 means values == NULL.  Misaligned buffers take
- * the scalar tile passes whatever this returns.  The environment variable
- * PPO_AMD_GAE_RESIDENT=0 turns off the resident pass and the column pass
- * wherever its workgroups exchange statistics.
+ * the column pass where T and N allow it, else the scalar tile passes.  The environment variable PPO_AMD_GAE_RESIDENT=0 turns the
+ * resident pass off.
  */
 #define PPO_GAE_ROUTE_NONE 0      /* empty or oversized rollout                */
 #define PPO_GAE_ROUTE_RESIDENT 1  /* one launch, whole rollout in registers    */
 #define PPO_GAE_ROUTE_STRIP 2     /* strip walk (+ normalise pass)             */
 #define PPO_GAE_ROUTE_SPAN 3      /* span passes + carry scan (+ normalise)    */
 #define PPO_GAE_ROUTE_TILES 4     /* tile passes + carry scan                  */
-#define PPO_GAE_ROUTE_COLUMN 5    /* one launch, a workgroup per few envs      */
+#define PPO_GAE_ROUTE_COLUMN 5    /* a workgroup per few envs (+ normalise)    */
 int ppo_gae_route(int64_t T, int64_t N, int normalize, int has_values);
 
 /* ------------------------------------------------------------------------ */

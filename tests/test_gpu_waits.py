@@ -97,36 +97,33 @@ def test_gae_resident_giveup_writes_nan_and_reports(dev, giveup, T, N, norm, gam
         assert np.array_equal(again[0].cpu().numpy(), adv_ref.astype(np.float32))
 
 
-@pytest.mark.parametrize("T,N", [(1000, 64), (200, 4000)])
-def test_gae_column_giveup_writes_nan_and_reports(dev, giveup, monkeypatch, T, N):
-    """The column pass's exchange of statistics; PPO_AMD_GAE_RESIDENT=0 keeps
-    to passes that wait for nothing."""
+@pytest.mark.parametrize("T,N", [(128, 64), (1000, 64), (1000, 1023), (200, 4000), (2048, 128),
+                                 (8192, 16), (4096, 64)])
+def test_gae_short_rollouts_wait_for_nothing(dev, giveup, T, N):
+    """Rollouts of fewer than 128 resident tiles take passes whose workgroups
+    do not wait for one another, with the normaliser too: the poll limit of
+    zero changes nothing."""
     lib = _lib.load()
-    assert _lib.GAE_ROUTES[lib.ppo_gae_route(T, N, 1, 1)] == "column"
-    print(f"waits gae column T={T} N={N}", flush=True)
+    print(f"waits gae short T={T} N={N}", flush=True)
+    for norm in (1, 0):
+        assert _lib.GAE_ROUTES[lib.ppo_gae_route(T, N, norm, 1)] != "resident"
     r, v, d, lv = (x.to(dev) for x in _rollout(T, N, 0.01, 5))
-    run = lambda: ops.gae_normalize(r, v, d, lv, 0.99, 0.95)  # noqa: E731
+    run = lambda: (*ops.gae(r, v, d, lv, 0.99, 0.95),  # noqa: E731
+                   *ops.gae_normalize(r, v, d, lv, 0.99, 0.95))
     good = [x.clone() for x in run()]
-    ops.check_waits(dev)
-    with giveup:
-        bad = run()
-        torch.cuda.synchronize(dev)
-    for x in bad:
-        assert bool(torch.isnan(x).all())
-    _expect_timeout(dev)
-    for a, b in zip(good, run()):
-        assert torch.equal(a, b)
-    ops.check_waits(dev)
-    monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
-    assert _lib.GAE_ROUTES[lib.ppo_gae_route(T, N, 1, 1)] in ("strip", "span", "tiles")
     with giveup:
         other = run()
         torch.cuda.synchronize(dev)
     ops.check_waits(dev)
-    # (the passes compose a segment's carry in different orders in fp64: at most
-    # one fp32 ulp, 2^-23, after rounding)
-    torch.testing.assert_close(other[0], good[0], rtol=2.0 ** -23, atol=1e-9)
-    torch.testing.assert_close(other[2], good[2], rtol=1e-5, atol=1e-6)
+    for a, b in zip(good, other):
+        assert torch.equal(a, b)
+    adv_ref, _ = ref.gae_numpy(r.cpu().numpy(), v.cpu().numpy(), d.cpu().numpy(),
+                               lv.cpu().numpy(), 0.99, 0.95)
+    adv_ref = torch.from_numpy(adv_ref.astype(np.float32))
+    # (carries are composed in another fp64 order: at most one fp32 ulp, 2^-23)
+    torch.testing.assert_close(good[0].cpu(), adv_ref, rtol=2.0 ** -23, atol=1e-9)
+    n_ref = ref.normalize_reference(adv_ref.reshape(-1)).reshape(T, N)
+    torch.testing.assert_close(good[4].cpu(), n_ref, rtol=1e-5, atol=1e-6)
 
 
 def _gauss(dev, B, D, seed):

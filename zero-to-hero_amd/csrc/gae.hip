@@ -287,22 +287,20 @@ struct ResPlan {
 // measured 38.2-38.5 us per call in the north-star step against 39.1-39.3 us
 // for 64-env tiles; 256-env tiles were slower, their look-back folding 15
 // tiles per column, so 128-env tiles are taken only up to 8 tiles per column).  Rollouts that
-// give fewer than `min_tiles` tiles, or more than 16 tiles per env column
+// give fewer than kResMinTiles tiles, or more than 16 tiles per env column
 // without filling the device, take the other paths: measured on MI355X, 2048 x
 // 4096 runs 45 us against 55 us, 4096 x 2048 45 us against 72 and 32768 x 256 (64
-// tiles per column, 256 tiles) 57 us against 67.  From 128 tiles on the resident
-// pass comes first; with fewer (kResFewTiles) it follows the column pass, where
-// that declines or is slower (gae_route): 2048 x 256 with the normaliser
-// 13.3 us against 15.4 of columns and 19.4 of the span passes, 8192 x 16 13.2
-// against 18.4.
+// tiles per column, 256 tiles) 57 us against 67.  (Fewer tiles would gain as
+// well, 8192 x 16 with the normaliser 12.6 us against 17.7 of the span passes, but
+// would make small rollouts wait for a whole grid to be resident.)
 // Without the normaliser, rollouts too long for one round (more than 256
 // tiles of 16 steps per thread) run in rounds of 256 tiles, from the end of
 // the horizon backwards (at most kResMaxRounds), each round handing the
 // advantage at its left edge to the next.
 constexpr long kResMaxRounds = 8;
-constexpr long kResManyTiles = 128, kResFewTiles = 2;
+constexpr long kResMinTiles = 128;
 
-ResPlan res_plan(long T, long N, bool norm, long min_tiles) {
+ResPlan res_plan(long T, long N, bool norm) {
   ResPlan best = {0, 0, 0, 0, 0, 0, 0};
   if (!PPO_GAE_RES || T <= 0 || N <= 0 || T * N >= (1L << 30)) return best;
   const int Es[4] = {128, 64, 32, 16};
@@ -329,7 +327,7 @@ ResPlan res_plan(long T, long N, bool norm, long min_tiles) {
       }
     }
   }
-  if (best.E && (best.tiles() < min_tiles || (best.nt > 16 && best.tiles() < kResMaxTiles)))
+  if (best.E && (best.tiles() < kResMinTiles || (best.nt > 16 && best.tiles() < kResMaxTiles)))
     best.E = 0;
   if (best.E || norm) return best;
   // rounds: the widest tile of at most 64 envs dividing N, 16 steps per thread
@@ -366,19 +364,21 @@ struct ColPlan {
 
 // A workgroup touches every row of the horizon once per array whatever E is (16,
 // 32 or 64 bytes of it), so its time grows with T: taken to T = 2048 (2048 x 64
-// with the normaliser 12 us, 4096 x 64 28 us against 19 of the span passes).
-// Narrow columns give more workgroups, wide ones longer row pieces: 16 envs to
-// 256 steps, then 4, or 8 where 4 would give more than 64 workgroups (1000 x 64
-// 10.2 against 11.6 us, 1000 x 1023 17.2 against 16.5; 2048 x 2047 without the
-// normaliser 31 against 21).  A rollout that one workgroup holds needs no exchange
-// (512 x 16 with the normaliser 7.9 us with 16 envs, 9.6 with 8).  The exchange
-// needs the grid resident at once (256 workgroups).  Where the tile or strip
-// passes have enough rows in flight they win: past 512 columns (512 x 20001 without
-// the normaliser 124 us against 76), with most threads idle (16 x 30000 13 against
-// 7), and past 1024 steps of more than 64 envs (2000 x 129 20.0 against 18.1, 1500 x
-// 257 19.7 against 18.4, 2048 x 1300 without the normaliser 28 against 25) unless
-// the normaliser's extra passes (2048 x 700 22 against 60) or an N that no vector
-// width divides (2048 x 2047 21 against 36) cost them more.
+// with the normaliser 12.8 us against 17.7 of the span passes; a workgroup holds
+// no more).  Narrow columns give more workgroups, wide ones longer row pieces: 16
+// envs to 256 steps, then 4, or 8 where 4 would give more than 64 workgroups (with
+// the normaliser, 4 and 8: 1000 x 64 10.5 and 11.2 us, 2048 x 700 30.0 and 21.3, 1000
+// x 1023 15.6 and 14.4).  A rollout that one workgroup holds needs no second launch
+// (512 x 16 with the normaliser 7.2 us with 16 envs, 8.5 with 8).  With the
+// normaliser more than 256 workgroups take the next width (1000 x 2049 19 us).
+// Where the tile or strip passes have enough rows in flight they win: past 512
+// columns (512 x 20001 without the normaliser 124 us against 76), with most threads
+// idle (16 x 30000 13 against 7), and without the normaliser past 1024 steps of
+// more than 64 envs (1500 x 769 14.8, 2048 x 1300 23.7) up to the width where no
+// vector access helps them (1100 x 1025 14.5 against 10.1 of columns, 2000 x 1793
+// 31.8 against 19.9).  With the normaliser their extra passes cost them more
+// (2048 x 128 18.3 against 13.3, 1200 x 256 18.7 and 12.4, 1100 x 641 18.4 and 15.4,
+// 2000 x 769 22.4 and 22.3, 2048 x 700 60 and 21).
 ColPlan col_plan(long T, long N, bool norm) {
   const ColPlan none = {0, 0, 0};
   if (T <= 0 || N <= 0 || T > 2048 || T * N >= (1L << 30)) return none;
@@ -394,8 +394,7 @@ ColPlan col_plan(long T, long N, bool norm) {
   }
   const long wgs = (N + E - 1) / E, per = steps(E);
   if (wgs > 2 * kResMaxTiles || (wgs > kResMaxTiles && T * E < kColBlock)) return none;
-  if (T > 1024 && N > 64 && (norm ? N < (N % 4 ? 768 : 384) : N <= 1024 || N % 4 == 0))
-    return none;
+  if (!norm && T > 1024 && N > 64 && (N <= 1024 || N % 4 == 0)) return none;
   return {E, per <= 2 ? 2 : (per <= 4 ? 4 : (per <= 8 ? 8 : 16)), wgs};
 }
 
@@ -407,21 +406,13 @@ constexpr size_t kResSlotBase = kSyncWords;
 // per workgroup: n, sum and sum of squares of its advantages, and the centred
 // sum of squares of the exact second pass (gae_resident_kernel, step 4)
 constexpr size_t kResPartWords = 4;
-// column pass of up to kColTagged workgroups, per workgroup: n, sum and sum of
-// squares as tagged words
-constexpr long kColTagged = 64;
-constexpr size_t kColPartWords = 6;
 size_t res_slot_words(const ResPlan& rp) {
   if (!rp.E) return 0;
   return kResSlotBase + (size_t)rp.tiles() * 2 * rp.E + (size_t)rp.rounds * rp.nc * rp.E +
          (size_t)rp.grid() * kResPartWords;
 }
 size_t res_slot_words_max(long T, long N) {
-  const ColPlan cp = col_plan(T, N, true);
-  return std::max({res_slot_words(res_plan(T, N, true, kResFewTiles)),
-                   res_slot_words(res_plan(T, N, false, kResFewTiles)),
-                   cp.wgs <= kColTagged ? (size_t)cp.wgs * kColPartWords
-                                        : kResSlotBase + (size_t)cp.wgs * kResPartWords});
+  return std::max(res_slot_words(res_plan(T, N, true)), res_slot_words(res_plan(T, N, false)));
 }
 
 struct GaeLayout {
@@ -447,7 +438,9 @@ GaeLayout make_layout(const GaePlan& p, long N) {
     const CarryPlan cp = make_carry_plan(p.Tt, N);
     const SpanPlan sp = span_plan(p.T, N, kSpanMaxBlocks);
     const long parts = std::max<long>(std::max<long>(p.blocks(), cp.groups * cp.nchunks),
-                                      std::max<long>(strip_plan(p).strips, sp.nstrips * sp.spans));
+                                      std::max<long>(std::max<long>(strip_plan(p).strips,
+                                                                    sp.nstrips * sp.spans),
+                                                     col_plan(p.T, N, true).wgs));
     off += align_up((size_t)parts * 4 * sizeof(double), 256);
   }
   l.slots = off;
@@ -2202,13 +2195,12 @@ const void* res_kernel(const ResPlan& rp, bool stats, bool has_v) {
   return res_kernel_e<16>(rp.L, stats, has_v, rounds);
 }
 
-// The environment variable PPO_AMD_GAE_RESIDENT=0 turns the resident pass
-// off (every rollout then takes the strip walk, span or tile passes), so that
-// those paths can be tested on shapes the resident pass would take.
-bool resident_ok(long T, long N, bool norm, bool has_v, long min_tiles) {
+// The environment variable PPO_AMD_GAE_RESIDENT=0 turns the resident pass off
+// (the other passes wait for no other workgroup).
+bool resident_ok(long T, long N, bool norm, bool has_v) {
   const char* env = getenv("PPO_AMD_GAE_RESIDENT");
   if (env && env[0] == '0') return false;
-  const ResPlan rp = res_plan(T, N, norm, min_tiles);
+  const ResPlan rp = res_plan(T, N, norm);
   if (rp.E == 0) return false;
   const void* kern = res_kernel(rp, norm, has_v);
   return kern && resident_blocks(kern, kResBlock, 0, 0) >= rp.grid();
@@ -2216,7 +2208,7 @@ bool resident_ok(long T, long N, bool norm, bool has_v, long min_tiles) {
 
 // Launches the resident pass (resident_ok).
 int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
-  const ResPlan rp = res_plan(T, N, norm, kResFewTiles);
+  const ResPlan rp = res_plan(T, N, norm);
   const void* kern = res_kernel(rp, norm, a.v != nullptr);
   a.res_nc = rp.nc;
   a.res_nt = rp.nt;
@@ -2231,20 +2223,24 @@ int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
 }
 
 // ---------------------------------------------------------------------------
-// Column pass: one launch for rollouts whose horizon fits one workgroup.  A
-// 1024-thread workgroup owns E envs for the whole horizon (1024 / E segments of L
-// steps, one env per thread, rows in registers from load to store, any N and
-// any alignment), so no carry crosses workgroups; with the normaliser the
-// workgroups exchange only their fp64 (n, sum, sum of squares) through the
-// words of grid_sync.hpp (a single workgroup exchanges nothing) and write the
-// normalised advantages from the registers.
+// Column pass, for rollouts whose horizon fits one workgroup.  A 1024-thread
+// workgroup owns E envs for the whole horizon (1024 / E segments of L steps, one
+// env per thread, rows in registers from load to store, any N and any alignment),
+// so no carry crosses workgroups and none waits for another.  With the normaliser
+// a single workgroup normalises from its registers; several leave their fp64 (n,
+// sum, sum of squares) to the elementwise normaliser, which reads the advantages
+// back out of the caches.  (An exchange of the sums inside the launch saves that
+// second launch, 0 to 1.4 us -- 128 x 64 6.8 us, 1000 x 1023 14.0, 2048 x 2047 28.2 --
+// but needs the whole grid resident at once and gives up where another stream's
+// waiting grid holds the chip.)
 //
-// What bounds it: latency -- one round of loads, the scan, the exchange, the
-// stores.  Measured on MI355X against the 3 or 4 launches of the span and tile
-// passes (T x N, us of device time per call, with / without the normaliser):
-//   128 x 8      15.0 -> 5.3 / 5.9 -> 3.6      1000 x 64    18.2 -> 10.3 / 11.6 -> 5.6
-//   1000 x 1023  21.4 -> 16.4 / 16.2 -> 10.8   2048 x 64    18.4 -> 12.4 / 11.4 -> 8.0
-//   200 x 2048   19.2 -> 10.3 / 14.4 -> 4.9    2048 x 2047  45.5 -> 30.2 / 36.0 -> 21.4
+// What bounds it: latency -- one round of loads, the scan, the stores, and with
+// the normaliser a second launch.  Measured on MI355X against the 1 to 4 launches
+// of the span and tile passes (T x N, us of device time per call, with / without the
+// normaliser):
+//   128 x 8      14.2 -> 4.6 / 5.9 -> 3.6      1000 x 64    17.6 -> 10.5 / 11.6 -> 5.6
+//   1000 x 1023  18.7 -> 14.4 / 13.3 -> 8.1    2048 x 64    17.7 -> 12.8 / 11.0 -> 7.4
+//   200 x 2048   18.7 -> 10.6 / 13.7 -> 4.3    2048 x 2047  45.1 -> 27.7 / 36.0 -> 20.0
 // ---------------------------------------------------------------------------
 constexpr int kColWaves = kColBlock / kWave;
 
@@ -2253,7 +2249,6 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
   constexpr int SW = kWave / E;  // segments per wave
   __shared__ double2 s_wc[kColWaves][E];
   __shared__ float s_norm[2];
-  __shared__ CallTag s_tag;
   const int tid = threadIdx.x;
   const int lane = tid % kWave, w = tid / kWave, j = lane / E, e = tid % E;
   // Neighbouring columns, which share cache lines, on one XCD: workgroup b runs on
@@ -2265,20 +2260,6 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
   const long xcd = blockIdx.x % kXcds, rest = nwg % kXcds;
   const long col = xcd * (nwg / kXcds) + (xcd < rest ? xcd : rest) + blockIdx.x / kXcds;
   const bool multi = kStats && nwg > 1;
-  // up to kColTagged workgroups exchange tagged words, more of them slots behind
-  // a start barrier (us of device time, tagged and slots: 128 x 64, 4 workgroups,
-  // 7.2 and 8.6; 2048 x 64, 16 workgroups, 12.4 and 13.1; 1000 x 1023, 128
-  // workgroups, 17.7 and 16.5)
-  const bool tagged = nwg <= kColTagged;
-  uint64_t* part = a.slots + kResSlotBase;  // (slots) [grid][kResPartWords]
-  int fail = 0;
-  uint64_t epoch = 0;  // (thread 0)
-  unsigned nonce = 0;  // (thread 0) the start barrier's tag
-  if (multi && tagged && tid == 0) s_tag = call_tag(&a.hdr->epoch, a.nonce, epoch);
-  if (multi && !tagged && w == 0) {
-    nonce = launch_tag(&a.hdr->epoch, a.nonce, epoch);
-    sync_start(a.slots, part + (size_t)blockIdx.x * kResPartWords, (int)kResPartWords, nonce);
-  }
   const long env = col * E + e;
   const long T = a.T;
   const unsigned n32 = (unsigned)a.N, env32 = (unsigned)(env < a.N ? env : a.N - 1);
@@ -2360,7 +2341,7 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
         nvd = vd;
         r[i] = (float)x;  // the advantage replaces the reward
         const unsigned off = row(t0 + i);
-        if (!kStats || a.adv != a.adv_n) a.adv[off] = r[i];
+        if (!kStats || multi || a.adv != a.adv_n) a.adv[off] = r[i];
         if (a.ret) a.ret[off] = r[i] + v[i];
         if constexpr (kStats) {
           const double xf = r[i];
@@ -2373,47 +2354,24 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
   if constexpr (kStats) {
     block_sum_lds<3>(acc);
     if (multi) {
-      // (every workgroup reads all partials in one order: the same bits in each)
-      if (tagged) {
-        const CallTag tag = s_tag;
-        if (tid == 0) {
-          uint64_t* pp = a.slots + (size_t)blockIdx.x * kColPartWords;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) tagged_put(pp + 2 * k, acc[k], tag);
-        }
-        acc[0] = acc[1] = acc[2] = 0.0;
-        if (tid < nwg)
-          tagged_get<3>(a.slots + (size_t)tid * kColPartWords, tag, a.wc.spin, fail, acc);
-      } else {
-        if (tid == 0) {
-          uint64_t* pp = part + (size_t)blockIdx.x * kResPartWords;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) slot_put(pp + k, acc[k]);
-          if (!res_wait(a.slots, nonce, gridDim.x, a.wc.spin)) fail = 1;
-        }
-        lds_barrier();
-        acc[0] = acc[1] = acc[2] = 0.0;
-        if (tid < nwg) {
-          uint64_t* pp = part + (size_t)tid * kResPartWords;
-#pragma unroll
-          for (int k = 0; k < 3; ++k) acc[k] = slot_get(pp + k, a.wc.spin, fail);
-        }
+      if (tid == 0) {
+        double* pp = a.partial + 4 * (long)blockIdx.x;
+        pp[0] = acc[0];
+        pp[1] = acc[1];
+        pp[2] = acc[2];
       }
-      block_sum_lds<3>(acc);
-      if (blockIdx.x == 0 && tid == 0) epoch_advance(&a.hdr->epoch, epoch);
+      return;
     }
     if (tid == 0) {
       const NormParams np_ = norm_params_of(acc, a.eps);
       s_norm[0] = np_.mean_used;
       s_norm[1] = np_.denom;
-      if (blockIdx.x == 0) {
-        a.hdr->stats[0] = np_.mean_used;
-        a.hdr->stats[1] = np_.std;
-        a.hdr->stats[2] = np_.denom;
-        if (a.stats_out) {
-          a.stats_out[0] = np_.mean;
-          a.stats_out[1] = np_.std;
-        }
+      a.hdr->stats[0] = np_.mean_used;
+      a.hdr->stats[1] = np_.std;
+      a.hdr->stats[2] = np_.denom;
+      if (a.stats_out) {
+        a.stats_out[0] = np_.mean;
+        a.stats_out[1] = np_.std;
       }
     }
     lds_barrier();
@@ -2422,17 +2380,6 @@ __global__ void __launch_bounds__(kColBlock) gae_column_kernel(GaeArgs a) {
     for (int i = 0; i < L; ++i) {
       asm volatile("" : "+v"(r[i]));  // (as above: the rows' fp64 copies)
       if (i < nvalid) a.adv_n[row(t0 + i)] = (r[i] - mean) / denom;
-    }
-    // A wait that gave up (grid not co-resident): NaN over everything this
-    // workgroup wrote, and the device's wait-status word.
-    if (multi && __syncthreads_or(fail)) {
-      if (tid == 0) wait_report(a.wc.status);
-      const float qnan = __builtin_nanf("");
-      for (int i = 0; i < nvalid; ++i) {
-        a.adv[row(t0 + i)] = qnan;
-        if (a.ret) a.ret[row(t0 + i)] = qnan;
-        a.adv_n[row(t0 + i)] = qnan;
-      }
     }
   }
 }
@@ -2454,28 +2401,15 @@ const void* column_kernel(const ColPlan& cp, bool stats, bool has_v) {
   return column_kernel_e<4>(cp.L, stats, has_v);
 }
 
-// Whether a column pass runs here: the normaliser's exchange needs the whole
-// grid resident at once (and no PPO_AMD_GAE_RESIDENT=0, which asks for passes
-// that wait for nothing).
-bool column_ok(long T, long N, bool norm, bool has_v) {
-  const ColPlan cp = col_plan(T, N, norm);
-  if (!cp.E) return false;
-  if (!norm || cp.wgs == 1) return true;
-  const char* env = getenv("PPO_AMD_GAE_RESIDENT");
-  if (env && env[0] == '0') return false;
-  return resident_blocks(column_kernel(cp, norm, has_v), kColBlock, 0, 0) >= cp.wgs;
-}
-
 int launch_column(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
   const ColPlan cp = col_plan(T, N, norm);
-  if (norm && cp.wgs > 1) {
-    a.nonce = next_nonce();
-    const int st = wait_ctl(a.wc);
-    if (st) return st;
-  }
   void* args[] = {&a};
-  return hip_status(hipLaunchKernel(column_kernel(cp, norm, a.v != nullptr),
-                                    dim3((unsigned)cp.wgs), dim3(kColBlock), args, 0, stream));
+  const int st = hip_status(hipLaunchKernel(column_kernel(cp, norm, a.v != nullptr),
+                                            dim3((unsigned)cp.wgs), dim3(kColBlock), args, 0,
+                                            stream));
+  if (st || !norm || cp.wgs == 1) return st;
+  return launch_normalize(a.partial, cp.wgs, a.eps, a.adv, a.adv_n, T * N, a.hdr, a.stats_out,
+                          stream);
 }
 
 // Pass kernels by (VW, L, solo) geometry.
@@ -2591,13 +2525,8 @@ bool span_route(long T, long N, bool norm) {
 int gae_route(long T, long N, bool norm, bool has_v, bool vec, bool all_vec) {
   // aligned rollouts of many tiles that all fit on the device at once: one
   // read of the rollout, one write of each output
-  if (all_vec && resident_ok(T, N, norm, has_v, kResManyTiles)) return PPO_GAE_ROUTE_RESIDENT;
-  const bool column = column_ok(T, N, norm, has_v);
-  // fewer tiles: long horizons, or many columns of a horizon past 1024
-  if (all_vec && (!column || (T > 1024 && N > 64)) &&
-      resident_ok(T, N, norm, has_v, kResFewTiles))
-    return PPO_GAE_ROUTE_RESIDENT;
-  if (column) return PPO_GAE_ROUTE_COLUMN;
+  if (all_vec && resident_ok(T, N, norm, has_v)) return PPO_GAE_ROUTE_RESIDENT;
+  if (col_plan(T, N, norm).E) return PPO_GAE_ROUTE_COLUMN;
   if (vec && span_route(T, N, norm)) return PPO_GAE_ROUTE_SPAN;
   const GaePlan p = make_plan(T, N, vec && !narrow_scalar(T, N, norm) ? 4 : 1);
   return strip_plan(p).E > 0 ? PPO_GAE_ROUTE_STRIP : PPO_GAE_ROUTE_TILES;

@@ -148,8 +148,8 @@ def check_waits(device: Optional[torch.device] = None) -> None:
     """Synchronises torch's current stream on `device` (default: the current
     device) and raises PPOLibraryError with code PPO_ERR_WAIT_TIMEOUT if a
     bounded in-kernel wait on that device gave up since the last check (on
-    any stream).  The launches with such waits (the resident and the
-    column GAE pass, the losses' in-kernel finish, the fused clip + Adam of
+    any stream).  The launches with such waits (the resident GAE
+    pass, the losses' in-kernel finish, the fused clip + Adam of
     ppo_mlp_cat_step) assume their whole grid runs at once; when another
     process or stream on the GPU prevents that, the affected outputs are NaN
     or the affected parameters unwritten, and this check reports it (and

@@ -146,8 +146,8 @@ class VecPPO:
     The results equal the eager fused path's: the same kernels run on the
     same data.
 
-    `check_waits` reports in-kernel waits that gave up (GAE resident and
-    column passes, the losses' in-kernel finish, fused clip + Adam) as PPOLibraryError
+    `check_waits` reports in-kernel waits that gave up (GAE resident pass,
+    the losses' in-kernel finish, fused clip + Adam) as PPOLibraryError
     (PPO_ERR_WAIT_TIMEOUT): "deferred" (default, also True) checks each
     update's status at the end of the next update (ops.WaitPoller: no
     synchronisation per update) and `flush_waits()` checks at once; "sync"
