@@ -170,8 +170,8 @@ int ppo_gae_norm_f32(const float* rewards, const float* values,
  * a T x N rollout with 16-byte-aligned buffers on the current device, as one
  * of the PPO_GAE_ROUTE_* values (diagnostics and tests; no counterpart in the
  * reference).  has_values = 0 means values == NULL.  Misaligned buffers take
- * the column pass where T and N allow it, else the scalar tile passes.  The environment variable PPO_AMD_GAE_RESIDENT=0 turns the
- * resident pass off.
+ * the column pass where T and N allow it, else the scalar tile passes.  The environment variables PPO_AMD_GAE_RESIDENT=0 and
+ * PPO_AMD_GAE_COLUMN=0 turn the resident and the column pass off.
  */
 #define PPO_GAE_ROUTE_NONE 0      /* empty or oversized rollout                */
 #define PPO_GAE_ROUTE_RESIDENT 1  /* one launch, whole rollout in registers    */

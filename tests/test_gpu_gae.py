@@ -29,11 +29,23 @@ def _c_oracle():
     ref.build_c()
 
 
+def _other_passes(monkeypatch):
+    """Turns the resident and the column pass off, so shapes that these would
+    take run on the strip walk / span / tile passes they are chosen to
+    exercise."""
+    monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
+    monkeypatch.setenv("PPO_AMD_GAE_COLUMN", "0")
+
+
 @pytest.fixture
 def no_resident(monkeypatch):
-    """Turns the resident pass off, so shapes it would take run on the strip
-    walk / span / tile passes they are chosen to exercise."""
-    monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
+    _other_passes(monkeypatch)
+
+
+def _route(T, N, norm, has_values=True):
+    from ppo_amd import _lib
+
+    return _lib.GAE_ROUTES[_lib.load().ppo_gae_route(T, N, int(norm), int(has_values))]
 
 
 def _inputs(T, N, p_done, seed, last=True):
@@ -121,9 +133,13 @@ def test_gae_without_bootstrap(dev):
     _run(dev, 1000, 12, 0.01, seed=4, last=False)
 
 
-def test_gae_misaligned_buffers(dev):
+@pytest.mark.parametrize("column", [True, False])
+def test_gae_misaligned_buffers(dev, monkeypatch, column):
     """Views that start one element into an allocation are not 16-byte
-    aligned: the kernel must take its scalar path and still agree."""
+    aligned: the kernel must take its scalar path (or the column pass, which
+    has no other) and still agree."""
+    if not column:
+        _other_passes(monkeypatch)
     T, N = 300, 8
     r, v, d, lv = _inputs(T, N, 0.05, seed=9)
     rb = torch.empty(T * N + 1, device=dev)
@@ -291,15 +307,18 @@ def test_discounted_returns_vectorised_with_dones(dev):
     ],
 )
 def test_gae_strip_walk_matches_oracle(no_resident, dev, T, N, p):
+    assert _route(T, N, False) == ("strip" if T > 100 else "tiles")
     exact = _run(dev, T, N, p, seed=T * 31 + N)
     assert exact > 0.99
 
 
 def test_gae_strip_walk_without_bootstrap(no_resident, dev):
+    assert _route(700, 4096, False) == "strip"
     _run(dev, 700, 4096, 0.01, seed=41, last=False)
 
 
 def test_gae_strip_walk_all_or_no_dones(no_resident, dev):
+    assert _route(300, 2048, False) == "strip"
     _run(dev, 300, 2048, 1.0, seed=42)
     _run(dev, 300, 2048, 0.0, seed=43)
 
@@ -307,6 +326,7 @@ def test_gae_strip_walk_all_or_no_dones(no_resident, dev):
 def test_discounted_returns_strip_walk(no_resident, dev):
     """values = None (REINFORCE returns) on the strip walk."""
     T, N = 600, 4096
+    assert _route(T, N, False, has_values=False) == "strip"
     g = torch.Generator().manual_seed(44)
     r = torch.randn(T, N, generator=g)
     d = (torch.rand(T, N, generator=g) < 0.01).to(torch.uint8)
@@ -320,6 +340,7 @@ def test_discounted_returns_strip_walk(no_resident, dev):
 def test_gae_normalize_strip_walk_matches_separate_ops(no_resident, dev):
     g = torch.Generator().manual_seed(45)
     T, N = 777, 2056
+    assert _route(T, N, True) == _route(T, N, False) == "strip"
     r = torch.randn(T, N, generator=g).to(dev)
     v = torch.randn(T, N, generator=g).to(dev)
     d = (torch.rand(T, N, generator=g) < 0.02).to(torch.uint8).to(dev)
@@ -378,6 +399,8 @@ def _gae_abi(dev, r, v, d, lv, gamma, lam, norm=False, fill=0xAB):
 def test_gae_span_matches_oracle(no_resident, dev, T, N, p):
     """With the normaliser every aligned rollout narrower than the strip walk
     takes the span passes; without it the narrow (N < 64), large ones do."""
+    assert _route(T, N, True) == "span"
+    assert _route(T, N, False) == ("span" if N < 64 and T * N >= 1 << 20 else "tiles")
     r, v, d, lv = _inputs(T, N, p, seed=T + 31 * N)
     a_ref, _ = ref.gae_c(r.numpy(), v.numpy(), d.numpy(), lv.numpy(), 0.99, 0.95)
     for norm in (True, False):
@@ -393,6 +416,7 @@ def test_gae_span_matches_oracle(no_resident, dev, T, N, p):
 
 def test_gae_span_normalize_matches_separate_ops(no_resident, dev):
     T, N = 20_000, 24
+    assert _route(T, N, True) == "span"
     r, v, d, lv = (x.to(dev) for x in _inputs(T, N, 0.01, seed=12))
     print(f"gae span norm T={T} N={N}", flush=True)
     adv, ret, adv_n = _gae_abi(dev, r, v, d, lv, 0.995, 0.9, norm=True)
@@ -406,6 +430,7 @@ def test_gae_span_normalize_matches_separate_ops(no_resident, dev):
 def test_discounted_returns_span_passes(no_resident, dev, T, N):
     """REINFORCE returns (values absent) on shapes that take the span passes
     (aligned, N < 64, >= 2^20 elements): GAE with lambda = 1 and zero values."""
+    assert _route(T, N, False, has_values=False) == "span"
     g = torch.Generator().manual_seed(T + N)
     r = torch.randn(T, N, generator=g)
     d = (torch.rand(T, N, generator=g) < 0.002).to(torch.uint8)
@@ -419,6 +444,7 @@ def test_discounted_returns_span_passes(no_resident, dev, T, N):
 
 def test_gae_span_workspace_contents_do_not_matter(no_resident, dev):
     T, N = 65_536, 16
+    assert _route(T, N, False) == "span"
     r, v, d, lv = (x.to(dev) for x in _inputs(T, N, 0.001, seed=13))
     outs = [_gae_abi(dev, r, v, d, lv, 0.999, 0.95, fill=f)[0] for f in (0x00, 0xFF, 0x7F)]
     assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
@@ -449,7 +475,8 @@ def _sweep_shapes(count=24, seed=2024, max_elems=1 << 21):
 @pytest.mark.parametrize("T,N,p,norm", _sweep_shapes())
 def test_gae_routing_sweep_matches_oracle(dev, monkeypatch, T, N, p, norm, resident):
     if not resident:
-        monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
+        _other_passes(monkeypatch)
+    assert resident or _route(T, N, norm) in ("strip", "span", "tiles")
     seed = T * 31 + N * 7 + int(norm)
     r, v, d, lv = _inputs(T, N, p, seed)
     print(f"gae sweep T={T} N={N} p={p} norm={norm} seed={seed} resident={resident}", flush=True)
@@ -492,12 +519,6 @@ RESIDENT_SHAPES = [
 ]
 
 
-def _route(T, N, norm, has_values=True):
-    from ppo_amd import _lib
-
-    return _lib.GAE_ROUTES[_lib.load().ppo_gae_route(T, N, int(norm), int(has_values))]
-
-
 def _resident_case(dev, T, N, p, norm, seed, last=True, fill=0xAB):
     assert _route(T, N, norm) == "resident"
     r, v, d, lv = (None if x is None else x.to(dev) for x in _inputs(T, N, p, seed, last))
@@ -521,9 +542,17 @@ COLUMN_SHAPES = [
     (1, 1), (1, 5), (3, 4), (127, 8), (128, 17), (256, 16), (257, 33), (512, 16), (513, 16),
     (1000, 8), (1024, 9), (1000, 255), (1000, 257), (1025, 64), (2048, 3), (2047, 65), (2048, 2047),
     (2049, 7), (255, 4096), (60, 4097), (200, 8192), (16, 8192), (500, 4100),
+    (255, 4092), (250, 8188),
     # workgroup counts of every remainder by the 8 XCDs
     (300, 2049), (300, 2057), (300, 2065), (300, 2073), (300, 2081), (300, 2089), (300, 2097),
 ]
+
+# (T, N, norm) of these that other passes take
+COLUMN_DECLINED = {
+    (2047, 65, False), (2049, 7, True), (2049, 7, False), (60, 4097, True), (60, 4097, False),
+    (255, 4096, True), (255, 4096, False), (200, 8192, True), (200, 8192, False),
+    (250, 8188, True), (16, 8192, True), (16, 8192, False), (500, 4100, True), (500, 4100, False),
+}
 
 
 @pytest.mark.parametrize("p", [0.0, 0.02])
@@ -533,6 +562,8 @@ def test_gae_column_pass(dev, T, N, p):
     buffer of random bytes as workspace, on misaligned arrays, without values,
     and with infinities late in the horizon."""
     r, v, d, lv = (x.to(dev) for x in _inputs(T, N, p, T + N, True))
+    for norm in (True, False):
+        assert (_route(T, N, norm) == "column") == ((T, N, norm) not in COLUMN_DECLINED)
     print(f"gae column T={T} N={N} p={p} routes {_route(T, N, True)} {_route(T, N, False)}",
           flush=True)
     a_ref, _ = ref.gae_c(r.cpu().numpy(), v.cpu().numpy(), d.cpu().numpy(), lv.cpu().numpy(),
@@ -668,6 +699,7 @@ def test_gae_resident_agrees_with_strip_walk_bitwise_mostly(dev, monkeypatch):
     r, v, d, lv = (x.to(dev) for x in _inputs(2048, 4096, 0.01, seed=24))
     a1, _, n1 = ppo_amd.gae_normalize(r, v, d, lv)
     monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
+    assert _route(2048, 4096, True) == "strip"
     a2, _, n2 = ppo_amd.gae_normalize(r, v, d, lv)
     same = float((a1 == a2).float().mean())
     print(f"  resident vs strip walk: {same:.6f} of advantages bit-identical", flush=True)
@@ -792,24 +824,27 @@ def test_discounted_returns_resident_rounds(dev):
 
 
 @pytest.mark.parametrize(
-    "T,N,norm",
+    "T,N,norm,route",
     [
-        (2048, 4096, True),    # one round, 128-env tiles, with the normaliser
-        (1024, 1024, True),    # one round, 64-env tiles, 4 steps per thread
-        (200_000, 128, False), # rounds
+        (2048, 4096, True, "resident"),    # one round, 128-env tiles, with the normaliser
+        (1024, 1024, True, "resident"),    # one round, 64-env tiles, 4 steps per thread
+        (200_000, 128, False, "resident"), # rounds
+        (128, 8, True, "column"),          # one workgroup
+        (2048, 64, True, "column"),        # workgroups' sums through the workspace
+        (1000, 1023, True, "column"),
     ],
 )
-def test_gae_resident_graph_replays_match_eager(dev, T, N, norm):
+def test_gae_resident_graph_replays_match_eager(dev, T, N, norm, route):
     """A captured resident-pass call replays with the nonce of its capture: the
     start barrier must reset the counters that the previous replay (or an eager
     call in between) completed.  Every replay, with new inputs copied in, and
     an eager call on the same workspace after it must equal a call on a fresh
-    workspace bit for bit."""
+    workspace bit for bit; so must those of the column pass."""
     from ppo_amd import _lib
 
     lib = _lib.load()
-    assert _route(T, N, norm) == "resident"
-    print(f"gae resident graph replays T={T} N={N} norm={norm}", flush=True)
+    assert _route(T, N, norm) == route
+    print(f"gae {route} graph replays T={T} N={N} norm={norm}", flush=True)
     g = torch.Generator(device=dev).manual_seed(T + N)
 
     def rollout():
@@ -861,21 +896,23 @@ def test_gae_resident_graph_replays_match_eager(dev, T, N, norm):
 # no dones and no bootstrap gives suffix sums of the rewards (fp64, to 1 ulp).
 # ---------------------------------------------------------------------------
 EDGE_ROUTES = [
-    (2048, 1024, True),     # resident pass
-    (2048, 1024, False),    # the same rollout off the resident pass
-    (1 << 18, 16, True),    # resident pass in rounds
-    (1 << 18, 16, False),   # span passes
-    (300, 7, False),        # unaligned N: tile passes
+    (2048, 1024, "resident"),
+    (2048, 1024, "tiles"),    # the same rollout off the resident pass
+    (1 << 18, 16, "resident"),  # in rounds
+    (1 << 18, 16, "span"),
+    (600, 4096, "strip"),
+    (300, 7, "tiles"),        # unaligned N
+    (300, 7, "column"),
+    (1500, 40, "column"),
 ]
 
 
 @pytest.mark.parametrize("gamma,lam", [(0.99, 0.0), (0.0, 0.95), (1.0, 1.0), (0.9, 1.0)])
-@pytest.mark.parametrize("T,N,resident", EDGE_ROUTES)
-def test_gae_hyperparameter_edges(dev, monkeypatch, T, N, resident, gamma, lam):
-    if not resident:
-        monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
-    route = _route(T, N, False)
-    assert (route == "resident") == resident
+@pytest.mark.parametrize("T,N,route", EDGE_ROUTES)
+def test_gae_hyperparameter_edges(dev, monkeypatch, T, N, route, gamma, lam):
+    if route not in ("resident", "column"):
+        _other_passes(monkeypatch)
+    assert _route(T, N, False) == route
     suffix = gamma == 1.0 and lam == 1.0
     r, v, d, lv = _inputs(T, N, 0.0 if suffix else 0.01, seed=T + N + int(gamma * 10))
     if suffix:

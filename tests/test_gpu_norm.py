@@ -11,6 +11,7 @@ import pytest
 import torch
 
 import ppo_amd
+from ppo_amd import _lib
 from oracle import ppo_oracle as ref
 
 pytestmark = pytest.mark.gpu
@@ -100,23 +101,27 @@ def test_fused_matches_separate_ops(dev):
 # relative, and adv_n = (adv - mean) / (std + eps) evaluated with the
 # reported statistics.
 OFFSET_ROUTES = [
-    (2048, 4096, True),    # resident pass
-    (2048, 4096, False),   # strip walk
-    (16_384, 64, False),   # span passes
-    (512, 259, False),     # unaligned N: tile passes
+    (2048, 4096, "resident"),
+    (2048, 4096, "strip"),
+    (16_384, 64, "span"),
+    (512, 259, "tiles"),   # unaligned N
+    (512, 259, "column"),  # several workgroups
+    (128, 8, "column"),    # one workgroup
 ]
 
 
 @pytest.mark.parametrize("mu", [1e2, 1e3, 1e4])
-@pytest.mark.parametrize("T,N,resident", OFFSET_ROUTES)
-def test_gae_normalize_large_mean(dev, monkeypatch, T, N, resident, mu):
-    if not resident:
+@pytest.mark.parametrize("T,N,route", OFFSET_ROUTES)
+def test_gae_normalize_large_mean(dev, monkeypatch, T, N, route, mu):
+    if route not in ("resident", "column"):
         monkeypatch.setenv("PPO_AMD_GAE_RESIDENT", "0")
+        monkeypatch.setenv("PPO_AMD_GAE_COLUMN", "0")
+    assert _lib.GAE_ROUTES[_lib.load().ppo_gae_route(T, N, 1, 1)] == route
     g = torch.Generator().manual_seed(int(mu) + N)
     r = mu + torch.randn(T, N, generator=g)
     v = torch.zeros(T, N)
     d = torch.ones(T, N, dtype=torch.uint8)  # every step done: adv = r - v
-    print(f"gae_normalize large mean T={T} N={N} resident={resident} mu={mu}", flush=True)
+    print(f"gae_normalize large mean T={T} N={N} route={route} mu={mu}", flush=True)
     adv, _, adv_n, stats = ppo_amd.gae_normalize(r.to(dev), v.to(dev), d.to(dev), None, 0.99,
                                                  0.95, return_stats=True)
     a64 = adv.cpu().double()

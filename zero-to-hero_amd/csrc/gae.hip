@@ -2195,11 +2195,17 @@ const void* res_kernel(const ResPlan& rp, bool stats, bool has_v) {
   return res_kernel_e<16>(rp.L, stats, has_v, rounds);
 }
 
-// The environment variable PPO_AMD_GAE_RESIDENT=0 turns the resident pass off
-// (the other passes wait for no other workgroup).
+bool switched_off(const char* name) {
+  const char* env = getenv(name);
+  return env && env[0] == '0';
+}
+
+// The environment variables PPO_AMD_GAE_RESIDENT=0 and PPO_AMD_GAE_COLUMN=0 turn
+// the resident and the column pass off: the first for callers that share the GPU
+// (no other pass waits for another workgroup), both so that the strip walk, the
+// span and the tile passes can be tested on shapes that these would take.
 bool resident_ok(long T, long N, bool norm, bool has_v) {
-  const char* env = getenv("PPO_AMD_GAE_RESIDENT");
-  if (env && env[0] == '0') return false;
+  if (switched_off("PPO_AMD_GAE_RESIDENT")) return false;
   const ResPlan rp = res_plan(T, N, norm);
   if (rp.E == 0) return false;
   const void* kern = res_kernel(rp, norm, has_v);
@@ -2526,7 +2532,7 @@ int gae_route(long T, long N, bool norm, bool has_v, bool vec, bool all_vec) {
   // aligned rollouts of many tiles that all fit on the device at once: one
   // read of the rollout, one write of each output
   if (all_vec && resident_ok(T, N, norm, has_v)) return PPO_GAE_ROUTE_RESIDENT;
-  if (col_plan(T, N, norm).E) return PPO_GAE_ROUTE_COLUMN;
+  if (col_plan(T, N, norm).E && !switched_off("PPO_AMD_GAE_COLUMN")) return PPO_GAE_ROUTE_COLUMN;
   if (vec && span_route(T, N, norm)) return PPO_GAE_ROUTE_SPAN;
   const GaePlan p = make_plan(T, N, vec && !narrow_scalar(T, N, norm) ? 4 : 1);
   return strip_plan(p).E > 0 ? PPO_GAE_ROUTE_STRIP : PPO_GAE_ROUTE_TILES;
