@@ -93,8 +93,8 @@ def test_mlp_grads_match_oracle(dev, n, D, H, A, act, B):
 # block, and a last block of 1 and of 15 rows
 @pytest.mark.parametrize("H,B", [(128, 16 * 128 + 1), (128, 2 * 16 * 128 + 15), (64, 16 * 256 + 1),
                                  (32, 16 * 512 + 15), (16, 2 * 16 * 1024 + 1)])
-# both sides of the tiles of observations (16, then 64) and of actions (16, 32)
-@pytest.mark.parametrize("D,A", [(1, 1), (16, 16), (17, 17), (64, 32)])
+# both sides of the tiles of observations (16, 32, then 64) and of actions (16, 32)
+@pytest.mark.parametrize("D,A", [(1, 1), (16, 16), (17, 17), (32, 5), (33, 18), (64, 32)])
 def test_mlp_grads_blocks_and_tiles(dev, H, B, D, A):
     _check(dev, B + 3, D, H, A, "tanh", B, seed=H + D + A, vf_clip=0.2)
 

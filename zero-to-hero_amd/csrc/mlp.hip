@@ -1215,11 +1215,18 @@ MlpLayout mlp_layout(long B, int D, int H, int A) {
   return l;
 }
 
+// Observations padded to 16, 32 or 64 columns, actions to 16 or 32.  (Without
+// the 32 columns, D = 24 at H = 16 and 17 at H = 32 took longer than one 16-row
+// block per workgroup did: us, that / 64 columns / 32: 4096 rows 24-16-16-6 15.7 /
+// 16.8 / 13.9, 17-32-32-18 19.1 / 21.3 / 16.8; 32,768 rows 17-128-128-18 350 / 156 / 133.)
 template <int H, int kAct>
 const void* mlp_kernel_tiles(int D, int A) {
   if (D <= 16)
     return A <= 16 ? (const void*)mlp_cat_grad_kernel<H, kAct, 1, 1>
                    : (const void*)mlp_cat_grad_kernel<H, kAct, 1, 2>;
+  if (D <= 32)
+    return A <= 16 ? (const void*)mlp_cat_grad_kernel<H, kAct, 2, 1>
+                   : (const void*)mlp_cat_grad_kernel<H, kAct, 2, 2>;
   return A <= 16 ? (const void*)mlp_cat_grad_kernel<H, kAct, 4, 1>
                  : (const void*)mlp_cat_grad_kernel<H, kAct, 4, 2>;
 }
