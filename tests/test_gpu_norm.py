@@ -22,7 +22,7 @@ def _c_oracle():
     ref.build_c()
 
 
-@pytest.mark.parametrize("n", [2, 3, 4, 5, 255, 1024, 4099, 1_000_003])
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 255, 1024, 4099, 12_289, 524_288, 1_000_003])
 def test_normalize_matches_reference(dev, n):
     g = torch.Generator().manual_seed(n)
     a = torch.randn(n, generator=g) * 2.5 + 0.7

@@ -104,15 +104,20 @@ __global__ void __launch_bounds__(kBlock) normalize_kernel(const float* adv, flo
 // The finaliser fused into the elementwise pass, for few partials: every
 // block derives the normaliser parameters itself with norm_params (same
 // block size as the one-block finaliser, so the same fixed order and
-// bit-identical values), after issuing its first kNormU float4 loads so that
+// bit-identical values), after issuing its first U float4 loads so that
 // the partials' reduction overlaps them.  Block 0 also stores the parameters
-// in the header and {mean, std} in stats_out.
+// in the header and {mean, std} in stats_out.  U = 1 while that gives at most a
+// block per CU: more CUs then share a short pass's loads and stores (the GAE call
+// 2048 x 64 12.7 us with U = 4, 11.3 with 1; 200 x 2048 10.6 and 9.1, 1000 x 1023 14.5
+// and 13.1).
 #ifndef PPO_NORM_U
 #define PPO_NORM_U 4
 #endif
 constexpr int kNormU = PPO_NORM_U;
+constexpr long kNormCus = 256;
 constexpr long kFusedNormMaxPartials = 512;
 
+template <int U>
 __global__ void __launch_bounds__(kFinalBlock) normalize_stats_kernel(
     const float* adv, float* out, long n, const double* partials, long count, double eps,
     WsHeader* hdr, float* stats_out) {
@@ -123,9 +128,9 @@ __global__ void __launch_bounds__(kFinalBlock) normalize_stats_kernel(
   f4* o4 = reinterpret_cast<f4*>(out);
   const long stride = (long)gridDim.x * kFinalBlock;
   const long gid = (long)blockIdx.x * kFinalBlock + threadIdx.x;
-  f4 x[kNormU];
+  f4 x[U];
 #pragma unroll
-  for (int u = 0; u < kNormU; ++u) {
+  for (int u = 0; u < U; ++u) {
     const long i = gid + u * stride;
     x[u] = a4[i < n4 ? i : 0];  // unconditional (n >= 4): element 0 stands in past the end
   }
@@ -146,7 +151,7 @@ __global__ void __launch_bounds__(kFinalBlock) normalize_stats_kernel(
   __syncthreads();
   const float mean = s_par[0], denom = s_par[1];
 #pragma unroll
-  for (int u = 0; u < kNormU; ++u) {
+  for (int u = 0; u < U; ++u) {
     const long i = gid + u * stride;
     if (i < n4) {
       f4 y;
@@ -157,7 +162,7 @@ __global__ void __launch_bounds__(kFinalBlock) normalize_stats_kernel(
       __builtin_nontemporal_store(y, o4 + i);
     }
   }
-  for (long i = gid + kNormU * stride; i < n4; i += stride) {
+  for (long i = gid + U * stride; i < n4; i += stride) {
     const f4 v = a4[i];
     f4 y;
     y[0] = (v[0] - mean) / denom;
@@ -182,11 +187,13 @@ int launch_normalize(const double* partials, long count, double eps, const float
                      long n, WsHeader* hdr, float* stats_out, hipStream_t stream) {
   if (n <= 0) return PPO_OK;
   if (count <= kFusedNormMaxPartials && n >= 4 && aligned(adv, 16) && aligned(out, 16)) {
-    const long per_block = (long)kFinalBlock * kNormU;
+    const bool small = (n + 3) / 4 <= kNormCus * kFinalBlock;
+    const long per_block = (long)kFinalBlock * (small ? 1 : kNormU);
     long blocks = ((n + 3) / 4 + per_block - 1) / per_block;
     blocks = std::max(1L, std::min(blocks, 4096L));
-    hipLaunchKernelGGL(normalize_stats_kernel, dim3((unsigned)blocks), dim3(kFinalBlock), 0,
-                       stream, adv, out, n, partials, count, eps, hdr, stats_out);
+    const auto kern = small ? normalize_stats_kernel<1> : normalize_stats_kernel<kNormU>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)blocks), dim3(kFinalBlock), 0, stream, adv, out, n,
+                       partials, count, eps, hdr, stats_out);
     return last_launch_status();
   }
   int st = launch_finalize_stats(partials, count, eps, hdr, stats_out, stream);
