@@ -542,16 +542,18 @@ COLUMN_SHAPES = [
     (1, 1), (1, 5), (3, 4), (127, 8), (128, 17), (256, 16), (257, 33), (512, 16), (513, 16),
     (1000, 8), (1024, 9), (1000, 255), (1000, 257), (1025, 64), (2048, 3), (2047, 65), (2048, 2047),
     (2049, 7), (255, 4096), (60, 4097), (200, 8192), (16, 8192), (500, 4100),
-    (255, 4092), (250, 8188),
+    (255, 4092), (250, 8188), (1500, 2052), (1500, 2044), (1100, 1300), (1500, 2049),
+    # the elementwise normaliser's last length of one load per thread, and past it
+    (1025, 1023), (1031, 1021),
     # workgroup counts of every remainder by the 8 XCDs
     (300, 2049), (300, 2057), (300, 2065), (300, 2073), (300, 2081), (300, 2089), (300, 2097),
 ]
 
 # (T, N, norm) of these that other passes take
 COLUMN_DECLINED = {
-    (2047, 65, False), (2049, 7, True), (2049, 7, False), (60, 4097, True), (60, 4097, False),
-    (255, 4096, True), (255, 4096, False), (200, 8192, True), (200, 8192, False),
-    (250, 8188, True), (16, 8192, True), (16, 8192, False), (500, 4100, True), (500, 4100, False),
+    (1500, 2052, True), (1500, 2052, False), (1500, 2049, True), (2049, 7, True), (2049, 7, False),
+    (60, 4097, True), (60, 4097, False), (255, 4096, True), (255, 4096, False), (200, 8192, True),
+    (200, 8192, False), (250, 8188, True), (16, 8192, True), (16, 8192, False), (500, 4100, True), (500, 4100, False),
 }
 
 

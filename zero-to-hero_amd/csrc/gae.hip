@@ -291,7 +291,7 @@ struct ResPlan {
 // without filling the device, take the other paths: measured on MI355X, 2048 x
 // 4096 runs 45 us against 55 us, 4096 x 2048 45 us against 72 and 32768 x 256 (64
 // tiles per column, 256 tiles) 57 us against 67.  (Fewer tiles would gain as
-// well, 8192 x 16 with the normaliser 12.6 us against 17.7 of the span passes, but
+// well, 8192 x 16 with the normaliser 12.6 us against 16.2 of the span passes, but
 // would make small rollouts wait for a whole grid to be resident.)
 // Without the normaliser, rollouts too long for one round (more than 256
 // tiles of 16 steps per thread) run in rounds of 256 tiles, from the end of
@@ -363,22 +363,20 @@ struct ColPlan {
 };
 
 // A workgroup touches every row of the horizon once per array whatever E is (16,
-// 32 or 64 bytes of it), so its time grows with T: taken to T = 2048 (2048 x 64
-// with the normaliser 12.8 us against 17.7 of the span passes; a workgroup holds
-// no more).  Narrow columns give more workgroups, wide ones longer row pieces: 16
-// envs to 256 steps, then 4, or 8 where 4 would give more than 64 workgroups (with
-// the normaliser, 4 and 8: 1000 x 64 10.5 and 11.2 us, 2048 x 700 30.0 and 21.3, 1000
-// x 1023 15.6 and 14.4).  A rollout that one workgroup holds needs no second launch
-// (512 x 16 with the normaliser 7.2 us with 16 envs, 8.5 with 8).  With the
-// normaliser more than 256 workgroups take the next width (1000 x 2049 19 us).
-// Where the tile or strip passes have enough rows in flight they win: past 512
-// columns (512 x 20001 without the normaliser 124 us against 76), with most threads
-// idle (16 x 30000 13 against 7), and without the normaliser past 1024 steps of
-// more than 64 envs (1500 x 769 14.8, 2048 x 1300 23.7) up to the width where no
-// vector access helps them (1100 x 1025 14.5 against 10.1 of columns, 2000 x 1793
-// 31.8 against 19.9).  With the normaliser their extra passes cost them more
-// (2048 x 128 18.3 against 13.3, 1200 x 256 18.7 and 12.4, 1100 x 641 18.4 and 15.4,
-// 2000 x 769 22.4 and 22.3, 2048 x 700 60 and 21).
+// 32 or 64 bytes of it), so its time grows with T; it holds 2048 rows (2048 x 64
+// with the normaliser 11.3 us against 16.4 of the span passes).  Narrow columns give
+// more workgroups, wide ones longer row pieces: 16 envs to 256 steps, then 4, or 8
+// where 4 would give more than 64 workgroups (with the normaliser, 4 and 8: 1000 x
+// 64 9.2 and 9.9 us, 2048 x 128 11.9 and 13.7, 1000 x 1023 14.5 and 13.1, 2048 x 2047
+// 38.9 and 28.2).  A rollout that one workgroup holds needs no second launch (512 x
+// 16 with the normaliser 7.2 us with 16 envs, 8.3 with 8).  With the normaliser more
+// than 256 workgroups take the next width (1000 x 2049 24.3 us with 8 envs, 19.5
+// with 16, 28.6 on the tile passes).  Where the other passes have enough rows in
+// flight they win: past 512 columns (512 x 20001 without the normaliser 124 us
+// against 74), with most threads idle (16 x 30000 13 against 7), and past 1024 steps
+// in a second round of workgroups against the strip walk (without the normaliser
+// 1030 x 4092 23.3 against 19.8, 2047 x 4092 35.6 against 31.2; in one round 1030 x
+// 2044 12.0 against 15.2, 2047 x 1300 17.0 against 23.7 of the tile passes).
 ColPlan col_plan(long T, long N, bool norm) {
   const ColPlan none = {0, 0, 0};
   if (T <= 0 || N <= 0 || T > 2048 || T * N >= (1L << 30)) return none;
@@ -394,7 +392,7 @@ ColPlan col_plan(long T, long N, bool norm) {
   }
   const long wgs = (N + E - 1) / E, per = steps(E);
   if (wgs > 2 * kResMaxTiles || (wgs > kResMaxTiles && T * E < kColBlock)) return none;
-  if (!norm && T > 1024 && N > 64 && (N <= 1024 || N % 4 == 0)) return none;
+  if (T > 1024 && wgs > kResMaxTiles && N % 4 == 0) return none;
   return {E, per <= 2 ? 2 : (per <= 4 ? 4 : (per <= 8 ? 8 : 16)), wgs};
 }
 
@@ -2235,18 +2233,18 @@ int launch_resident(long T, long N, GaeArgs a, bool norm, hipStream_t stream) {
 // so no carry crosses workgroups and none waits for another.  With the normaliser
 // a single workgroup normalises from its registers; several leave their fp64 (n,
 // sum, sum of squares) to the elementwise normaliser, which reads the advantages
-// back out of the caches.  (An exchange of the sums inside the launch saves that
-// second launch, 0 to 1.4 us -- 128 x 64 6.8 us, 1000 x 1023 14.0, 2048 x 2047 28.2 --
-// but needs the whole grid resident at once and gives up where another stream's
-// waiting grid holds the chip.)
+// back out of the caches.  (An exchange of the sums inside the launch takes 6.8 us
+// against 7.5 at 128 x 64, 11.9 against 11.3 at 2048 x 64, 14.0 against 13.1 at 1000 x
+// 1023; it needs the whole grid resident at once and gives up where another
+// stream's waiting grid holds the chip.)
 //
 // What bounds it: latency -- one round of loads, the scan, the stores, and with
 // the normaliser a second launch.  Measured on MI355X against the 1 to 4 launches
 // of the span and tile passes (T x N, us of device time per call, with / without the
 // normaliser):
-//   128 x 8      14.2 -> 4.6 / 5.9 -> 3.6      1000 x 64    17.6 -> 10.5 / 11.6 -> 5.6
-//   1000 x 1023  18.7 -> 14.4 / 13.3 -> 8.1    2048 x 64    17.7 -> 12.8 / 11.0 -> 7.4
-//   200 x 2048   18.7 -> 10.6 / 13.7 -> 4.3    2048 x 2047  45.1 -> 27.7 / 36.0 -> 20.0
+//   128 x 8      14.2 -> 4.6 / 5.9 -> 3.6      1000 x 64    17.8 -> 9.2 / 11.6 -> 5.6
+//   1000 x 1023  18.5 -> 13.1 / 13.3 -> 8.1    2048 x 64    17.8 -> 11.3 / 11.0 -> 7.4
+//   200 x 2048   18.6 -> 9.1 / 13.7 -> 4.3     2048 x 2047  44.3 -> 27.6 / 36.0 -> 20.0
 // ---------------------------------------------------------------------------
 constexpr int kColWaves = kColBlock / kWave;
 
