@@ -67,12 +67,12 @@ struct LossArgs {
   float* dval;
   float* scalars;
   double* partial;
-  uint64_t* epoch;  // Gaussian: the workspace header's call counter
-  int tag_slot;     // Gaussian: partial slot holding each workgroup's arrival tag
-  int finish;       // Gaussian: 1 = collect in-kernel, 0 = loss_gauss_finish_kernel does
+  uint64_t* epoch;  // in-kernel finish: the workspace header's call counter
+  int tag_slot;     // in-kernel finish: partial slot holding each workgroup's arrival tag
+  int finish;       // 1 = collect in-kernel, 0 = a finaliser launch does
   int nopoll;       // the collection follows the loss launch: read the partials without polling
-  int collector;    // wave-tile kernels: workgroups 0 .. collector-1 only collect (no tiles)
-  WaitCtl wc;       // Gaussian in-kernel finish: poll limit, the device's wait-status word
+  int collector;    // workgroups 0 .. collector-1 only collect (no tiles)
+  WaitCtl wc;       // in-kernel finish: poll limit, the device's wait-status word
 };
 
 // Streamed arrays are touched once: nontemporal loads/stores keep them from
@@ -584,7 +584,7 @@ __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long
 // consecutive logits each in C chunks (lane q of the group holds columns
 // (q + c G) VW ..), so a wave loads 64 / G whole rows per step straight from
 // memory, coalesced, and needs no LDS transposition.  A wave tile is I steps
-// (I * 64 / G rows, I <= G): the tile's logits stay in registers (at most 64
+// (I * 64 / G rows, I <= G): the tile's logits stay in registers (at most 32
 // VGPRs) from their one load to the gradient's store.  Per step a DPP tree
 // over the group forms the row's max, s = sum e and S = sum e t, and lane i of
 // each group keeps step i's: the row's scalar math (log, the ratio's exp,
@@ -606,7 +606,8 @@ __global__ void __launch_bounds__(kBlock) loss_cat_wtile_kernel(LossArgs a, long
 //   B = 8,388,608, A = 4: 132 -> 104 us;  B = 2,000,000, A = 16: 64 -> 59 us
 //     (rows padded in LDS before, ~40 instructions per logit)
 //   misaligned B = 1,000,000, A = 18: 70 -> 45 us
-// Steps of 4 (16 logits per lane at most): 8 or 16 steps put more loads in
+// 4 steps (16 logits per lane, 32 from A = 65 on; 2 steps of 16 logits past A =
+// 512): 8 or 16 steps put more loads in
 // flight per wave but leave fewer waves (A = 64: 31 us at 4 steps, 33 at 8, 35
 // at 16; 2 steps, 39).  128-byte row segments per step: 8 lanes x 2 chunks
 // instead of 16 x 1 measures the same at A = 64 and 38 against 29 us at A = 50,

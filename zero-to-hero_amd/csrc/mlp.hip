@@ -111,7 +111,7 @@ __device__ __forceinline__ float act_grad(float g, float y) {
 // along the contraction, lane l supplies A(l % 16, k0 + l / 16) and
 // B(k0 + l / 16, l % 16); the result C(4 * (l / 16) + r, l % 16) is element r.
 // Every GEMM here has one 16-row side (the workgroup's minibatch rows) and
-// is cut into such tiles, spread over the workgroup's 4 waves.
+// is cut into such tiles, spread over the workgroup's waves.
 // ---------------------------------------------------------------------------
 typedef float v4f __attribute__((ext_vector_type(4)));
 
