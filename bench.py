@@ -5,7 +5,7 @@ T x N = 2048 x 4096 = 8,388,608 samples (the benchmark's GAE + normalise rollout
   1. ppo_gae_norm_f32  — GAE with bootstrap + returns + advantage
                          normalisation (rl/deep/agents/ppo.py:123-127): the
                          advantages, returns and normalised advantages of
-                         BASELINE config 2
+                         T = 2048 x N = 4096
   2. ppo_loss_cat_f32  — fused categorical PPO loss forward+backward over all
                          B = T*N samples, A = 18 actions, vf_clip = 0.2
                          (ppo.py:150-169; A = 18, value clipping 0.2)
@@ -19,7 +19,7 @@ launched on.  `cpu_baseline` times the CPU restatement of the same path
 
 --suite additionally prints one line per benchmark configuration (2-5) kernel, for
 the roofline table; --update-suite times the whole minibatch update loop;
-the driver's contract line is always the last line.
+the default workload's JSON line is always the last line.
 """
 
 from __future__ import annotations
@@ -104,7 +104,7 @@ ROLLOUT_KEYS = ("rewards", "values", "dones", "last_value")
 class Step:
     """The two C-ABI calls of one update step, on torch's current stream,
     with preallocated outputs (nothing allocated inside the timed loop).
-    The GAE call writes all three outputs BASELINE config 2 names
+    The GAE call writes all three outputs
     (advantages, returns, normalised advantages: 21 bytes per sample with its
     inputs); `--suite` also times the in-place form the library's own update
     loop uses (config2_gae_norm_in_place).
@@ -438,7 +438,7 @@ def suite(torch, lib, dev, stream_timing=True, cpu=True):
             mc, lc, ac, rc[0], rc[1], rc[2], rc[3], rc[4], 0.2, 0.2, 0.5, 0.01))
         del mc, lc, ac, rc
     del mu, acts, rows, w, make
-    # the north-star step with A = 2 (CartPole's action count): GAE+norm + loss
+    # the default step with A = 2 (CartPole's action count): GAE+norm + loss
     x = synthetic_rollout(torch, dev, T_STEPS, N_ENVS, 2, seed=26)
     steps = [Step(torch, lib, x, dev)]
     if stream_timing:

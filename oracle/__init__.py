@@ -4,7 +4,7 @@ This package restates, on the CPU, the arithmetic of the reference's PPO
 update (mrhooray/zero-to-hero, rl/deep/agents/ppo.py:113-193).  It exists to
 check the MI355X library, never to stand in for it: only tests/,
 __graft_entry__.smoke() and bench.py's cpu_baseline leg may import it, and
-only as the checker or as the timed CPU baseline.  The product package
+only as the oracle or as the timed CPU baseline.  The product package
 (ppo_amd) never imports it and fails loudly when its HIP library is missing.
 
 Contents (each function cites the reference lines it follows):

@@ -1,7 +1,7 @@
 """CPU restatement of the reference PPO update path — TEST INFRASTRUCTURE ONLY.
 
 Only tests/, __graft_entry__.smoke() and bench.py's cpu_baseline leg may use
-this module, as the checker or as the timed CPU baseline; the product package
+this module, as the oracle or as the timed CPU baseline; the product package
 (ppo_amd) never imports it.
 
 Reference: mrhooray/zero-to-hero rl/deep/agents/ppo.py (PPOAgent), whose

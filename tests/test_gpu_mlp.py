@@ -4,7 +4,7 @@ against the CPU oracle update_batch_grads_reference (torch autograd on the
 same networks in fp64).
 
 Tolerance: every parameter gradient within rel 1e-4 plus an absolute floor
-of 1e-5 x max|g| of that tensor (north star: rel 1e-4 for gradients in fp32;
+of 1e-5 x max|g| of that tensor (rel 1e-4 for gradients in fp32;
 the floor covers elements that cancel to ~0), loss scalars rel 1e-5 (approx_kl,
 a cancellation, 1e-6 absolute).  The kernel computes in fp32 like torch; its
 sums over the minibatch run in another order than torch's GEMMs.

@@ -1,4 +1,4 @@
-"""Pins the CPU oracle (oracle/) before it is trusted as the checker.
+"""Pins the CPU oracle (oracle/) before it is trusted.
 
 Each oracle function is checked against something other than itself: the
 reference's own known answer (rl/deep/tests/test_ppo.py:34-44), closed forms,

@@ -284,7 +284,7 @@ struct ResPlan {
 // that still fit on the device at once (<= 256), with no more than a quarter
 // of a column's threads idle past the horizon; ties go to wider tiles (longer
 // row segments: at T x N = 2048 x 4096 with the normaliser, 128-env tiles
-// measured 38.2-38.5 us per call in the north-star step against 39.1-39.3 us
+// measured 38.2-38.5 us per call in the GAE + loss step against 39.1-39.3 us
 // for 64-env tiles; 256-env tiles were slower, their look-back folding 15
 // tiles per column, so 128-env tiles are taken only up to 8 tiles per column).  Rollouts that
 // give fewer than kResMinTiles tiles, or more than 16 tiles per env column

@@ -78,8 +78,8 @@ struct LossArgs {
 // Streamed arrays are touched once: nontemporal loads/stores keep them from
 // displacing reusable lines (measured on MI355X: a float4 copy goes from 5.5
 // to 6.3 TB/s with nontemporal accesses and 4 loads in flight per thread).
-// Ordinary stores make this kernel look faster in isolation (the north-star
-// loss 268 -> 241 us after a read-only cache flush) but leave ~0.6 GB of
+// Ordinary stores make this kernel look faster in isolation (the loss of
+// 8,388,608 rows, A = 18, 268 -> 241 us after a read-only cache flush) but leave ~0.6 GB of
 // dirty lines whose write-back lands in the next kernel: in the GAE + loss
 // step the GAE call went from 53 to 69 us and the step from 305 to 333 us.
 typedef float f4 __attribute__((ext_vector_type(4)));
